@@ -64,7 +64,7 @@ def listed():
 
 # sizes that draw() spreads over, by kind and matrix
 RANGES = {
-    "op": {"lap27": (24, 192), "aniso": (80, 2048), "fv7": (24, 192), "graph": (6000, 600000)},
+    "op": {"lap27": (48, 192), "aniso": (320, 2048), "fv7": (48, 192), "graph": (30000, 600000)},
     "cycle": {"lap27": (16, 128), "aniso": (64, 1024), "fv7": (16, 96)},
     "solve": {"lap27": (16, 160), "aniso": (64, 1024), "fv7": (16, 96)},
     "adjoint": {"fv7": (16, 96)},
@@ -131,7 +131,9 @@ def host_matrix(case, seed):
     if case["matrix"] == "graph":
         return _graph(case["m"], seed)
     if case["matrix"] == "fv7":
-        return ra.gallery_fv7(case["m"], seed=seed)
+        # a Galerkin product's interpolation is one the program kept: its
+        # coefficients do not follow the seed (rescaled() makes the new ones)
+        return ra.gallery_fv7(case["m"], seed=3 if case["kind"] == "galerkin" else seed)
     return _gallery(case["matrix"], case["m"])
 
 
@@ -314,7 +316,8 @@ def run(st):
         sizes, nnz, _ = ml.level_sizes()
         A.free()
         ml.free()
-        return {"x": st["out"], "rows": sizes, "entries": nnz}
+        # by level, zero below the coarsest (the number of levels follows the coefficients)
+        return {"x": st["out"], "rows": np.pad(sizes, (0, 25 - sizes.size)), "entries": np.pad(nnz, (0, 25 - nnz.size))}
     raise ValueError(kind)
 
 
