@@ -328,12 +328,13 @@ int ramd_hier_load(ramd_ctx ctx, const char* path, ramd_hier* out);
 /* Builds the FP32 copies of every level used by RAMD_PREC_FP32 cycles. */
 int ramd_hier_enable_fp32(ramd_hier h);
 /* Coarse tail: the cycle of the small coarsest levels (up to 2048 rows and
- * 16384 entries of A and P each, coarse system of at most 64 rows), with
- * the restriction into them and the interpolation out, as one workgroup in
- * one launch instead of one launch per operation.  Same bits either way.
+ * 32768 entries of A and P each, their vectors together in one compute
+ * unit's LDS, coarse system of at most 64 rows), with the restriction into
+ * them and the interpolation out, as one workgroup in one launch instead of
+ * one launch per operation.  Same bits either way.
  * level -1: off; 0 (default): automatic -- the first cycle in each
- * precision times a V-cycle without a tail and with every level that can
- * start one, and keeps the fastest; >= 1: the tail starts at that level
+ * precision times V-cycles with the three largest tails and keeps the
+ * fastest; >= 1: the tail starts at that level
  * (RAMD_E_ARG if it cannot).  No reference counterpart
  * (ParMultilevel::cycle, multilevel/par_multilevel.hpp:341-457, is one
  * routine per level); a tuning switch. */

@@ -1071,7 +1071,7 @@ static void bcycle(ramd_hier_s* h, BlockState* bs, int l, X* x, const X* b)
     if (l == (int)h->levels.size() - 1) {
         const int n = h->coarse_n;
         if (n && n <= kCoarseWave)
-            hipLaunchKernelGGL((bcoarse_wave<X>), dim3(k), dim3(64), sizeof(double) * n * n, s, n, k, h->lu, h->piv,
+            hipLaunchKernelGGL((bcoarse_wave<X>), dim3(k), dim3(64), sizeof(double) * n * n, s, n, k, h->lu, h->perm,
                                b, x);
         else if (n)
             hipLaunchKernelGGL((bcoarse_solve<X>), dim3(k), dim3(256), sizeof(double) * n, s, n, k, h->lu, h->piv, b,

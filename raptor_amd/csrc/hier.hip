@@ -236,265 +236,19 @@ __global__ void to_f64(int64_t n, const float* __restrict__ a, double* __restric
 // ---------------------------------------------------------------------------
 template <typename TB, typename TX>
 __global__ __launch_bounds__(64) void coarse_wave_kernel(int n, const double* __restrict__ lu,
-                                                         const int* __restrict__ piv, const TB* __restrict__ b,
+                                                         const int* __restrict__ perm, const TB* __restrict__ b,
                                                          TX* __restrict__ x)
 {
     extern __shared__ double ls[];
-    coarse_solve_wave<TB, TX>(n, lu, piv, b, x, 1, ls);
+    coarse_solve_wave<TB, TX>(n, lu, perm, b, x, 1, ls);
 }
 
-// ---------------------------------------------------------------------------
-// Coarse tail: the restriction into a run of small levels, their whole
-// V-cycle (smoothing, residuals, restrictions, the coarse LU solve,
-// interpolations) and the interpolation back out, by one workgroup in one
-// launch instead of about five launches per level.  Each operation runs
-// over its rows with a workgroup barrier after it; a row is computed by one
-// thread with the operations of stream_kernel's phase 2 on the CSR arrays
-// (products rounded, then added left to right in stored order; Jacobi's
-// diagonal rules), so every value is the one the per-level kernels produce.
-// ---------------------------------------------------------------------------
+// Coarse tail (tail.hip): the levels it takes.
 constexpr int kTailMax = 8;          // levels in the tail, the coarsest included
-constexpr int kTailThreads = 1024;
 constexpr int kTailMaxRows = 2048;   // a tail level's rows
-constexpr int64_t kTailMaxNnz = 16384;   // a tail level's A (and P) entries
-constexpr int kTailMaxOuterRows = 8192;  // rows of the level above the tail
+constexpr int64_t kTailMaxNnz = 32768;   // a tail level's A (and P) entries
+constexpr int kTailMaxOuterRows = 8190;  // rows of the level above the tail (16-bit byte offsets)
 constexpr int64_t kTailMaxOuterNnz = 65536;  // entries of its P
-
-template <typename X>
-struct TailLevel {
-    int n = 0;
-    int jfz = 0;  // the restriction into this level forms its first Jacobi sweep from zero
-    int adf = 0;  // A stores every row's diagonal first
-    const int *arp = nullptr, *acol = nullptr;
-    const X* aval = nullptr;
-    const X* diag = nullptr;
-    const int *prp = nullptr, *pcol = nullptr;  // P: this level to the next
-    const X* pval = nullptr;
-    const int *rrp = nullptr, *rcol = nullptr;  // R = P^T
-    const X* rval = nullptr;
-    X *x = nullptr, *b = nullptr, *t = nullptr, *r = nullptr;
-};
-template <typename X>
-struct TailArgs {
-    int nl = 0;  // levels lv[0 .. nl), lv[nl - 1] the coarsest
-    int nb = 0;  // rows of the level above the tail
-    const int *bprp = nullptr, *bpcol = nullptr;  // its P and R
-    const X* bpval = nullptr;
-    const int *brrp = nullptr, *brcol = nullptr;
-    const X* brval = nullptr;
-    const X* rb = nullptr;    // its residual
-    const X* curb = nullptr;  // its iterate
-    X* outb = nullptr;        // receives curb + P x_tail
-    int coarse_n = 0;
-    const double* lu = nullptr;
-    const int* piv = nullptr;
-    X omega = 0;
-    int sweeps = 0;
-    TailLevel<X> lv[kTailMax];
-};
-
-// One operation over rows [0, n) of a CSR matrix (n <= kTailThreads *
-// kTailRowsPerThread): OP_SPMV, OP_SPMV_JFZ (y2 = the first Jacobi sweep
-// from zero on y, diagonal dvec), OP_RESIDUAL, OP_ADD_INTO (y = b + A x) and
-// OP_JACOBI (x old iterate, y new; df: diagonal stored first, dvec its
-// values).  The workgroup forms the products of a window of the matrix's
-// entries together (independent loads) into prod (LDS, kTailLds entries),
-// then each row's thread adds its entries of the window in stored order,
-// carrying its sum to the next window: stream_kernel's operations.
-constexpr int kTailRowsPerThread = 8;
-constexpr int kTailLdsBytes = 65536;
-static_assert(kCoarseWave * kCoarseWave * (int)sizeof(double) <= kTailLdsBytes, "coarse LU must fit the tail's LDS");
-static_assert(kTailMaxOuterRows <= kTailThreads * kTailRowsPerThread && kTailMaxRows <= kTailMaxOuterRows,
-              "tail rows per thread");
-
-template <int OP, typename X>
-__device__ void tail_op(X* prod, int n, const int* __restrict__ rp, const int* __restrict__ col,
-                        const X* __restrict__ val, const X* x, const X* b, X* y, X omega, const X* dvec, X* y2,
-                        int df)
-{
-    constexpr int CAP = kTailLdsBytes / (int)sizeof(X);
-    constexpr int RT = kTailRowsPerThread;
-    const int tid = threadIdx.x;
-    const int e0 = rp[0], E = rp[n] - e0;
-    int lo[RT], hi[RT];
-    X acc[RT], diag[RT];
-#pragma unroll
-    for (int u = 0; u < RT; u++) {
-        const int row = tid + u * kTailThreads;
-        lo[u] = hi[u] = 0;
-        acc[u] = diag[u] = X(0);
-        if (row < n) {
-            const int rs = rp[row] - e0, re = rp[row + 1] - e0;
-            lo[u] = rs;
-            hi[u] = re;
-            if (OP == OP_RESIDUAL) acc[u] = b[row];
-            if (OP == OP_JACOBI && df && rs < re) {
-                // the diagonal (first) entry is not added; a row without a
-                // usable one keeps its value
-                bool use;
-                if (dvec) {
-                    const X dg = dvec[row];
-                    use = fabs(dg) > X(1e-16);
-                    if (use) diag[u] = dg;
-                } else {
-                    use = col[e0 + rs] == row;
-                    if (use) diag[u] = val[e0 + rs];
-                }
-                lo[u] = use ? rs + 1 : re;
-            }
-        }
-    }
-    for (int c0 = 0; c0 < E; c0 += CAP) {
-        const int cn = min(CAP, E - c0);
-        __syncthreads();  // the previous window's products are read
-        // eight entries per thread and step, every load issued before the products
-        constexpr int U = 8;
-        for (int j0 = tid; j0 < cn; j0 += U * kTailThreads) {
-            int cc[U];
-            X vv[U], xx[U];
-#pragma unroll
-            for (int v = 0; v < U; v++) {
-                const int j = j0 + v * kTailThreads;
-                if (j < cn) {
-                    cc[v] = col[e0 + c0 + j];
-                    vv[v] = val[e0 + c0 + j];
-                }
-            }
-#pragma unroll
-            for (int v = 0; v < U; v++)
-                if (j0 + v * kTailThreads < cn) xx[v] = x[cc[v]];
-#pragma unroll
-            for (int v = 0; v < U; v++)
-                if (j0 + v * kTailThreads < cn) prod[j0 + v * kTailThreads] = vv[v] * xx[v];
-        }
-        __syncthreads();
-#pragma unroll
-        for (int u = 0; u < RT; u++) {
-            const int k0 = max(lo[u], c0), k1 = min(hi[u], c0 + cn);
-            const int row = tid + u * kTailThreads;
-            if (OP == OP_JACOBI && !df) {
-                for (int k = k0; k < k1; k++) {
-                    if (col[e0 + k] == row) diag[u] = val[e0 + k];
-                    else acc[u] = acc[u] + prod[k - c0];
-                }
-            } else {
-                // eight LDS reads in flight, the additions in order
-                int k = k0;
-                for (; k + 8 <= k1; k += 8) {
-                    X t[8];
-#pragma unroll
-                    for (int v = 0; v < 8; v++) t[v] = prod[k - c0 + v];
-#pragma unroll
-                    for (int v = 0; v < 8; v++) acc[u] = (OP == OP_RESIDUAL) ? acc[u] - t[v] : acc[u] + t[v];
-                }
-                for (; k < k1; k++) acc[u] = (OP == OP_RESIDUAL) ? acc[u] - prod[k - c0] : acc[u] + prod[k - c0];
-            }
-        }
-    }
-#pragma unroll
-    for (int u = 0; u < RT; u++) {
-        const int row = tid + u * kTailThreads;
-        if (row >= n) continue;
-        if (OP == OP_JACOBI) {
-            const X xo = x[row];
-            y[row] = (fabs(diag[u]) > X(1e-16)) ? ((X(1.0) - omega) * xo) + (omega * ((b[row] - acc[u]) / diag[u]))
-                                                 : xo;
-        } else if (OP == OP_ADD_INTO) {
-            y[row] = b[row] + acc[u];
-        } else {
-            y[row] = acc[u];
-            if (OP == OP_SPMV_JFZ) y2[row] = jacobi_zero_row(acc[u], dvec[row], omega);
-        }
-    }
-}
-
-// The cycle of cycle64 / cycle32 from the restriction into lv[0] to the
-// interpolation out of it, entered with every tail level's x = 0.
-template <typename X>
-__global__ __launch_bounds__(kTailThreads) void tail_cycle_kernel(TailArgs<X> a)
-{
-    // LDS: each operation's products, and the coarse LU for the solve
-    __shared__ double lds[kTailLdsBytes / sizeof(double)];
-    X* prod = reinterpret_cast<X*>(lds);
-    double* ls = lds;
-    {
-        const TailLevel<X>& C = a.lv[0];
-        if (C.jfz)
-            tail_op<OP_SPMV_JFZ, X>(prod, C.n, a.brrp, a.brcol, a.brval, a.rb, nullptr, C.b, a.omega, C.diag, C.x, 0);
-        else tail_op<OP_SPMV, X>(prod, C.n, a.brrp, a.brcol, a.brval, a.rb, nullptr, C.b, X(0), nullptr, nullptr, 0);
-        __syncthreads();
-    }
-    unsigned in_t = 0;  // bit j: level j's iterate is in t after its pre-smoothing
-    for (int j = 0; j + 1 < a.nl; j++) {
-        const TailLevel<X>& L = a.lv[j];
-        X* cur = L.x;
-        X* other = L.t;
-        if (a.sweeps <= 0) {  // no sweep to start from zero: x = 0
-            for (int i = threadIdx.x; i < L.n; i += kTailThreads) cur[i] = X(0);
-            __syncthreads();
-        }
-        for (int it = 0; it < a.sweeps; it++) {
-            if (it == 0 && L.jfz) continue;
-            if (it == 0) {
-                for (int i = threadIdx.x; i < L.n; i += kTailThreads)
-                    cur[i] = jacobi_zero_row(L.b[i], L.diag[i], a.omega);
-            } else {
-                tail_op<OP_JACOBI, X>(prod, L.n, L.arp, L.acol, L.aval, cur, L.b, other, a.omega, L.diag, nullptr,
-                                      L.adf);
-                X* tmp = cur;
-                cur = other;
-                other = tmp;
-            }
-            __syncthreads();
-        }
-        if (cur != L.x) in_t |= 1u << j;
-        tail_op<OP_RESIDUAL, X>(prod, L.n, L.arp, L.acol, L.aval, cur, L.b, L.r, X(0), nullptr, nullptr, 0);
-        __syncthreads();
-        const TailLevel<X>& C = a.lv[j + 1];
-        if (C.jfz)
-            tail_op<OP_SPMV_JFZ, X>(prod, C.n, L.rrp, L.rcol, L.rval, L.r, nullptr, C.b, a.omega, C.diag, C.x, 0);
-        else tail_op<OP_SPMV, X>(prod, C.n, L.rrp, L.rcol, L.rval, L.r, nullptr, C.b, X(0), nullptr, nullptr, 0);
-        __syncthreads();
-    }
-    {  // the coarsest level: the wavefront LU solve (FP64, rounded once on output)
-        const TailLevel<X>& C = a.lv[a.nl - 1];
-        const int n = a.coarse_n;
-        for (int t = threadIdx.x; t < n * n; t += kTailThreads) ls[t] = a.lu[t];
-        __syncthreads();
-        if (threadIdx.x < 64) {
-            const int lane = threadIdx.x;
-            const int pv = lane < n ? a.piv[lane] : 0;
-            double v = lane < n ? (double)C.b[lane] : 0.0;
-            v = coarse_lu_lane(n, ls, pv, v, lane);
-            if (lane < n) C.x[lane] = (X)v;
-        }
-        __syncthreads();
-    }
-    for (int j = a.nl - 2; j >= 0; j--) {
-        const TailLevel<X>& L = a.lv[j];
-        const TailLevel<X>& C = a.lv[j + 1];
-        X* cur = ((in_t >> j) & 1u) ? L.t : L.x;
-        X* other = ((in_t >> j) & 1u) ? L.x : L.t;
-        tail_op<OP_ADD_INTO, X>(prod, L.n, L.prp, L.pcol, L.pval, C.x, cur, other, X(0), nullptr, nullptr, 0);
-        X* tmp = cur;
-        cur = other;
-        other = tmp;
-        __syncthreads();
-        for (int it = 0; it < a.sweeps; it++) {
-            tail_op<OP_JACOBI, X>(prod, L.n, L.arp, L.acol, L.aval, cur, L.b, other, a.omega, L.diag, nullptr,
-                                  L.adf);
-            tmp = cur;
-            cur = other;
-            other = tmp;
-            __syncthreads();
-        }
-        if (cur != L.x) {
-            for (int i = threadIdx.x; i < L.n; i += kTailThreads) L.x[i] = cur[i];
-            __syncthreads();
-        }
-    }
-    tail_op<OP_ADD_INTO, X>(prod, a.nb, a.bprp, a.bpcol, a.bpval, a.lv[0].x, a.curb, a.outb, X(0), nullptr, nullptr, 0);
-}
 
 static bool multicolour(const ramd_hier_s* h);
 static bool jfz_fused(const ramd_hier_s* h, int l);
@@ -511,16 +265,29 @@ static std::vector<int> tail_candidates(const ramd_hier_s* h)
     if (h->track || multicolour(h) || nlev < 2 || h->coarse_n > kCoarseWave) return c;
     auto small = [&](int l) {
         const Level& L = h->levels[l];
-        return L.n <= kTailMaxRows && (!L.A || L.A->nnz <= kTailMaxNnz) && (!L.P || L.P->nnz <= kTailMaxNnz);
+        return L.n <= kTailMaxRows && L.A->diag_first && L.A->nnz <= kTailMaxNnz &&
+               (!L.P || L.P->nnz <= kTailMaxNnz);
     };
-    if (!small(nlev - 1)) return c;
-    int l0 = nlev - 1;
-    while (l0 - 1 >= 1 && nlev - (l0 - 1) <= kTailMax && small(l0 - 1)) l0--;
-    for (int l = l0; l < nlev; l++) {
+    // the level above: its rows and the padded P and R
+    auto outer = [&](int l) {
         const Level& B = h->levels[l - 1];
-        if (B.n <= kTailMaxOuterRows && B.P->nnz <= kTailMaxOuterNnz) c.push_back(l);
-    }
+        return B.n <= kTailMaxOuterRows && B.P->nnz <= kTailMaxOuterNnz && tail_fits(B.P) && tail_fits(B.R);
+    };
+    if (!small(nlev - 1) || !outer(nlev - 1)) return c;
+    int l0 = nlev - 1;
+    while (l0 - 1 >= 1 && nlev - (l0 - 1) <= kTailMax && small(l0 - 1) && tail_fits(h->levels[l0 - 1].A) &&
+           outer(l0 - 1) && tail_lds_bytes(h, l0 - 1, 0) <= (size_t)kTailLdsBytes)
+        l0--;
+    if (tail_lds_bytes(h, l0, 0) > (size_t)kTailLdsBytes) return c;
+    for (int l = l0; l < nlev; l++) c.push_back(l);
     return c;
+}
+
+// Packs the largest tail's levels for cycles in precision prec.
+static void pack_tail(ramd_hier_s* h, int prec)
+{
+    const std::vector<int> c = tail_candidates(h);
+    if (!c.empty()) tail_pack(h, c[0], prec);
 }
 
 // First level of the coarse tail for a cycle in precision prec (0 FP64,
@@ -545,10 +312,15 @@ static void cycle64(ramd_hier_s* h, int l, double* x, const double* b, bool x_ze
 static void cycle32(ramd_hier_s* h, int l, float* x, const float* b, bool x_zero, bool first_done);
 
 // Automatic mode: the first cycle in each precision times whole V-cycles
-// without a tail and with every candidate start, back to back and in turn
-// (seven rounds: the coarse levels stay cached between cycles as they do in
-// a solve), and keeps the candidate with the smallest median (same bits for
-// all).  Uses the fine level's own x and b vectors.
+// with the three largest tails, back to back and in turn (five rounds: the
+// coarse levels stay cached between cycles as they do in a solve), and keeps
+// the one with the smallest median (same bits for all).  No smaller tail and
+// not the cycle without one: an operation inside the tail costs 0.7-2.5 us,
+// a launch of its own 3-5 us; only the largest levels' operations, bound by
+// what one compute unit reads, are in doubt (9-point anisotropic 100^2, FP64,
+// tails from levels of 780, 362, 168, 76, 34 rows and none: 96.6, 93.2,
+// 103.8, 121.0, 134.6, 142.7 us a cycle).  Uses the fine level's own x and b
+// vectors.
 void cycle_prepare(ramd_hier_s* h, int prec)
 {
     if (prec == 1) enable_fp32(h);
@@ -558,7 +330,11 @@ void cycle_prepare(ramd_hier_s* h, int prec)
         h->tail_pick[prec] = -1;
         return;
     }
-    cand.insert(cand.begin(), -1);
+    if (cand.size() > 3) cand.resize(3);
+    if (cand.size() == 1) {
+        h->tail_pick[prec] = cand[0];
+        return;
+    }
     Level& L = h->levels[0];
     hipStream_t s = h->ctx->stream;
     std::function<void()> run;
@@ -570,7 +346,7 @@ void cycle_prepare(ramd_hier_s* h, int prec)
         run = [&] { cycle64(h, 0, L.x, L.b, true, false); };
     }
     RAMD_HIP(hipGetLastError());
-    constexpr int kRounds = 7;
+    constexpr int kRounds = 5;
     const int nc = (int)cand.size();
     std::vector<hipEvent_t> ev(2 * (size_t)nc * kRounds, nullptr);
     std::vector<float> ms(ev.size() / 2, 0.f);
@@ -612,85 +388,12 @@ void cycle_prepare(ramd_hier_s* h, int prec)
     h->tail_pick[prec] = best;
 }
 
-template <typename X>
-static const X* vals_of(const ramd_csr_s* M)
-{
-    if constexpr (sizeof(X) == 8) {
-        return M->val;
-    } else {
-        RAMD_CHECK(M->val32, RAMD_E_STATE, "coarse tail: FP32 values missing");
-        return M->val32;
-    }
-}
-
-// Launches the tail below level lb (restriction of r, the tail levels'
-// cycle, out = cur + P_lb x).
-template <typename X>
-static void launch_tail(ramd_hier_s* h, int lb, const X* r, const X* cur, X* out)
-{
-    const int nlev = (int)h->levels.size();
-    TailArgs<X> a;
-    a.nl = nlev - (lb + 1);
-    RAMD_CHECK(a.nl >= 1 && a.nl <= kTailMax, RAMD_E_STATE, "coarse tail: %d levels", a.nl);
-    const Level& B = h->levels[lb];
-    a.nb = B.n;
-    a.bprp = B.P->rowptr;
-    a.bpcol = B.P->col;
-    a.bpval = vals_of<X>(B.P);
-    a.brrp = B.R->rowptr;
-    a.brcol = B.R->col;
-    a.brval = vals_of<X>(B.R);
-    a.rb = r;
-    a.curb = cur;
-    a.outb = out;
-    a.coarse_n = h->coarse_n;
-    a.lu = h->lu;
-    a.piv = h->piv;
-    a.omega = (X)h->opts.relax_weight;
-    a.sweeps = h->opts.num_smooth_sweeps;
-    for (int j = 0; j < a.nl; j++) {
-        const int l = lb + 1 + j;
-        Level& L = h->levels[l];
-        TailLevel<X>& t = a.lv[j];
-        t.n = L.n;
-        t.jfz = (int)jfz_fused(h, l);
-        if constexpr (sizeof(X) == 8) {
-            t.x = L.x;
-            t.b = L.b;
-            t.t = L.t;
-            t.r = L.r;
-            t.diag = L.diag;
-        } else {
-            t.x = L.x32;
-            t.b = L.b32;
-            t.t = L.t32;
-            t.r = L.r32;
-            t.diag = L.diag32;
-        }
-        if (l == nlev - 1) continue;
-        t.adf = (int)L.A->diag_first;
-        t.arp = L.A->rowptr;
-        t.acol = L.A->col;
-        t.aval = vals_of<X>(L.A);
-        t.prp = L.P->rowptr;
-        t.pcol = L.P->col;
-        t.pval = vals_of<X>(L.P);
-        t.rrp = L.R->rowptr;
-        t.rcol = L.R->col;
-        t.rval = vals_of<X>(L.R);
-    }
-    RAMD_CHECK(a.lv[a.nl - 1].n == a.coarse_n, RAMD_E_STATE, "coarse tail: coarsest level has %d rows, LU %d",
-               a.lv[a.nl - 1].n, a.coarse_n);
-    hipLaunchKernelGGL((tail_cycle_kernel<X>), dim3(1), dim3(kTailThreads), 0, h->ctx->stream, a);
-    RAMD_HIP(hipGetLastError());
-}
-
 static void coarse_solve64(ramd_hier_s* h, const double* b, double* x)
 {
     const int n = h->coarse_n;
     if (n <= kCoarseWave)
         hipLaunchKernelGGL((coarse_wave_kernel<double, double>), dim3(1), dim3(64), sizeof(double) * n * n,
-                           h->ctx->stream, n, h->lu, h->piv, b, x);
+                           h->ctx->stream, n, h->lu, h->perm, b, x);
     else
         hipLaunchKernelGGL(coarse_solve_kernel, dim3(1), dim3(256), sizeof(double) * n, h->ctx->stream, n, h->lu,
                            h->piv, b, x);
@@ -868,7 +571,7 @@ static void cycle32(ramd_hier_s* h, int l, float* x, const float* b, bool x_zero
         if (n <= kCoarseWave) {
             // FP64 solve of the widened right-hand side, rounded once on output
             hipLaunchKernelGGL((coarse_wave_kernel<float, float>), dim3(1), dim3(64), sizeof(double) * n * n, s, n,
-                               h->lu, h->piv, b, x);
+                               h->lu, h->perm, b, x);
         } else {
             hipLaunchKernelGGL(to_f64, grid1(n), dim3(256), 0, s, (int64_t)n, b, h->cb);
             coarse_solve64(h, h->cb, h->cx);
@@ -959,7 +662,8 @@ static void hier_free(ramd_hier_s* h)
     dfree(h->fpart);
     h->spans.release();
     for (Level& L : h->levels) free_level(L);
-    for (void* p : {(void*)h->lu, (void*)h->piv, (void*)h->cb, (void*)h->cx, (void*)h->pr, (void*)h->pz, (void*)h->pp,
+    tail_free(h->tail);
+    for (void* p : {(void*)h->lu, (void*)h->piv, (void*)h->perm, (void*)h->cb, (void*)h->cx, (void*)h->pr, (void*)h->pz, (void*)h->pp,
                     (void*)h->pAp, (void*)h->pr32, (void*)h->pz32})
         dfree(p);
     delete h;
@@ -1220,11 +924,16 @@ static void finish_hierarchy(ramd_hier_s* h, int n, const std::vector<double>& l
     h->coarse_n = n;
     h->lu = dalloc<double>((size_t)n * n);
     h->piv = dalloc<int>((size_t)n);
+    h->perm = dalloc<int>((size_t)n);
+    std::vector<int> perm((size_t)n);  // the row swaps applied in order
+    for (int i = 0; i < n; i++) perm[i] = i;
+    for (int j = 0; j < n; j++) std::swap(perm[j], perm[piv[j]]);
     h->cb = dalloc<double>((size_t)n);
     h->cx = dalloc<double>((size_t)n);
     if (n) {
         RAMD_HIP(hipMemcpyAsync(h->lu, lu.data(), sizeof(double) * n * n, hipMemcpyHostToDevice, ctx->stream));
         RAMD_HIP(hipMemcpyAsync(h->piv, piv.data(), sizeof(int) * n, hipMemcpyHostToDevice, ctx->stream));
+        RAMD_HIP(hipMemcpyAsync(h->perm, perm.data(), sizeof(int) * n, hipMemcpyHostToDevice, ctx->stream));
     }
     const int n0 = h->levels[0].n;
     h->pr = dalloc<double>((size_t)n0);
@@ -1244,6 +953,7 @@ static void finish_hierarchy(ramd_hier_s* h, int n, const std::vector<double>& l
         }
     }
     if (multicolour(h)) build_colours(h);
+    pack_tail(h, 0);
     RAMD_HIP(hipStreamSynchronize(ctx->stream));
     for (Level& L : h->levels) L.A->borrowed = true;
     for (Level& L : h->levels)
@@ -1363,6 +1073,7 @@ void enable_fp32(ramd_hier_s* h)
     const int n0 = h->levels[0].n;
     h->pr32 = dalloc<float>((size_t)n0);
     h->pz32 = dalloc<float>((size_t)n0);
+    pack_tail(h, 1);
     RAMD_HIP(hipStreamSynchronize(s));
     h->fp32 = true;
 }

@@ -33,48 +33,84 @@ struct Level {
 // Largest coarse system solved by one wavefront (LU staged in LDS).
 constexpr int kCoarseWave = 64;
 
-// The substitutions of coarse_solve_wave: lane `lane` of the wavefront
-// holds b_i (i = lane) and its pivot pv, the LU factors are in ls; returns
-// x_i.  Every lane of the wavefront calls it.
-__device__ __forceinline__ double coarse_lu_lane(int n, const double* ls, int pv, double v, int lane)
+// Lane `lane`'s value of a double held by lane j (j uniform).
+__device__ __forceinline__ double lane_value(double v, int j)
 {
-    for (int j = 0; j < n; j++) {
-        const int p = __shfl(pv, j);
-        if (p != j) {
-            const double vj = __shfl(v, j), vp = __shfl(v, p);
-            if (lane == j) v = vp;
-            else if (lane == p) v = vj;
+    const long long b = __double_as_longlong(v);
+    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(b & 0xffffffffll), j);
+    const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(b >> 32), j);
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
+// The substitutions of coarse_solve_wave: lane `lane` of the wavefront
+// holds the permuted b_i (i = lane), the LU factors are in ls; returns x_i.
+// Every lane of the wavefront calls it.  A chain of n + n dependent steps of
+// one wavefront, bound by its instruction issue: b_j goes to all lanes
+// through readlane (a scalar register; shuffles through LDS cost about 100
+// cycles per step more), the factors' columns are read from LDS four steps
+// at a time, ahead of the chain, and there is no branch inside (steps past n
+// change nothing).  n = 34: 3000 cycles forward, 7300 back; with the
+// division by Markstein's reciprocal form instead of the general one 10100.
+__device__ __forceinline__ double coarse_lu_lane(int n, const double* ls, double v, int lane)
+{
+    constexpr int U = 4;
+    const int row = lane < n ? lane : n - 1;
+#pragma unroll 1
+    for (int j0 = 0; j0 < n; j0 += U) {
+        double c[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) c[u] = ls[row + min(j0 + u, n - 1) * n];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const double bj = lane_value(v, j0 + u);
+            const double t = v - bj * c[u];
+            v = lane > j0 + u ? t : v;  // lanes past n hold nothing
         }
     }
-    for (int j = 0; j < n; j++) {
-        const double bj = __shfl(v, j);
-        if (lane > j && lane < n) v -= bj * ls[lane + j * n];
-    }
-    for (int j = n - 1; j >= 0; j--) {
-        if (lane == j) v /= ls[j + j * n];
-        const double bj = __shfl(v, j);
-        if (lane < j) v -= bj * ls[lane + j * n];
+#pragma unroll 1
+    for (int j0 = (n - 1) / U * U; j0 >= 0; j0 -= U) {
+        double c[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) c[u] = ls[row + min(j0 + u, n - 1) * n];
+#pragma unroll
+        for (int u = U - 1; u >= 0; u--) {
+            const int j = j0 + u;
+            const double q = v / c[u];  // of use on lane j: row j of column j, the pivot
+            v = lane == j ? q : v;
+            const double bj = lane_value(v, j);
+            const double t = v - bj * c[u];
+            v = lane < (j < n ? j : 0) ? t : v;
+        }
     }
     return v;
 }
 
 // dgetrs_('N') on one right-hand side by one wavefront, n <= kCoarseWave:
-// lane i holds b_i; the row swaps, the unit-lower and the upper substitution
-// run in the reference BLAS column order with the same operations per entry
-// as the workgroup kernel (b_i -= b_j * l_ij; b_j /= u_jj), so the result is
-// bit-identical.  b and x are read and written with element stride `stride`;
-// `ls` is n*n doubles of LDS.  All 64 lanes must call it.
+// lane i holds b_perm[i] (perm: the row swaps applied in order); the
+// unit-lower and the upper substitution run in the reference BLAS column
+// order with the same operations per entry as the workgroup kernel
+// (b_i -= b_j * l_ij; b_j /= u_jj), so the result is bit-identical.  b and x
+// are read and written with element stride `stride`; `ls` is n*n doubles of
+// LDS.  All 64 lanes must call it.
 template <typename TB, typename TX>
-__device__ __forceinline__ void coarse_solve_wave(int n, const double* __restrict__ lu, const int* __restrict__ piv,
+__device__ __forceinline__ void coarse_solve_wave(int n, const double* __restrict__ lu, const int* __restrict__ perm,
                                                   const TB* __restrict__ b, TX* __restrict__ x, size_t stride,
                                                   double* ls)
 {
     const int lane = threadIdx.x;
-    for (int t = lane; t < n * n; t += 64) ls[t] = lu[t];
-    const int pv = lane < n ? piv[lane] : 0;
-    double v = lane < n ? (double)b[(size_t)lane * stride] : 0.0;
+    double v = lane < n ? (double)b[(size_t)perm[lane] * stride] : 0.0;
+    // sixteen loads in flight per lane
+    constexpr int U = 16;
+    for (int t0 = lane; t0 < n * n; t0 += 64 * U) {
+        double c[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) c[u] = lu[min(t0 + 64 * u, n * n - 1)];
+#pragma unroll
+        for (int u = 0; u < U; u++)
+            if (t0 + 64 * u < n * n) ls[t0 + 64 * u] = c[u];
+    }
     __syncthreads();
-    v = coarse_lu_lane(n, ls, pv, v, lane);
+    v = coarse_lu_lane(n, ls, v, lane);
     if (lane < n) x[(size_t)lane * stride] = (TX)v;
 }
 
@@ -111,6 +147,40 @@ ramd_csr_s* gpu_sa_subtract(const ramd_csr_s* P, const ramd_csr_s* Q);
 
 // One FP64 V-cycle from x = 0 (ParMultilevel::cycle on the fine level).
 void vcycle_from_zero(ramd_hier_s* h, double* x, const double* b);
+
+// Coarse tail (tail.hip): one operation of the tail's list.  Offsets are
+// into the workgroup's LDS vectors; the matrix's slices of 64 rows start at
+// entry slice0 of the slice table (-1: no matrix).
+enum TailType { kTailSpmv, kTailSpmvJfz, kTailResidual, kTailJacobi, kTailAdd, kTailFill, kTailCoarse };
+struct TailOp {
+    int type, n, slice0, x, b, y, y2, d, pad, unused[3];
+};
+// The tail levels' packed matrices and operation list (per precision where
+// two entries: FP64, FP32).  A tail that starts at level l runs operations
+// first[l] .. last[l]; the residual and the iterate of the level above go to
+// rb_off[l] and cb_off[l], the result comes from rb_off[l].
+struct TailPack {
+    int l0 = -1;
+    int* table = nullptr;  // device: n_ops TailOps, then the slice table
+    int n_ops = 0, n_table = 0;
+    void* cols[2] = {nullptr, nullptr};
+    void* vals[2] = {nullptr, nullptr};
+    void* diags[2] = {nullptr, nullptr};
+    int diag_off = 0, n_diag = 0;
+    size_t lds[2] = {0, 0};
+    std::vector<int> first, last, rb_off, cb_off;
+};
+constexpr int kTailLdsBytes = 160 * 1024;    // LDS of a compute unit
+constexpr int64_t kTailMaxPadded = 1 << 18;  // entries of a packed matrix, padding included
+void tail_free(TailPack* t);
+// Packs levels l0.. for cycles in precision prec (0 FP64, 1 FP32), once.
+void tail_pack(ramd_hier_s* h, int l0, int prec);
+size_t tail_lds_bytes(const ramd_hier_s* h, int l0, int prec);
+bool tail_fits(const ramd_csr_s* M);
+// Launches the tail below level lb: restriction of r, the tail levels'
+// cycle, out = cur + P_lb x.
+template <typename X>
+void launch_tail(ramd_hier_s* h, int lb, const X* r, const X* cur, X* out);
 
 struct BlockState;  // multi-vector work space (block.hip)
 void block_free(BlockState* b);
@@ -166,6 +236,8 @@ struct ramd_hier_s {
     int coarse_info = 0;   // dgetrf's info for the coarse matrix (> 0: zero pivot)
     double* lu = nullptr;  // column-major LU of the coarse matrix read column-major (A_c^T)
     int* piv = nullptr;
+    int* perm = nullptr;   // the pivots' row swaps as one permutation
+    ramd::TailPack* tail = nullptr;
     double* cb = nullptr;  // FP64 staging for the FP32 cycle's coarse solve
     double* cx = nullptr;
     double times[5] = {0, 0, 0, 0, 0};

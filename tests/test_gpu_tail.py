@@ -1,0 +1,52 @@
+"""The coarse tail's packed matrices and operation list at their edges: level
+sizes around a slice of 64 rows, coarse systems from 1 to 64 rows (the LU's
+steps of four), rows of one entry and rows past one step of eight, sweep
+counts 0 to 2, each start level, both precisions -- every cycle bit for bit
+the one with a launch per operation."""
+import numpy as np
+import pytest
+
+import raptor_amd as ra
+
+pytestmark = pytest.mark.gpu
+
+
+def laplace_1d(n, wide=1):
+    """Symmetric diagonally dominant band matrix of 2 * wide + 1 diagonals."""
+    rng = np.random.default_rng(n + wide)
+    d = np.zeros((n, n))
+    for k in range(1, min(wide, n - 1) + 1):
+        off = -rng.uniform(0.5, 1.5, n - k)
+        d += np.diag(off, k) + np.diag(off, -k)
+    d += np.diag(1.001 * np.abs(d).sum(axis=1) + 0.01)
+    rp = np.concatenate([[0], np.cumsum((d != 0).sum(axis=1))])
+    return rp.astype(np.int32), np.nonzero(d)[1].astype(np.int32), d[d != 0]
+
+
+@pytest.mark.parametrize("sweeps", [0, 1, 2])
+@pytest.mark.parametrize("n,wide,max_coarse", [(129, 1, 64), (130, 1, 33), (131, 9, 20), (257, 1, 1), (500, 4, 63),
+                                               (1000, 17, 64), (2100, 1, 40)])
+def test_tail_levels_bit_exact(ctx, n, wide, max_coarse, sweeps):
+    ml = ra.ParRugeStubenSolver(ctx, 0.25, ra.PMIS, ra.Direct, ra.Classical, ra.Jacobi)
+    ml.relax_weight = 2.0 / 3.0
+    ml.max_coarse = max_coarse
+    ml.num_smooth_sweeps = sweeps
+    ml.setup(*laplace_1d(n, wide))
+    ml.enable_fp32()
+    _, first = ml.tail_level()
+    assert first >= 1
+    b = np.random.default_rng(n).standard_normal(n)
+    b[::7] = 0.0  # exact zeros reach the coarse levels too
+    out = {}
+    for mode in [-1] + list(range(first, ml.num_levels)):
+        ml.set_tail(mode)
+        x = ra.ParVector.from_numpy(ctx, np.full(n, 3.0))
+        ml.cycle(x, ra.ParVector.from_numpy(ctx, b), x_is_zero=True)
+        x32 = ra.ParVector.from_numpy(ctx, np.full(n, 3.0, np.float32))
+        ml.cycle_fp32(x32, ra.ParVector.from_numpy(ctx, b.astype(np.float32)))
+        out[mode] = (x.numpy(), x32.numpy())
+        assert np.isfinite(out[mode][0]).all()
+    for mode in out:
+        assert np.array_equal(out[mode][0], out[-1][0]), mode
+        assert np.array_equal(out[mode][1], out[-1][1]), mode
+    ml.free()
