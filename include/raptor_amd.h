@@ -90,6 +90,10 @@ int ramd_csr_set_values(ramd_csr A, const double* val_d);
  * for square matrices of >= 4096 rows with <= 32 distinct column offsets,
  * <= 15% padding and one common per-row order); 0 when it is CSR only. */
 int ramd_csr_diagonals(ramd_csr A, int* nd);
+/* 1 when every stored diagonal has one value in all rows that store it and
+ * the diagonals are those of the 27- or 7-point box, so that the plane-march
+ * kernel reads no values (followed through ramd_csr_set_values); else 0. */
+int ramd_csr_uniform(ramd_csr A, int* uniform);
 /* Kernel variant of the stencil-diagonal form for the precision pair pp
  * (0 FP64 values and vectors, 1 FP32/FP32, 2 FP32 values/FP64 vectors):
  * mode 0 gathers x from memory, 1 stages each workgroup's x window in LDS,

@@ -187,6 +187,13 @@ class ParCSRMatrix:
         check(lib().ramd_csr_diagonals(self.h, C.byref(nd)))
         return nd.value
 
+    def uniform(self):
+        """Whether the plane-march kernel reads no values: one value per
+        diagonal on the 27- or 7-point box (ramd_csr_uniform)."""
+        u = C.c_int()
+        check(lib().ramd_csr_uniform(self.h, C.byref(u)))
+        return bool(u.value)
+
     def to_csr(self):
         rp = np.empty(self.n_rows + 1, np.int32)
         col = np.empty(max(1, self.nnz), np.int32)

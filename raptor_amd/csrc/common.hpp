@@ -214,6 +214,18 @@ struct DiaBox {
     BoxArgs args{};
     int zc[3] = {kBoxPlanes, kBoxPlanes, kBoxPlanes};  // planes per workgroup, per precision pair
 };
+// The 27- and 7-point operators' offsets in ascending order are the whole
+// box or its axes: the kernels of uniform operators have the LDS offsets of
+// such operators built in.
+constexpr int box_dz(int nd, int k) { return nd == 27 ? k / 9 - 1 : (k == 6) - (k == 0); }
+constexpr int box_dy(int nd, int k) { return nd == 27 ? k / 3 % 3 - 1 : (k == 5) - (k == 1); }
+constexpr int box_dx(int nd, int k) { return nd == 27 ? k % 3 - 1 : (k == 4) - (k == 2); }
+// diagonal of slot t: ascending, or the centre first
+constexpr int box_slot(int nd, bool diag_first, int t)
+{
+    const int c = nd / 2;
+    return !diag_first ? t : (t == 0 ? c : (t <= c ? t - 1 : t));
+}
 struct Dia {
     int nd = 0;
     int center = -1;            // diagonal index of offset 0 (-1 if none)
@@ -225,6 +237,11 @@ struct Dia {
     // geometry only), 1 = stage the x window in LDS, 0 = gather, -1 = not
     // timed yet (gather).  Chosen by timing; the result bits are the same.
     int lds_x[3] = {-1, -1, -1};
+    // every diagonal has one value in all rows that store it (constant
+    // coefficients): uval[t] is slot t's; the kernels of uniform operators
+    // read no values
+    bool uniform = false;
+    double uval[kDiaMax] = {};
     unsigned* mask = nullptr;   // device, n
     double* v64 = nullptr;      // device, dia_slots<double>(nd) * n, dia_index layout
     float* v32 = nullptr;       // device, dia_slots<float>(nd) * n (built with the FP32 copy)
@@ -346,6 +363,13 @@ void dia_box_detect(const long long* offs, int nd, int n, DiaBox& b);
 // Workgroups of the stencil-diagonal kernels of A for precision pair pp
 // (the number of per-workgroup partial sums of a fused product).
 int dia_grid(const ramd_csr_s* A, int pp);
+// The kernel of precision pair pp: lds_x[pp], and where it was not timed yet
+// (-1) the plane march for a uniform operator of a box geometry and the
+// gather for all others.
+int dia_mode(const Dia* d, int pp);
+// A uniform operator whose diagonals are the built-in ones of the box (27- or
+// 7-point), in ascending order or with the centre first (*diag_first).
+bool dia_uni_box(const Dia* d, bool* diag_first);
 // An upper bound of dia_grid over every kernel choice and precision pair.
 int dia_grid_bound(const ramd_csr_s* A);
 void dia_free(Dia* d);

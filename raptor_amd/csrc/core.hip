@@ -203,8 +203,7 @@ __global__ void dia_offsets_kernel(int n, const int* __restrict__ rp, const int*
 
 // Planes (plane k of row r at k * n + r, k = rank of the offset among the
 // sorted offs) and row masks; flags: 1 a repeated column, 2 a row not in
-// ascending diagonal order, 4 a row not in diagonal-first order, 8 a value
-// not exact in FP32.
+// ascending diagonal order, 4 a row not in diagonal-first order.
 __global__ void dia_fill_kernel(int n, int nd, int center, DiaArgs offs, const int* __restrict__ rp,
                                 const int* __restrict__ col, const double* __restrict__ val,
                                 double* __restrict__ planes, unsigned* __restrict__ mask, int* __restrict__ flags)
@@ -226,7 +225,6 @@ __global__ void dia_fill_kernel(int n, int nd, int center, DiaArgs offs, const i
         m |= 1u << k;
         const double v = val[j];
         planes[(size_t)k * n + i] = v;
-        if ((double)(float)v != v) f |= 8;
         const int rd = k == center ? -1 : k;
         if (k <= prev_a) f |= 2;
         if (rd <= prev_d) f |= 4;
@@ -235,6 +233,84 @@ __global__ void dia_fill_kernel(int n, int nd, int center, DiaArgs offs, const i
     }
     mask[i] = m;
     if (f) atomicOr(flags, f);
+}
+
+// Sets flag 8 when a value of the planes is not exact in FP32 and 16 when two
+// rows store different values (different bits) of one diagonal; ref[t]
+// receives the value's bits where slot t has one.  Each workgroup compares its
+// rows' values in LDS and touches ref once per slot.
+constexpr unsigned long long kNoRef = 0x7ff4dead0000beefull;  // a signalling NaN: never taken as uniform
+__global__ __launch_bounds__(kBlockThreads) void dia_check_kernel(int n, int nd, DiaArgs a,
+                                                                  const unsigned* __restrict__ mask,
+                                                                  const double* __restrict__ v64,
+                                                                  unsigned long long* __restrict__ ref,
+                                                                  int* __restrict__ flags)
+{
+    __shared__ unsigned long long r[kDiaMax];
+    if (threadIdx.x < kDiaMax) r[threadIdx.x] = kNoRef;
+    __syncthreads();
+    int f = 0;
+    for (int i = blockIdx.x * kBlockThreads + threadIdx.x; i < n; i += gridDim.x * kBlockThreads) {
+        const unsigned m = mask[i];
+        for (int t = 0; t < nd; t++) {
+            if (!((m >> a.ord[t]) & 1u)) continue;
+            const double v = v64[dia_index<double>(t, i, n)];
+            if ((double)(float)v != v) f |= 8;
+            const unsigned long long bits = (unsigned long long)__double_as_longlong(v);
+            unsigned long long o = r[t];
+            if (o == kNoRef) o = atomicCAS(&r[t], kNoRef, bits);
+            if ((o != kNoRef && o != bits) || bits == kNoRef) f |= 16;
+        }
+    }
+    __syncthreads();
+    if ((int)threadIdx.x < nd && r[threadIdx.x] != kNoRef) {
+        const unsigned long long o = atomicCAS(&ref[threadIdx.x], kNoRef, r[threadIdx.x]);
+        if (o != kNoRef && o != r[threadIdx.x]) f |= 16;
+    }
+    if (f) atomicOr(flags, f);
+}
+
+__global__ void dia_check_init_kernel(unsigned long long* __restrict__ ref, int* __restrict__ flags)
+{
+    ref[threadIdx.x] = kNoRef;
+    if (threadIdx.x == 0) *flags = 0;
+}
+
+// v32_exact, uniform and uval of the planes' current values.
+static void dia_check(ramd_csr_s* A)
+{
+    Dia* d = A->dia;
+    hipStream_t s = A->ctx->stream;
+    const int n = A->n_rows;
+    struct Out {
+        unsigned long long ref[kDiaMax];
+        int flags, pad;
+    } out;
+    unsigned long long* buf = dalloc<unsigned long long>(kDiaMax + 1);
+    int* flags = reinterpret_cast<int*>(buf + kDiaMax);
+    try {
+        hipLaunchKernelGGL(dia_check_init_kernel, dim3(1), dim3(kDiaMax), 0, s, buf, flags);
+        hipLaunchKernelGGL(dia_check_kernel, dim3((unsigned)std::min((n + kBlockThreads - 1) / kBlockThreads, 2048)),
+                           dim3(kBlockThreads), 0, s, n, d->nd, d->args, d->mask, d->v64, buf, flags);
+        RAMD_HIP(hipGetLastError());
+        RAMD_HIP(hipMemcpyAsync(&out, buf, sizeof(unsigned long long) * (kDiaMax + 1), hipMemcpyDeviceToHost, s));
+        RAMD_HIP(hipStreamSynchronize(s));
+    } catch (...) {
+        dfree(buf);
+        throw;
+    }
+    dfree(buf);
+    const bool exact = !(out.flags & 8), uniform = !(out.flags & 16);
+    bool same = d->v32_exact == exact && d->uniform == uniform;
+    for (int t = 0; t < d->nd && uniform; t++) {
+        double v = 0.0;
+        if (out.ref[t] != kNoRef) std::memcpy(&v, &out.ref[t], sizeof v);
+        same = same && std::memcmp(&v, &d->uval[t], sizeof v) == 0;
+        d->uval[t] = v;
+    }
+    d->v32_exact = exact;
+    d->uniform = uniform;
+    if (!same) A->forms++;  // the kernels chosen, and the values they are passed
 }
 
 void dia_box_detect(const long long* offs, int nd, int n, DiaBox& b)
@@ -337,7 +413,7 @@ bool dia_build(ramd_csr_s* A)
     int flags = 0;
     RAMD_HIP(hipMemcpyAsync(&flags, keys + kDiaTable + 2, sizeof(int), hipMemcpyDeviceToHost, s));
     RAMD_HIP(hipStreamSynchronize(s));
-    const bool all_asc = !(flags & 2), all_dfirst = !(flags & 4), exact32 = !(flags & 8);
+    const bool all_asc = !(flags & 2), all_dfirst = !(flags & 4);
     if ((flags & 1) || (!all_asc && !all_dfirst)) return false;
     Dia* d = new Dia();
     d->nd = nd;
@@ -372,7 +448,6 @@ bool dia_build(ramd_csr_s* A)
         }
         w.win = tot;
     }
-    d->v32_exact = exact32;
     dia_box_detect(offs.data(), nd, n, d->box);
     try {
         const int ns = dia_slots<double>(nd);
@@ -389,6 +464,7 @@ bool dia_build(ramd_csr_s* A)
     }
     A->dia = d;
     A->forms++;
+    dia_check(A);
     return true;
 }
 
@@ -925,18 +1001,6 @@ __global__ void dia_scatter_kernel(int n, DiaArgs a, int nd, const int* __restri
     }
 }
 
-// per-workgroup count of values that FP32 does not hold exactly
-__global__ __launch_bounds__(kBlockThreads) void inexact32_kernel(const double* __restrict__ v, int64_t m,
-                                                                  double* __restrict__ partials)
-{
-    double c = 0;
-    const int64_t stride = (int64_t)gridDim.x * kBlockThreads;
-    for (int64_t i = (int64_t)blockIdx.x * kBlockThreads + threadIdx.x; i < m; i += stride)
-        c += ((double)(float)v[i] != v[i]) ? 1.0 : 0.0;
-    c = block_sum(c);
-    if (threadIdx.x == 0) partials[blockIdx.x] = c;
-}
-
 void csr_set_values(ramd_csr_s* A, const double* val_d)
 {
     ramd_ctx ctx = A->ctx;
@@ -963,17 +1027,7 @@ void csr_set_values(ramd_csr_s* A, const double* val_d)
         hipLaunchKernelGGL(dia_scatter_kernel, dim3((n + 255) / 256), dim3(256), 0, s, n, d->args, d->nd, A->rowptr,
                            A->col, A->val, d->v64);
         RAMD_HIP(hipGetLastError());
-        const int64_t m = (int64_t)dia_slots<double>(d->nd) * n;  // padding slots hold exact zeros
-        const int g = (int)std::max<int64_t>(1, std::min<int64_t>(kRedBlocks, (m + 255) / 256));
-        double* part = ctx_partials(ctx, (size_t)g);
-        hipLaunchKernelGGL(inexact32_kernel, dim3(g), dim3(kBlockThreads), 0, s, d->v64, m, part);
-        RAMD_HIP(hipGetLastError());
-        launch_reduce_final(ctx, part, g, ctx->red_result + 8);
-        double inexact = 0;
-        fetch_scalars(ctx, ctx->red_result + 8, 1, &inexact);
-        // the FP32-value operator is chosen only while it is exact
-        if (d->v32_exact != (inexact == 0.0)) A->forms++;
-        d->v32_exact = inexact == 0.0;
+        dia_check(A);
         if (d->v32) dia_make_fp32(A);
     }
     RAMD_HIP(hipStreamSynchronize(s));
@@ -1289,6 +1343,15 @@ int ramd_csr_diagonals(ramd_csr A, int* nd)
     return guarded([&] {
         RAMD_CHECK(A && nd, RAMD_E_ARG, "ramd_csr_diagonals: NULL argument");
         *nd = A->dia ? A->dia->nd : 0;
+    });
+}
+
+int ramd_csr_uniform(ramd_csr A, int* uniform)
+{
+    return guarded([&] {
+        RAMD_CHECK(A && uniform, RAMD_E_ARG, "ramd_csr_uniform: NULL argument");
+        bool df;
+        *uniform = A->dia && dia_uni_box(A->dia, &df) ? 1 : 0;
     });
 }
 

@@ -933,11 +933,161 @@ __global__ __launch_bounds__(kBlockThreads) void dia_box_kernel(int n, int L, in
     }
 }
 
+// Uniform operators (one value per diagonal): the plane march without the
+// value streams.  What is left to read per row is the mask, the staged x and
+// b, so the kernel is bound by the vectors' traffic and, close behind, by its
+// instructions; hence the LDS offsets and the order of the diagonals are
+// compiled in (ND = 27: the whole box, ND = 7: its axes; DF: the centre
+// first), a wavefront whose rows all store every diagonal skips the selects,
+// and the row's mask and b are loaded one plane ahead.  The operations of a
+// row and their order are dia_box_kernel's: the same bits.  27 points, 256^3:
+// the outer product 420 -> 137 us, the FP32 residual and Jacobi 409 and 388
+// -> 101 and 97 us; FP64 residual at 192^3, 351 (gather) -> 58 us, 198 MB of
+// vectors and masks at 3.4 TB/s.
+template <typename X>
+struct DiaUni {
+    X v[kDiaMax];
+};
+
+template <int OP, typename X, int ND, int TX, bool DF>
+__global__ __launch_bounds__(kBlockThreads) void dia_uni_box_kernel(int n, int L, int P, int nxt, int nyt, int zc,
+                                                                   DiaUni<X> uv, const unsigned* __restrict__ mask,
+                                                                   const X* __restrict__ x, const X* __restrict__ b,
+                                                                   X* __restrict__ y, X omega,
+                                                                   double* __restrict__ dotp)
+{
+    constexpr int TY = kBlockThreads / TX;
+    constexpr int RW = TX + 2;
+    constexpr int TILE = RW * (TY + 2);
+    constexpr int PL = (TILE + 7) / 8 * 8;
+    constexpr int NLD = (TILE + kBlockThreads - 1) / kBlockThreads;
+    constexpr int C = ND / 2;  // the centre
+    constexpr unsigned FULL = ND == 32 ? ~0u : (1u << (ND & 31)) - 1u;
+    constexpr bool NEEDB = OP == OP_RESIDUAL || OP == OP_JACOBI;
+    __shared__ X xs[4 * PL];
+    const int blk = xcd_remap(blockIdx.x, gridDim.x);
+    const int xt = blk % nxt, yt = (blk / nxt) % nyt, zt = blk / (nxt * nyt);
+    const int x0 = xt * TX, y0 = yt * TY, z0 = zt * zc;
+    const int nz = n / P, ny = P / L;
+    const int z1 = min(z0 + zc, nz);
+    const int tid = threadIdx.x;
+    const int tx = tid % TX, ty = tid / TX;
+    const bool col_ok = x0 + tx < L && y0 + ty < ny;
+    const int lb = (ty + 1) * RW + tx + 1;  // the lane's own position in a plane
+    int goff[NLD];
+#pragma unroll
+    for (int i = 0; i < NLD; i++) {
+        const int e = tid + i * kBlockThreads;
+        goff[i] = (y0 + e / RW - 1) * L + x0 + e % RW - 1;
+    }
+    auto load_plane = [&](int zp, X (&r)[NLD]) {
+#pragma unroll
+        for (int i = 0; i < NLD; i++) {
+            if (tid + i * kBlockThreads < TILE) {
+                int g = zp * P + goff[i];
+                g = g < 0 ? 0 : (g >= n ? n - 1 : g);
+                r[i] = dia_gather(x, g);
+            }
+        }
+    };
+    auto store_plane = [&](int zp, const X (&r)[NLD]) {
+        X* dst = xs + (zp & 3) * PL;
+#pragma unroll
+        for (int i = 0; i < NLD; i++)
+            if (tid + i * kBlockThreads < TILE) dst[tid + i * kBlockThreads] = r[i];
+    };
+    X nx[NLD], nx0[NLD];
+    load_plane(z0 - 1, nx0);
+    load_plane(z0, nx);
+    const int c0 = (y0 + ty) * L + x0 + tx;
+    unsigned mpf = col_ok ? mask[z0 * P + c0] : 0u;
+    X bpf = NEEDB && col_ok ? b[z0 * P + c0] : X(0);
+    store_plane(z0 - 1, nx0);
+    store_plane(z0, nx);
+    load_plane(z0 + 1, nx);
+    double dsum = 0.0;
+    for (int z = z0; z < z1; z++) {
+        store_plane(z + 1, nx);
+        if (z + 2 <= z1) load_plane(z + 2, nx);
+        const int row = z * P + c0;
+        const unsigned m = mpf;
+        const X bv = bpf;
+        if (z + 1 < z1 && col_ok) {
+            mpf = mask[row + P];
+            if (NEEDB) bpf = b[row + P];
+        }
+        __syncthreads();
+        const X* pl[3] = {xs + ((z + 3) & 3) * PL + lb, xs + (z & 3) * PL + lb, xs + ((z + 1) & 3) * PL + lb};
+        X acc = OP == OP_RESIDUAL ? bv : X(0);
+        X diag = 0;
+        auto add = [&](auto all) {
+#pragma unroll
+            for (int t = 0; t < ND; t++) {
+                const int k = box_slot(ND, DF, t);
+                const bool on = decltype(all)::value || ((m >> k) & 1u);
+                if (OP == OP_JACOBI && k == C) {
+                    diag = on ? uv.v[t] : X(0);
+                    continue;
+                }
+                const X p = uv.v[t] * pl[box_dz(ND, k) + 1][box_dy(ND, k) * RW + box_dx(ND, k)];
+                const X nxt_ = OP == OP_RESIDUAL ? acc - p : acc + p;
+                acc = on ? nxt_ : acc;
+            }
+        };
+        if (__all(m == FULL)) add(std::true_type{});
+        else add(std::false_type{});
+        if (col_ok) {
+            const X xo = pl[1][0];
+            if (OP == OP_JACOBI)
+                y[row] = (m != 0u && fabs(diag) > X(1e-16)) ? ((X(1.0) - omega) * xo) + (omega * ((bv - acc) / diag))
+                                                            : xo;
+            else y[row] = acc;
+            if (OP == OP_SPMV && dotp) dsum += (double)xo * (double)acc;
+        }
+    }
+    if (OP == OP_SPMV && dotp) {
+        const double v = block_sum(dsum);
+        if (tid == 0) dotp[blk] = v;
+    }
+}
+
+bool dia_uni_box(const Dia* d, bool* diag_first)
+{
+    if (!d->uniform || d->box.L <= 0 || (d->nd != 27 && d->nd != 7) || d->center != d->nd / 2) return false;
+    const int rw = d->box.tx + 2;
+    for (int k = 0; k < d->nd; k++)
+        if (d->box.args.dz[k] != box_dz(d->nd, k) ||
+            d->box.args.rel[k] != box_dy(d->nd, k) * rw + box_dx(d->nd, k))
+            return false;
+    for (const bool df : {false, true}) {
+        bool ok = true;
+        for (int t = 0; t < d->nd; t++) ok = ok && d->args.ord[t] == box_slot(d->nd, df, t);
+        if (ok) {
+            *diag_first = df;
+            return true;
+        }
+    }
+    return false;
+}
+
+int dia_mode(const Dia* d, int pp)
+{
+    bool df;
+    return d->lds_x[pp] >= 0 ? d->lds_x[pp] : (dia_uni_box(d, &df) ? 2 : 0);
+}
+
+// Whether launches of op read no values.
+static bool dia_reads_no_values(const Dia* d, int op, int pp)
+{
+    bool df;
+    return (op == OP_SPMV || op == OP_RESIDUAL || op == OP_JACOBI) && dia_mode(d, pp) == 2 && dia_uni_box(d, &df);
+}
+
 int dia_grid(const ramd_csr_s* A, int pp)
 {
     const Dia* d = A->dia;
     const int n = A->n_rows;
-    if (d->lds_x[pp] == 2 && d->box.L > 0) {
+    if (dia_mode(d, pp) == 2 && d->box.L > 0) {
         const DiaBox& bx = d->box;
         const int ty = kBlockThreads / bx.tx;
         const int nxt = (bx.L + bx.tx - 1) / bx.tx, nyt = (bx.P / bx.L + ty - 1) / ty;
@@ -969,12 +1119,40 @@ static void launch_dia_op(const ramd_csr_s* A, const V* val, const X* x, const X
     const int n = A->n_rows;
     dim3 grid((n + kBlockThreads - 1) / kBlockThreads), block(kBlockThreads);
     const int pp = sizeof(X) == 4 ? 1 : (sizeof(V) == 4 ? 2 : 0);
-    if (d->lds_x[pp] == 2 && d->box.L > 0) {
+    const int mode = dia_mode(d, pp);
+    if (mode == 2 && d->box.L > 0) {
         const DiaBox& bx = d->box;
         const int ty = kBlockThreads / bx.tx;
         const int nxt = (bx.L + bx.tx - 1) / bx.tx, nyt = (bx.P / bx.L + ty - 1) / ty;
         const int zc = bx.zc[pp];
         const dim3 bgrid((unsigned)dia_grid(A, pp));
+        if constexpr (OP == OP_SPMV || OP == OP_RESIDUAL || OP == OP_JACOBI) {
+            bool df = false;
+            if (dia_uni_box(d, &df)) {
+                DiaUni<X> uv{};
+                for (int t = 0; t < d->nd; t++) uv.v[t] = X(d->uval[t]);
+#define DIA_UNI(NDV, TXV, DFV)                                                                                        \
+    hipLaunchKernelGGL((dia_uni_box_kernel<OP, X, NDV, TXV, DFV>), bgrid, block, 0, s, n, bx.L, bx.P, nxt, nyt, zc, uv, \
+                       d->mask, x, b, y, omega, dotp)
+#define DIA_UNI_TX(NDV, DFV)                \
+    if (bx.tx == 64) DIA_UNI(NDV, 64, DFV); \
+    else if (bx.tx == 32) DIA_UNI(NDV, 32, DFV); \
+    else DIA_UNI(NDV, 16, DFV)
+                if (d->nd == 27 && df) {
+                    DIA_UNI_TX(27, true);
+                } else if (d->nd == 27) {
+                    DIA_UNI_TX(27, false);
+                } else if (df) {
+                    DIA_UNI_TX(7, true);
+                } else {
+                    DIA_UNI_TX(7, false);
+                }
+#undef DIA_UNI_TX
+#undef DIA_UNI
+                RAMD_HIP(hipGetLastError());
+                return;
+            }
+        }
 #define DIA_BOX(NDV, TXV)                                                                                            \
     hipLaunchKernelGGL((dia_box_kernel<OP, V, X, NDV, TXV>), bgrid, block, 0, s, n, bx.L, bx.P, nxt, nyt, zc, d->args, \
                        bx.args, d->nd, d->center, d->mask, val, x, b, y, omega, dotp)
@@ -991,7 +1169,7 @@ static void launch_dia_op(const ramd_csr_s* A, const V* val, const X* x, const X
         }
 #undef DIA_BOX_TX
 #undef DIA_BOX
-    } else if (d->lds_x[pp] == 1 && d->window.win <= kDiaWin) {
+    } else if (mode == 1 && d->window.win <= kDiaWin) {
 #define DIA_LDS(NDV)                                                                                            \
     hipLaunchKernelGGL((dia_lds_kernel<OP, V, X, NDV>), grid, block, 0, s, n, d->args, d->window, d->nd, d->center, \
                        d->mask, val, x, b, y, omega, dotp)
@@ -1043,11 +1221,13 @@ static hipEvent_t prof_event(ramd_ctx ctx)
 // ideal reuse (n_cols entries), the output written once; residual, Jacobi
 // and append read one more n-vector (b, or y for append).
 // In the stencil-diagonal form the matrix costs nd * n values (padding
-// included) plus a 4-byte mask per row, and no column indices.
+// included) plus a 4-byte mask per row, and no column indices; for a uniform
+// operator the mask only.
 static double op_bytes(const ramd_csr_s* A, int op, int sv, int sx, bool dia)
 {
     double b;
-    if (dia) b = (double)A->dia->nd * A->n_rows * sv + 4.0 * A->n_rows;
+    if (dia && dia_reads_no_values(A->dia, op, sx == 4 ? 1 : (sv == 4 ? 2 : 0))) b = 4.0 * A->n_rows;
+    else if (dia) b = (double)A->dia->nd * A->n_rows * sv + 4.0 * A->n_rows;
     else b = (double)A->nnz * (sv + 4.0) + 4.0 * (A->n_rows + 1);
     b += (double)sx * A->n_cols + (double)sx * A->n_rows;
     if (op == OP_SPMV_JFZ) b += 2.0 * sx * A->n_rows;  // the diagonal read, the sweep written
@@ -1515,6 +1695,10 @@ void dia_autotune(ramd_csr_s* A, int pp)
     if (d->box.L > 0) {
         cands.push_back({2, kBoxPlanes});
         cands.push_back({2, 2 * kBoxPlanes});
+        // a uniform operator's kernel reads little besides x, and the halo
+        // planes are a larger part of that
+        bool df;
+        if (dia_uni_box(d, &df)) cands = {{2, kBoxPlanes}, {2, 2 * kBoxPlanes}, {2, 4 * kBoxPlanes}};
     }
     float best = 1e30f;
     std::pair<int, int> pick = cands[0];

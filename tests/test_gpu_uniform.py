@@ -1,0 +1,97 @@
+"""Operators with one value per diagonal: the kernels that read no values give
+the oracle's bits on 27- and 7-point grids whose lines are multiples of 64, 32,
+16 or of none, with fewer planes than a workgroup walks and more, in ascending
+order and diagonal first; one changed value turns them off and back on."""
+import numpy as np
+import pytest
+
+import checkers as K
+import raptor_amd as ra
+
+pytestmark = pytest.mark.gpu
+
+
+def grid(nx, ny, nz, pts, seed=1):
+    """27- or 7-point operator on nx x ny x nz with one random value per offset."""
+    rng = np.random.default_rng(seed)
+    i, j, k = np.meshgrid(np.arange(nx), np.arange(ny), np.arange(nz), indexing="ij")
+    i, j, k = [t.transpose(2, 1, 0).ravel() for t in (i, j, k)]  # x fastest
+    row = np.arange(nx * ny * nz)
+    rows, cols, vals = [], [], []
+    for dz in (-1, 0, 1):
+        for dy in (-1, 0, 1):
+            for dx in (-1, 0, 1):
+                if pts == 7 and abs(dx) + abs(dy) + abs(dz) > 1:
+                    continue
+                ok = (0 <= i + dx) & (i + dx < nx) & (0 <= j + dy) & (j + dy < ny) & (0 <= k + dz) & (k + dz < nz)
+                rows.append(row[ok])
+                cols.append((row + dx + nx * dy + nx * ny * dz)[ok])
+                v = rng.standard_normal() + (30.0 if dx == dy == dz == 0 else 0.0)
+                vals.append(np.full(int(ok.sum()), np.float64(np.float32(v)) if seed % 2 else v))
+    rows, cols, vals = np.concatenate(rows), np.concatenate(cols), np.concatenate(vals)
+    order = np.lexsort((cols, rows))
+    rp = np.concatenate([[0], np.cumsum(np.bincount(rows, minlength=row.size))])
+    return K.Csr(rp.astype(np.int32), cols[order].astype(np.int32), vals[order])
+
+
+def check(ctx, D, A, seed=3):
+    rng = np.random.default_rng(seed)
+    n = A.n_rows
+    x, b = rng.standard_normal(n), rng.standard_normal(n)
+    x[::5], b[::3] = -0.0, -0.0
+    y = ra.ParVector(ctx, n)
+
+    def dev(a):
+        return ra.ParVector.from_numpy(ctx, a)
+
+    def same(got, want):
+        # the sign of zero too (a NaN's sign and payload are the hardware's)
+        got, want = [np.where(np.isnan(t), np.nan, t).view(np.int64) for t in (got, want)]
+        assert np.array_equal(got, want)
+
+    D.mult(dev(x), y)
+    same(y.numpy(), K.spmv(A, x))
+    D.residual(dev(x), dev(b), y)
+    same(y.numpy(), K.residual(A, x, b))
+    same_b = dev(b)
+    D.mult_append(dev(x), same_b)
+    same(same_b.numpy(), K.spmv_append(A, x, b))
+    xj = dev(x)
+    D.jacobi(xj, dev(b), ra.ParVector(ctx, n), 2, 2.0 / 3.0)
+    same(xj.numpy(), K.jacobi(A, x, b, 2, 2.0 / 3.0))
+
+
+@pytest.mark.parametrize("pts", [27, 7])
+@pytest.mark.parametrize("dims", [(16, 16, 16), (32, 16, 17), (64, 15, 16), (65, 18, 14), (17, 19, 23), (128, 14, 13)])
+@pytest.mark.parametrize("diag_first", [False, True])
+def test_uniform_operator_bit_exact(ctx, dims, pts, diag_first):
+    A = grid(*dims, pts, seed=sum(dims))
+    if diag_first:
+        A = K.move_diag(A)
+    D = ra.ParCSRMatrix.from_csr(ctx, A.rowptr, A.col, A.val)
+    assert D.diagonals() == pts and D.uniform()
+    check(ctx, D, A)  # the rule's choice
+    for mode, planes in ((0, 0), (2, 4), (2, 5), (2, 16)):
+        for pp in (0, 2):
+            D.set_dia_staging(pp, mode, planes)
+        check(ctx, D, A)
+
+
+@pytest.mark.parametrize("what", ["one value", "signed zero", "nan"])
+def test_value_changes_turn_it_off_and_on(ctx, what):
+    A = grid(17, 16, 18, 27, seed=8)
+    D = ra.ParCSRMatrix.from_csr(ctx, A.rowptr, A.col, A.val)
+    v = A.val.copy()
+    off = np.flatnonzero(A.col != np.repeat(np.arange(A.n_rows), np.diff(A.rowptr)))
+    if what == "signed zero":
+        d = A.col - np.repeat(np.arange(A.n_rows), np.diff(A.rowptr))
+        v[d == 1] = 0.0
+        v[np.flatnonzero(d == 1)[-1]] = -0.0
+    else:
+        v[off[-1]] = np.nan if what == "nan" else np.nextafter(v[off[-1]], 9.0)
+    D.set_values(ra.ParVector.from_numpy(ctx, v))
+    assert not D.uniform()
+    check(ctx, D, K.Csr(A.rowptr, A.col, v))
+    D.set_values(ra.ParVector.from_numpy(ctx, 2.0 * A.val))
+    assert D.uniform()
+    check(ctx, D, K.Csr(A.rowptr, A.col, 2.0 * A.val))
