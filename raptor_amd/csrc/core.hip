@@ -171,34 +171,59 @@ __global__ void fill_zero_kernel(T* __restrict__ p, int64_t n)
 // Distinct column offsets of the rows, into an open-addressing table of
 // kDiaTable ints (INT_MIN = empty); *count counts insertions and *fail is set
 // past kDiaMax distinct offsets or a full probe sequence (the form is then
-// not built).
+// not built).  Every workgroup collects its rows' offsets in an LDS table and
+// merges that into the global one once: looked up in the global table for
+// every entry (loads that bypass the caches), the 27-point 128^3 operator
+// took 4.7 ms.
 constexpr int kDiaTable = 256;
-__global__ void dia_offsets_kernel(int n, const int* __restrict__ rp, const int* __restrict__ col,
-                                   int* __restrict__ keys, int* __restrict__ count, int* __restrict__ fail)
+
+// Inserts offset d; returns false when the table has no room for it.
+__device__ __forceinline__ bool dia_insert(int* keys, int* count, int* fail, int d)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n || __atomic_load_n(fail, __ATOMIC_RELAXED)) return;
-    for (int j = rp[i]; j < rp[i + 1]; j++) {
-        const int d = col[j] - i;
-        int h = (int)(((unsigned)d * 2654435761u) >> 24);
-        bool placed = false;
-        for (int probe = 0; probe < kDiaTable && !placed; probe++, h = (h + 1) & (kDiaTable - 1)) {
-            int k = __atomic_load_n(&keys[h], __ATOMIC_RELAXED);
+    int h = (int)(((unsigned)d * 2654435761u) >> 24);
+    for (int probe = 0; probe < kDiaTable; probe++, h = (h + 1) & (kDiaTable - 1)) {
+        int k = __atomic_load_n(&keys[h], __ATOMIC_RELAXED);
+        if (k == INT_MIN) {
+            k = atomicCAS(&keys[h], INT_MIN, d);
             if (k == INT_MIN) {
-                k = atomicCAS(&keys[h], INT_MIN, d);
-                if (k == INT_MIN) {
-                    if (atomicAdd(count, 1) >= kDiaMax) atomicOr(fail, 1);
-                    placed = true;
-                    continue;
-                }
+                if (atomicAdd(count, 1) >= kDiaMax) atomicOr(fail, 1);
+                return true;
             }
-            placed = k == d;
         }
-        if (!placed) {
-            atomicOr(fail, 1);
-            return;
+        if (k == d) return true;
+    }
+    return false;
+}
+
+__global__ __launch_bounds__(kBlockThreads) void dia_offsets_kernel(int n, const int* __restrict__ rp,
+                                                                    const int* __restrict__ col,
+                                                                    int* __restrict__ keys, int* __restrict__ count,
+                                                                    int* __restrict__ fail)
+{
+    __shared__ int lk[kDiaTable];
+    __shared__ int lcount, lfail;
+    for (int t = threadIdx.x; t < kDiaTable; t += kBlockThreads) lk[t] = INT_MIN;
+    if (threadIdx.x == 0) lcount = lfail = 0;
+    __syncthreads();
+    for (int i = blockIdx.x * kBlockThreads + threadIdx.x; i < n; i += gridDim.x * kBlockThreads) {
+        if (__atomic_load_n(&lfail, __ATOMIC_RELAXED)) break;
+        for (int j = rp[i]; j < rp[i + 1]; j++) {
+            const int d = col[j] - i;
+            const int k = __atomic_load_n(&lk[(int)(((unsigned)d * 2654435761u) >> 24)], __ATOMIC_RELAXED);
+            if (k == d) continue;  // at its first place already
+            if (!dia_insert(lk, &lcount, &lfail, d)) {
+                atomicOr(&lfail, 1);
+                break;
+            }
         }
     }
+    __syncthreads();
+    if (lfail) {
+        if (threadIdx.x == 0) atomicOr(fail, 1);
+        return;
+    }
+    for (int t = threadIdx.x; t < kDiaTable; t += kBlockThreads)
+        if (lk[t] != INT_MIN && !dia_insert(keys, count, fail, lk[t])) atomicOr(fail, 1);
 }
 
 // Planes (plane k of row r at k * n + r, k = rank of the offset among the
@@ -383,7 +408,7 @@ bool dia_build(ramd_csr_s* A)
     } tmp{keys};
     hipLaunchKernelGGL(fill_int_kernel, dim3(1), dim3(256), 0, s, keys, (int64_t)kDiaTable, INT_MIN);
     hipLaunchKernelGGL(fill_int_kernel, dim3(1), dim3(256), 0, s, keys + kDiaTable, (int64_t)3, 0);
-    hipLaunchKernelGGL(dia_offsets_kernel, rows, blk, 0, s, n, A->rowptr, A->col, keys, keys + kDiaTable,
+    hipLaunchKernelGGL(dia_offsets_kernel, dim3(std::min(rows.x, 2048u)), blk, 0, s, n, A->rowptr, A->col, keys, keys + kDiaTable,
                        keys + kDiaTable + 1);
     RAMD_HIP(hipGetLastError());
     std::vector<int> tab(kDiaTable + 3);
@@ -744,7 +769,7 @@ void csr_free(ramd_csr_s* A)
 // Transpose kernels: column counts, a scatter of (row, value) to each
 // column's segment by atomic cursors, then every segment put back in row
 // order (the order of a counting sort over rows ascending, which is the
-// order CSR_to_CSC gives), one thread per column.
+// order CSR_to_CSC gives).
 __global__ void transpose_count_kernel(int64_t nnz, const int* __restrict__ col, int* __restrict__ cnt)
 {
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
@@ -764,23 +789,34 @@ __global__ void transpose_scatter_kernel(int n, const int* __restrict__ rp, cons
     }
 }
 
-__global__ void transpose_sort_kernel(int m, const int* __restrict__ tp, int* __restrict__ trow,
-                                      double* __restrict__ tval)
+// Every column's (row, value) pairs in row order: a group of G lanes per
+// column, each entry's place the number of smaller rows in its column (a row
+// that stores the column twice put its entries in stored order).  One thread per column with an insertion sort
+// took 5.6 ms on average for the aggregation hierarchy of the 7-point 96^3
+// operator, whose coarse columns hold hundreds of entries.
+template <int G>
+__global__ __launch_bounds__(kBlockThreads) void transpose_rank_kernel(int m, const int* __restrict__ tp,
+                                                                       const int* __restrict__ row_in,
+                                                                       const double* __restrict__ val_in,
+                                                                       int* __restrict__ row_out,
+                                                                       double* __restrict__ val_out)
 {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
+    const int c = (blockIdx.x * kBlockThreads + threadIdx.x) / G;
     if (c >= m) return;
     const int s = tp[c], e = tp[c + 1];
-    for (int a = s + 1; a < e; a++) {  // rows of one column are distinct
-        const int r = trow[a];
-        const double v = tval[a];
-        int b = a - 1;
-        while (b >= s && trow[b] > r) {
-            trow[b + 1] = trow[b];
-            tval[b + 1] = tval[b];
-            b--;
+    for (int a = s + (int)(threadIdx.x & (G - 1)); a < e; a += G) {
+        const int r = row_in[a];
+        int rank = 0, f = s;
+        for (; f + 8 <= e; f += 8) {
+            int t[8];
+#pragma unroll
+            for (int u = 0; u < 8; u++) t[u] = row_in[f + u];
+#pragma unroll
+            for (int u = 0; u < 8; u++) rank += t[u] < r || (t[u] == r && f + u < a);
         }
-        trow[b + 1] = r;
-        tval[b + 1] = v;
+        for (; f < e; f++) rank += row_in[f] < r || (row_in[f] == r && f < a);
+        row_out[s + rank] = r;
+        val_out[s + rank] = val_in[a];
     }
 }
 
@@ -894,7 +930,7 @@ int64_t device_rowptr(ramd_ctx ctx, const int* cnt, int n, int* rp, const char* 
     return total;
 }
 
-// longest column the per-thread insertion sort takes (longer: host sort)
+// longest column that is ranked (the square of its length; longer: host sort)
 constexpr int kTransposeMaxCol = 2048;
 
 ramd_csr_s* csr_transpose(ramd_csr_s* A)
@@ -928,15 +964,37 @@ ramd_csr_s* csr_transpose(ramd_csr_s* A)
         d_val = dalloc<double>((size_t)std::max<int64_t>(nnz, 1));
         RAMD_HIP(hipMemcpyAsync(d_rp, tp.data(), sizeof(int) * (m + 1), hipMemcpyHostToDevice, s));
         if (nnz && longest <= kTransposeMaxCol) {
-            int* cursor = dalloc<int>((size_t)std::max(m, 1));
-            RAMD_HIP(hipMemcpyAsync(cursor, d_rp, sizeof(int) * m, hipMemcpyDeviceToDevice, s));
+            struct Tmp {
+                int *cursor = nullptr, *row = nullptr;
+                double* val = nullptr;
+                ~Tmp()
+                {
+                    dfree(cursor);
+                    dfree(row);
+                    dfree(val);
+                }
+            } t;
+            t.cursor = dalloc<int>((size_t)std::max(m, 1));
+            t.row = dalloc<int>((size_t)nnz);
+            t.val = dalloc<double>((size_t)nnz);
+            RAMD_HIP(hipMemcpyAsync(t.cursor, d_rp, sizeof(int) * m, hipMemcpyDeviceToDevice, s));
             hipLaunchKernelGGL(transpose_scatter_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, n,
-                               A->rowptr, A->col, A->val, cursor, d_col, d_val);
-            hipLaunchKernelGGL(transpose_sort_kernel, dim3((unsigned)((m + 255) / 256)), dim3(256), 0, s, m, d_rp,
-                               d_col, d_val);
+                               A->rowptr, A->col, A->val, t.cursor, t.row, t.val);
+            // lanes per column: about half its average length, whole
+            // wavefronts from 32 entries on
+            const int64_t avg = nnz / std::max(m, 1);
+            auto grid = [&](int g) { return dim3((unsigned)(((int64_t)m * g + kBlockThreads - 1) / kBlockThreads)); };
+            if (avg < 12)
+                hipLaunchKernelGGL((transpose_rank_kernel<4>), grid(4), dim3(kBlockThreads), 0, s, m, d_rp, t.row,
+                                   t.val, d_col, d_val);
+            else if (avg < 32)
+                hipLaunchKernelGGL((transpose_rank_kernel<16>), grid(16), dim3(kBlockThreads), 0, s, m, d_rp, t.row,
+                                   t.val, d_col, d_val);
+            else
+                hipLaunchKernelGGL((transpose_rank_kernel<64>), grid(64), dim3(kBlockThreads), 0, s, m, d_rp, t.row,
+                                   t.val, d_col, d_val);
             RAMD_HIP(hipGetLastError());
             RAMD_HIP(hipStreamSynchronize(s));
-            dfree(cursor);
         } else if (nnz) {
             // a long column: the counting sort on the host
             std::vector<int> col((size_t)nnz), trow((size_t)nnz);
