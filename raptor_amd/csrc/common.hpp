@@ -341,6 +341,12 @@ namespace ramd {
 ramd_csr_s* csr_wrap(ramd_ctx ctx, int n_rows, int n_cols, int64_t nnz, int* rowptr_d, int* col_d,
                      double* val_d, const int* rowptr_host);
 void csr_free(ramd_csr_s* A);
+// Uploads host CSR arrays (rowptr non-decreasing from 0 to nnz): columns
+// outside [0, n_cols) throw RAMD_E_ARG in the name of `who`; with `order`
+// every row is sorted, its diagonal first (nullptr when a long unsorted row
+// needs the host's sort).  Sets diag_first; no stencil-diagonal form.
+ramd_csr_s* csr_upload(ramd_ctx ctx, int n_rows, int n_cols, int64_t nnz, const int* rowptr, const int* col,
+                       const double* val, bool order, const char* who);
 // Sliced-row form: pattern (sliced_build), values of one precision copied in
 // from A->val / A->val32 (sliced_values), release (sliced_free).
 void sliced_build(ramd_csr_s* A);

@@ -493,6 +493,122 @@ bool dia_build(ramd_csr_s* A)
     return true;
 }
 
+// One thread per row; flags: 1 a column outside [0, n_cols), 2 a diagonal
+// that is not its row's first entry.  rp is non-decreasing within [0, nnz].
+__global__ void csr_check_kernel(int n, int n_cols, const int* __restrict__ rp, const int* __restrict__ col,
+                                 int* __restrict__ flags)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    int f = 0;
+    const int s = rp[i], e = rp[i + 1];
+    for (int j = s; j < e; j++) {
+        const int c = col[j];
+        if (c < 0 || c >= n_cols) f |= 1;
+        if (c == i && j > s) f |= 2;
+    }
+    if (f) atomicOr(flags, f);
+}
+
+// Every row in ascending column order (stable), then its first diagonal entry
+// moved to the front (core/matrix.cpp:587-618, 729-787), one thread per row;
+// a row that is sorted already is only shifted.  flags: 2 as above
+// afterwards (a diagonal stored twice), 4 an unsorted row of more than
+// kOrderMaxRow entries, left as it was.
+constexpr int kOrderMaxRow = 512;
+__global__ void csr_order_kernel(int n, const int* __restrict__ rp, int* __restrict__ col, double* __restrict__ val,
+                                 int* __restrict__ flags)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const int s = rp[i], e = rp[i + 1];
+    bool sorted = true;
+    for (int j = s + 1; j < e && sorted; j++) sorted = col[j - 1] <= col[j];
+    if (!sorted) {
+        if (e - s > kOrderMaxRow) {
+            atomicOr(flags, 4);
+            return;
+        }
+        for (int a = s + 1; a < e; a++) {
+            const int c = col[a];
+            const double v = val[a];
+            int b = a - 1;
+            for (; b >= s && col[b] > c; b--) {
+                col[b + 1] = col[b];
+                val[b + 1] = val[b];
+            }
+            col[b + 1] = c;
+            val[b + 1] = v;
+        }
+    }
+    int d = s;
+    while (d < e && col[d] < i) d++;
+    if (d >= e || col[d] != i) return;
+    if (d + 1 < e && col[d + 1] == i) atomicOr(flags, 2);
+    const double v = val[d];
+    for (int k = d; k > s; k--) {
+        col[k] = col[k - 1];
+        val[k] = val[k - 1];
+    }
+    col[s] = i;
+    val[s] = v;
+}
+
+// Host CSR arrays on the device (rowptr non-decreasing from 0 to nnz), their
+// columns checked there and, with `order`, the rows put in the hierarchy's
+// order; nullptr when a row needs the host's sort.  The handle has no
+// stencil-diagonal form yet.
+ramd_csr_s* csr_upload(ramd_ctx ctx, int n_rows, int n_cols, int64_t nnz, const int* rowptr, const int* col,
+                       const double* val, bool order, const char* who)
+{
+    hipStream_t s = ctx->stream;
+    struct Tmp {
+        int *rp = nullptr, *col = nullptr, *flags = nullptr;
+        double* val = nullptr;
+        ~Tmp()
+        {
+            dfree(rp);
+            dfree(col);
+            dfree(flags);
+            dfree(val);
+        }
+    } t;
+    t.rp = dalloc<int>((size_t)n_rows + 1);
+    t.col = dalloc<int>((size_t)nnz);
+    t.val = dalloc<double>((size_t)nnz);
+    t.flags = dalloc<int>(1);
+    int flags = 0;
+    auto read_flags = [&] {
+        RAMD_HIP(hipGetLastError());
+        RAMD_HIP(hipMemcpyAsync(&flags, t.flags, sizeof(int), hipMemcpyDeviceToHost, s));
+        RAMD_HIP(hipStreamSynchronize(s));
+    };
+    const dim3 grid((unsigned)((n_rows + 255) / 256));
+    RAMD_HIP(hipMemcpyAsync(t.rp, rowptr, sizeof(int) * (n_rows + 1), hipMemcpyHostToDevice, s));
+    hipLaunchKernelGGL(fill_int_kernel, dim3(1), dim3(64), 0, s, t.flags, (int64_t)1, 0);
+    if (nnz) {
+        RAMD_HIP(hipMemcpyAsync(t.col, col, sizeof(int) * nnz, hipMemcpyHostToDevice, s));
+        hipLaunchKernelGGL(csr_check_kernel, grid, dim3(256), 0, s, n_rows, n_cols, t.rp, t.col, t.flags);
+        RAMD_HIP(hipMemcpyAsync(t.val, val, sizeof(double) * nnz, hipMemcpyHostToDevice, s));
+    }
+    read_flags();
+    if (flags & 1)
+        for (int64_t j = 0; j < nnz; j++)
+            RAMD_CHECK(col[j] >= 0 && col[j] < n_cols, RAMD_E_ARG, "%s: column %d of entry %lld outside [0,%d)", who,
+                       col[j], (long long)j, n_cols);
+    if (order && nnz) {
+        hipLaunchKernelGGL(fill_int_kernel, dim3(1), dim3(64), 0, s, t.flags, (int64_t)1, 0);
+        hipLaunchKernelGGL(csr_order_kernel, grid, dim3(256), 0, s, n_rows, t.rp, t.col, t.val, t.flags);
+        read_flags();
+        if (flags & 4) return nullptr;
+    }
+    ramd_csr_s* A = csr_wrap(ctx, n_rows, n_cols, nnz, t.rp, t.col, t.val, rowptr);
+    t.rp = t.col = nullptr;
+    t.val = nullptr;
+    A->diag_first = !(flags & 2);
+    return A;
+}
+
 bool host_diag_first(int n_rows, const int* rp, const int* col)
 {
     for (int i = 0; i < n_rows; i++)
@@ -1236,20 +1352,8 @@ int ramd_csr_create(ramd_ctx ctx, int32_t n_rows, int32_t n_cols, int64_t nnz, c
                    rowptr[n_rows], (long long)nnz);
         for (int i = 0; i < n_rows; i++)
             RAMD_CHECK(rowptr[i + 1] >= rowptr[i], RAMD_E_ARG, "ramd_csr_create: rowptr decreases at row %d", i);
-        for (int64_t j = 0; j < nnz; j++)
-            RAMD_CHECK(col[j] >= 0 && col[j] < n_cols, RAMD_E_ARG,
-                       "ramd_csr_create: column %d of entry %lld outside [0,%d)", col[j], (long long)j, n_cols);
         ctx->set_current();
-        int* d_rp = dalloc<int>((size_t)n_rows + 1);
-        int* d_col = dalloc<int>((size_t)nnz);
-        double* d_val = dalloc<double>((size_t)nnz);
-        RAMD_HIP(hipMemcpyAsync(d_rp, rowptr, sizeof(int) * (n_rows + 1), hipMemcpyHostToDevice, ctx->stream));
-        if (nnz) {
-            RAMD_HIP(hipMemcpyAsync(d_col, col, sizeof(int) * nnz, hipMemcpyHostToDevice, ctx->stream));
-            RAMD_HIP(hipMemcpyAsync(d_val, val, sizeof(double) * nnz, hipMemcpyHostToDevice, ctx->stream));
-        }
-        *out = csr_wrap(ctx, n_rows, n_cols, nnz, d_rp, d_col, d_val, rowptr);
-        (*out)->diag_first = host_diag_first(n_rows, rowptr, col);
+        *out = csr_upload(ctx, n_rows, n_cols, nnz, rowptr, col, val, false, "ramd_csr_create");
         dia_build(*out);
     });
 }

@@ -960,24 +960,39 @@ static void finish_hierarchy(ramd_hier_s* h, int n, const std::vector<double>& l
         if (L.P) L.P->borrowed = true;
 }
 
-static void hier_setup(ramd_hier_s* h, Csr Af)
+static void hier_setup(ramd_hier_s* h, int n0, int64_t nnz0, const int* rowptr, const int* col, const double* val)
 {
     const ramd_amg_opts& o = h->opts;
     ramd_ctx ctx = h->ctx;
     double tstart = now_s();
     double tlevel = tstart;
-    // levels[0]->A = Af->copy(); sort(); move_diag()  (par_multilevel.hpp:141-143)
-    host::sort_rows(Af);
-    host::move_diag(Af);
-    std::vector<double> weights;
-    if (o.weights) weights.assign(o.weights, o.weights + Af.n_rows);
-    else weights = host::reference_weights(Af.n_rows, 0);
-
+    // levels[0]->A = Af->copy(); sort(); move_diag()  (par_multilevel.hpp:141-143):
+    // on the device where the setup steps are, else (or for a long unsorted
+    // row) on the host
     h->levels.emplace_back();
-    h->levels[0].A = upload(ctx, Af);
-    alloc_level_vectors(h, h->levels[0]);
-    Csr A = std::move(Af);
+    Csr A;
     bool host_A = true;  // A holds the current level (the device path skips the copy)
+    if (device_rs(o) || device_sa(o)) {
+        h->levels[0].A = csr_upload(ctx, n0, n0, nnz0, rowptr, col, val, true, "ramd_hier_setup");
+        host_A = h->levels[0].A == nullptr;
+    }
+    if (host_A) {
+        for (int64_t j = 0; j < nnz0; j++)
+            RAMD_CHECK(col[j] >= 0 && col[j] < n0, RAMD_E_ARG, "ramd_hier_setup: column %d out of range", col[j]);
+        A.n_rows = A.n_cols = n0;
+        A.rowptr.assign(rowptr, rowptr + n0 + 1);
+        A.col.assign(col, col + nnz0);
+        A.val.assign(val, val + nnz0);
+        host::sort_rows(A);
+        host::move_diag(A);
+        h->levels[0].A = upload(ctx, A);
+    } else {
+        dia_build(h->levels[0].A);
+    }
+    std::vector<double> weights;
+    if (o.weights) weights.assign(o.weights, o.weights + n0);
+    else weights = host::reference_weights(n0, 0);
+    alloc_level_vectors(h, h->levels[0]);
     // SA near-nullspace candidate (aggregation/par_smoothed_aggregation_solver.hpp:38-49)
     std::vector<double> B;
     struct DeviceB {
@@ -985,12 +1000,10 @@ static void hier_setup(ramd_hier_s* h, Csr Af)
         ~DeviceB() { dfree(p); }
     } Bd;
     if (o.solver == RAMD_SOLVER_SA) {
-        B.assign((size_t)A.n_rows, 1.0);
+        B.assign((size_t)n0, 1.0);
         if (device_sa(o)) {
-            Bd.p = dalloc<double>((size_t)std::max(A.n_rows, 1));
-            if (A.n_rows)
-                RAMD_HIP(hipMemcpyAsync(Bd.p, B.data(), sizeof(double) * A.n_rows, hipMemcpyHostToDevice,
-                                        ctx->stream));
+            Bd.p = dalloc<double>((size_t)n0);
+            RAMD_HIP(hipMemcpyAsync(Bd.p, B.data(), sizeof(double) * n0, hipMemcpyHostToDevice, ctx->stream));
         }
     }
     while (h->levels.back().n > o.max_coarse &&
@@ -1810,14 +1823,9 @@ int ramd_hier_setup(ramd_ctx ctx, int32_t n, int64_t nnz, const int32_t* rowptr,
                    "ramd_hier_setup: relax_type %d is not available on the device (RAMD_JACOBI, RAMD_MC_SOR, "
                    "RAMD_MC_SSOR; the reference's sequential SOR/SSOR is host-only)",
                    opts->relax_type);
-        for (int64_t j = 0; j < nnz; j++)
-            RAMD_CHECK(col[j] >= 0 && col[j] < n, RAMD_E_ARG, "ramd_hier_setup: column %d out of range", col[j]);
+        for (int i = 0; i < n; i++)
+            RAMD_CHECK(rowptr[i + 1] >= rowptr[i], RAMD_E_ARG, "ramd_hier_setup: rowptr decreases at row %d", i);
         ctx->set_current();
-        Csr A;
-        A.n_rows = A.n_cols = n;
-        A.rowptr.assign(rowptr, rowptr + n + 1);
-        A.col.assign(col, col + nnz);
-        A.val.assign(val, val + nnz);
         std::unique_ptr<ramd_hier_s, void (*)(ramd_hier_s*)> h(new ramd_hier_s(), hier_free);
         h->ctx = ctx;
         h->opts = *opts;
@@ -1825,7 +1833,7 @@ int ramd_hier_setup(ramd_ctx ctx, int32_t n, int64_t nnz, const int32_t* rowptr,
         if (opts->weights) {
             h->opts.weights = opts->weights;
         }
-        hier_setup(h.get(), std::move(A));
+        hier_setup(h.get(), n, nnz, rowptr, col, val);
         h->opts.weights = nullptr;
         *out = h.release();
     });
