@@ -560,9 +560,25 @@ __device__ __forceinline__ int lanes_below(unsigned long long m)
     return (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
 }
 
+// lane j's value (j the same on every lane): through a scalar register, where
+// a shuffle goes through LDS
+__device__ __forceinline__ int lane_int(int v, int j) { return __builtin_amdgcn_readlane(v, j); }
+
+// The first pass counts every row's entries and keeps the rows of up to
+// kExtKeep entries (row i's at i * kExtKeep), the second (FILL) runs on the
+// longer rows only, listed in `rows`.  27-point 128^3: about 4 entries a row;
+// computing every row twice took 62 ms in all, a wavefront waiting for each
+// neighbour's row (now loaded one neighbour ahead) and for shuffles through LDS.
+constexpr int kExtKeep = 8;
+// longest strength row whose columns are all put into the hash table (with
+// the list's kExtCols it stays below full)
+constexpr int kExtTagRow = 160;
+constexpr int kExtTag = -2;  // position of a strong column that is not in the list
+
 template <bool FILL>
 __global__ __launch_bounds__(64 * kExtWaves) void ext_interp_kernel(
-    int n, const int* __restrict__ arp, const int* __restrict__ acol, const double* __restrict__ aval,
+    int n, const int* __restrict__ rows, int* __restrict__ kcol, double* __restrict__ kval, int* __restrict__ long_rows,
+    int* __restrict__ n_long, const int* __restrict__ arp, const int* __restrict__ acol, const double* __restrict__ aval,
     const int* __restrict__ srp, const int* __restrict__ scol, const int* __restrict__ states,
     const int* __restrict__ cmap, double filter, int* __restrict__ cnt, const int* __restrict__ prp,
     int* __restrict__ pcol, double* __restrict__ pval, int* __restrict__ overflow)
@@ -572,8 +588,9 @@ __global__ __launch_bounds__(64 * kExtWaves) void ext_interp_kernel(
     __shared__ int hkey[kExtWaves][kExtHash];
     __shared__ int hpos[kExtWaves][kExtHash];
     const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int i = blockIdx.x * kExtWaves + wv;
+    int i = blockIdx.x * kExtWaves + wv;
     if (i >= n) return;  // the whole wavefront leaves together
+    if (FILL) i = __builtin_amdgcn_readfirstlane(rows[i]);
     int* lc = lcol[wv];
     double* lv = lval[wv];
     int* hk = hkey[wv];
@@ -582,13 +599,10 @@ __global__ __launch_bounds__(64 * kExtWaves) void ext_interp_kernel(
     if (st != kUnselectedState) {
         if (lane == 0) {
             if (st == kSelectedState) {
-                if (FILL) {
-                    pcol[prp[i]] = cmap[i];
-                    pval[prp[i]] = 1;
-                } else {
-                    cnt[i] = 1;
-                }
-            } else if (!FILL) {
+                cnt[i] = 1;
+                kcol[(size_t)i * kExtKeep] = cmap[i];
+                kval[(size_t)i * kExtKeep] = 1;
+            } else {
                 cnt[i] = 0;
             }
         }
@@ -600,6 +614,7 @@ __global__ __launch_bounds__(64 * kExtWaves) void ext_interp_kernel(
     bool over = false;
     // discovery (host: the first loop over S row i)
     const int s_end = srp[i + 1];
+    const bool tagged = s_end - srp[i] <= kExtTagRow;
     for (int j = srp[i] + 1; j < s_end && !over; j++) {
         const int c = scol[j];
         const int sc = states[c];
@@ -616,7 +631,13 @@ __global__ __launch_bounds__(64 * kExtWaves) void ext_interp_kernel(
                     len++;
                 }
             }
-        } else if (sc == kUnselectedState) {
+            continue;
+        }
+        if (tagged) {  // strong, not in the list
+            if (lane == 0) ext_insert(hk, hv, c, kExtTag);
+            wave_sync();
+        }
+        if (sc == kUnselectedState) {
             const int e = srp[c + 1];
             for (int b0 = srp[c] + 1; b0 < e; b0 += 64) {
                 const int k = b0 + lane;
@@ -661,8 +682,8 @@ __global__ __launch_bounds__(64 * kExtWaves) void ext_interp_kernel(
         const int cj = inj ? acol[jl] : -1;
         const double vj = inj ? aval[jl] : 0.0;
         const int idxj = inj ? ext_lookup(hk, hv, cj) : -1;
-        bool strong = false;
-        for (int t0 = srp[i] + 1; t0 < s_end; t0 += 64) {
+        bool strong = tagged && idxj == kExtTag;
+        for (int t0 = srp[i] + 1; t0 < s_end && !tagged; t0 += 64) {
             const int sc = t0 + lane < s_end ? scol[t0 + lane] : -2;
             const int tn = min(64, s_end - t0);
             for (int t = 0; t < tn; t++) {
@@ -680,28 +701,43 @@ __global__ __launch_bounds__(64 * kExtWaves) void ext_interp_kernel(
             dgj = aval[skj];
         }
         const int nj = min(64, end - c0);
+        const unsigned long long strong_m = __ballot(strong), list_m = __ballot(idxj >= 0);
+        unsigned long long fnb_m = __ballot(fnb);
+        // the row of the next F neighbour in order, loaded ahead of its turn
+        double vn = 0.0;
+        int cn = -1;
+        auto load_next = [&] {
+            if (!fnb_m) return;
+            const int t = __ffsll((long long)fnb_m) - 1;
+            const int k = lane_int(skj, t) + 1 + lane;
+            const bool in = k < lane_int(ekj, t);
+            vn = in ? aval[k] : 0.0;
+            cn = in ? acol[k] : -1;
+        };
+        load_next();
         for (int t = 0; t < nj; t++) {
-            const double v = __shfl(vj, t);
-            const int idx = __shfl(idxj, t);
-            if (idx >= 0) {
-                if (lane == 0) lv[idx] += v;
-            } else if (__shfl((int)strong, t)) {
-                if (!__shfl((int)fnb, t)) continue;  // a strong neighbour that is not F
-                const int sk = __shfl(skj, t), ek = __shfl(ekj, t);
-                const int sign = __shfl(dgj, t) > 0 ? 1 : -1;
+            const double v = lane_value(vj, t);
+            if ((list_m >> t) & 1) {
+                if (lane == 0) lv[lane_int(idxj, t)] += v;
+            } else if ((strong_m >> t) & 1) {
+                if (!((fnb_m >> t) & 1)) continue;  // a strong neighbour that is not F
+                const int sk = lane_int(skj, t), ek = lane_int(ekj, t);
+                const int sign = lane_value(dgj, t) > 0 ? 1 : -1;
+                const double v0 = vn;
+                const int ck0 = cn;
+                fnb_m &= fnb_m - 1;
+                load_next();
                 // entries of the neighbour's row that count: opposite sign to
                 // its diagonal, column i or a column of the list; their sum in
                 // entry order
                 if (ek - sk - 1 <= 64) {
-                    const int k = sk + 1 + lane;
-                    const bool in = k < ek;
-                    const double vk = in ? aval[k] : 0.0;
-                    const int ck = in ? acol[k] : -1;
-                    const bool neg = in && vk * sign < 0;
+                    const double vk = v0;
+                    const int ck = ck0;
+                    const bool neg = sk + 1 + lane < ek && vk * sign < 0;
                     const int pk = (neg && ck != i) ? ext_lookup(hk, hv, ck) : -1;
                     double col_sum = 0;
                     for (unsigned long long m = __ballot(neg && (ck == i || pk >= 0)); m; m &= m - 1)
-                        col_sum += __shfl(vk, __ffsll((long long)m) - 1);
+                        col_sum += lane_value(vk, __ffsll((long long)m) - 1);
                     if (fabs(col_sum) < kSetupZeroTol) {
                         weak_sum += v;
                     } else {
@@ -709,7 +745,7 @@ __global__ __launch_bounds__(64 * kExtWaves) void ext_interp_kernel(
                         // distinct columns: each entry of the list gets at most one addition here
                         if (pk >= 0) lv[pk] += (col_sum * vk);
                         const unsigned long long mi = __ballot(neg && ck == i);
-                        if (mi) weak_sum += (col_sum * __shfl(vk, __ffsll((long long)mi) - 1));
+                        if (mi) weak_sum += (col_sum * lane_value(vk, __ffsll((long long)mi) - 1));
                     }
                 } else {
                     double col_sum = 0;
@@ -739,7 +775,7 @@ __global__ __launch_bounds__(64 * kExtWaves) void ext_interp_kernel(
                         }
                     }
                 }
-            } else if (__shfl(stj, t) != kNoNeighborsState) {
+            } else if (lane_int(stj, t) != kNoNeighborsState) {
                 weak_sum += v;
             }
             wave_sync();
@@ -783,7 +819,29 @@ __global__ __launch_bounds__(64 * kExtWaves) void ext_interp_kernel(
             }
         } else {
             cnt[i] = kept;
+            if (kept > kExtKeep) {
+                long_rows[atomicAdd(n_long, 1)] = i;
+            } else {
+                for (int k = 0; k < kept; k++) {
+                    kcol[(size_t)i * kExtKeep + k] = cmap[lc[k]];
+                    kval[(size_t)i * kExtKeep + k] = lv[k];
+                }
+            }
         }
+    }
+}
+
+// The kept rows to their places.
+__global__ void ext_place_kernel(int n, const int* __restrict__ prp, const int* __restrict__ kcol,
+                                 const double* __restrict__ kval, int* __restrict__ pcol, double* __restrict__ pval)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const int o = prp[i], len = prp[i + 1] - o;
+    if (len > kExtKeep) return;
+    for (int k = 0; k < len; k++) {
+        pcol[o + k] = kcol[(size_t)i * kExtKeep + k];
+        pval[o + k] = kval[(size_t)i * kExtKeep + k];
     }
 }
 
@@ -1028,50 +1086,64 @@ static ramd_csr_s* gpu_interpolation(const ramd_csr_s* A, const ramd_csr_s* S, c
     for (int i = 0; i < n; i++)
         if (states_h[i] == kSelectedState) cmap[i] = nc++;
     struct Bufs {
-        int *cmap = nullptr, *cnt = nullptr, *over = nullptr;
+        int *cmap = nullptr, *cnt = nullptr, *over = nullptr, *kcol = nullptr, *long_rows = nullptr;
+        double* kval = nullptr;
         ~Bufs()
         {
-            dfree(cmap);
-            dfree(cnt);
-            dfree(over);
+            for (int* p : {cmap, cnt, over, kcol, long_rows}) dfree(p);
+            dfree(kval);
         }
     } b;
     b.cmap = dalloc<int>((size_t)std::max(n, 1));
     b.cnt = dalloc<int>((size_t)std::max(n, 1));
-    b.over = dalloc<int>(1);
+    b.over = dalloc<int>(2);  // overflow, rows past kExtKeep
     RAMD_HIP(hipMemcpyAsync(b.cmap, cmap.data(), sizeof(int) * n, hipMemcpyHostToDevice, s));
-    RAMD_HIP(hipMemsetAsync(b.over, 0, sizeof(int), s));
-    const dim3 grid((unsigned)std::max(1, (n + kExtWaves - 1) / kExtWaves)), block(64 * kExtWaves);
-    // count pass (cnt) or fill pass (prp, pcol, pval)
-    auto launch = [&](int* cnt, const int* prp, int* pcol, double* pval) {
+    RAMD_HIP(hipMemsetAsync(b.over, 0, 2 * sizeof(int), s));
+    auto grid = [](int rows) { return dim3((unsigned)std::max(1, (rows + kExtWaves - 1) / kExtWaves)); };
+    const dim3 block(64 * kExtWaves);
+    if (!modc) {
+        b.kcol = dalloc<int>((size_t)std::max(n, 1) * kExtKeep);
+        b.kval = dalloc<double>((size_t)std::max(n, 1) * kExtKeep);
+        b.long_rows = dalloc<int>((size_t)std::max(n, 1));
+    }
+    // count pass (cnt), or fill pass (prp, pcol, pval) over `rows` rows
+    auto launch = [&](int rows, int* cnt, const int* prp, int* pcol, double* pval) {
         if (modc) {
             if (cnt)
-                hipLaunchKernelGGL((modc_interp_kernel<false>), grid, block, 0, s, n, A->rowptr, A->col, A->val,
+                hipLaunchKernelGGL((modc_interp_kernel<false>), grid(rows), block, 0, s, n, A->rowptr, A->col, A->val,
                                    S->rowptr, S->col, S->val, states_d, b.cmap, cnt, prp, pcol, pval, b.over);
             else
-                hipLaunchKernelGGL((modc_interp_kernel<true>), grid, block, 0, s, n, A->rowptr, A->col, A->val,
+                hipLaunchKernelGGL((modc_interp_kernel<true>), grid(rows), block, 0, s, n, A->rowptr, A->col, A->val,
                                    S->rowptr, S->col, S->val, states_d, b.cmap, cnt, prp, pcol, pval, b.over);
         } else {
             if (cnt)
-                hipLaunchKernelGGL((ext_interp_kernel<false>), grid, block, 0, s, n, A->rowptr, A->col, A->val,
-                                   S->rowptr, S->col, states_d, b.cmap, filter, cnt, prp, pcol, pval, b.over);
+                hipLaunchKernelGGL((ext_interp_kernel<false>), grid(rows), block, 0, s, rows, nullptr, b.kcol, b.kval,
+                                   b.long_rows, b.over + 1, A->rowptr, A->col, A->val, S->rowptr, S->col, states_d,
+                                   b.cmap, filter, cnt, prp, pcol, pval, b.over);
             else
-                hipLaunchKernelGGL((ext_interp_kernel<true>), grid, block, 0, s, n, A->rowptr, A->col, A->val,
-                                   S->rowptr, S->col, states_d, b.cmap, filter, cnt, prp, pcol, pval, b.over);
+                hipLaunchKernelGGL((ext_interp_kernel<true>), grid(rows), block, 0, s, rows, b.long_rows, nullptr,
+                                   nullptr, nullptr, nullptr, A->rowptr, A->col, A->val, S->rowptr, S->col, states_d,
+                                   b.cmap, filter, cnt, prp, pcol, pval, b.over);
         }
         RAMD_HIP(hipGetLastError());
     };
-    launch(b.cnt, nullptr, nullptr, nullptr);
-    int over = 0;
-    RAMD_HIP(hipMemcpyAsync(&over, b.over, sizeof(int), hipMemcpyDeviceToHost, s));
+    launch(n, b.cnt, nullptr, nullptr, nullptr);
+    int over[2] = {0, 0};
+    RAMD_HIP(hipMemcpyAsync(over, b.over, sizeof over, hipMemcpyDeviceToHost, s));
     std::vector<int> rp = host_rowptr(ctx, b.cnt, n);  // synchronizes
-    if (over) return nullptr;
+    if (over[0]) return nullptr;
     const int64_t nnz = rp[n];
     int* d_rp = dalloc<int>((size_t)n + 1);
     int* d_col = dalloc<int>((size_t)std::max<int64_t>(nnz, 1));
     double* d_val = dalloc<double>((size_t)std::max<int64_t>(nnz, 1));
     RAMD_HIP(hipMemcpyAsync(d_rp, rp.data(), sizeof(int) * (n + 1), hipMemcpyHostToDevice, s));
-    launch(nullptr, d_rp, d_col, d_val);
+    if (modc) {
+        launch(n, nullptr, d_rp, d_col, d_val);
+    } else {
+        hipLaunchKernelGGL(ext_place_kernel, rows_grid(n), dim3(256), 0, s, n, d_rp, b.kcol, b.kval, d_col, d_val);
+        RAMD_HIP(hipGetLastError());
+        if (over[1]) launch(over[1], nullptr, d_rp, d_col, d_val);
+    }
     RAMD_HIP(hipStreamSynchronize(s));
     return csr_wrap(ctx, n, nc, nnz, d_rp, d_col, d_val, rp.data());
 }
