@@ -1476,7 +1476,7 @@ __global__ void flush_kernel(uint4* __restrict__ p, int64_t n)
 float cold_median_ms(ramd_ctx ctx, const std::function<void()>& run, int reps, size_t op_bytes)
 {
     hipStream_t s = ctx->stream;
-    const bool flush = op_bytes < kFlushBytes;
+    const bool flush = op_bytes >= kFlushMin && op_bytes < kFlushBytes;
     if (flush && !ctx->flush_buf) ctx->flush_buf = dmalloc(kFlushBytes);
     std::vector<hipEvent_t> ev(2 * (size_t)reps, nullptr);
     std::vector<float> ms((size_t)reps, 0.f);
@@ -1542,9 +1542,9 @@ void csr_autotune(ramd_csr_s* A, int prec)
     const int op = A->n_rows == A->n_cols ? OP_RESIDUAL : OP_SPMV;
     ramd_csr_s::RowBlocks best = A->rb[prec];
     float best_ms = 1e30f;
-    // the median of seven launches for small operators, whose single
+    // the median of five launches for small operators, whose single
     // launches are too short to rank reliably, three above
-    const int reps = A->nnz < (int64_t)4 << 20 ? 7 : 3;
+    const int reps = A->nnz < (int64_t)4 << 20 ? 5 : 3;
     const size_t op_b = (size_t)A->nnz * (4 + w) + ((size_t)A->n_rows * 2 + (size_t)A->n_cols) * w;
     auto time_ms = [&] {
         return cold_median_ms(ctx, [&] {
@@ -1719,9 +1719,9 @@ void dia_autotune(ramd_csr_s* A, int pp)
                 launch_dia<double, double>(A, d->v64, op, (const double*)t.x, (const double*)t.b, (double*)t.y, 0.5,
                                            s, nullptr);
         };
-        // medians of seven launches: the candidates differ by a few percent
-        float ms = cold_median_ms(ctx, [&] { run(pp == 2 ? OP_SPMV : OP_RESIDUAL); }, 7, op_b);
-        if (pp != 2) ms += cold_median_ms(ctx, [&] { run(OP_JACOBI); }, 7, op_b);
+        // medians of five launches: the candidates differ by a few percent
+        float ms = cold_median_ms(ctx, [&] { run(pp == 2 ? OP_SPMV : OP_RESIDUAL); }, 5, op_b);
+        if (pp != 2) ms += cold_median_ms(ctx, [&] { run(OP_JACOBI); }, 5, op_b);
         if (ms < best) {
             best = ms;
             pick = c;
