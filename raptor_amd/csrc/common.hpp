@@ -337,9 +337,11 @@ struct ramd_csr_s {
 };
 
 namespace ramd {
-// Creates a handle around device arrays the library already owns.
+// Creates a handle around device arrays the library already owns.  temp: a
+// matrix that is never applied to vectors gets no row blocks, nor a host copy
+// of its row pointers that is not given (both are host loops over its rows).
 ramd_csr_s* csr_wrap(ramd_ctx ctx, int n_rows, int n_cols, int64_t nnz, int* rowptr_d, int* col_d,
-                     double* val_d, const int* rowptr_host);
+                     double* val_d, const int* rowptr_host, bool temp = false);
 void csr_free(ramd_csr_s* A);
 // Uploads host CSR arrays (rowptr non-decreasing from 0 to nnz): columns
 // outside [0, n_cols) throw RAMD_E_ARG in the name of `who`; with `order`

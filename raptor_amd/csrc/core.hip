@@ -74,7 +74,7 @@ std::vector<int> make_row_blocks(const int* rp, int n_rows, int cap)
 }
 
 ramd_csr_s* csr_wrap(ramd_ctx ctx, int n_rows, int n_cols, int64_t nnz, int* rowptr_d, int* col_d,
-                     double* val_d, const int* rowptr_host)
+                     double* val_d, const int* rowptr_host, bool temp)
 {
     static std::atomic<uint64_t> next_uid{1};
     ramd_csr_s* A = new ramd_csr_s();
@@ -88,12 +88,13 @@ ramd_csr_s* csr_wrap(ramd_ctx ctx, int n_rows, int n_cols, int64_t nnz, int* row
     A->val = val_d;
     if (rowptr_host) {
         A->h_rowptr.assign(rowptr_host, rowptr_host + n_rows + 1);
-    } else {
+    } else if (!temp) {
         A->h_rowptr.resize((size_t)n_rows + 1);
         RAMD_HIP(hipMemcpyAsync(A->h_rowptr.data(), rowptr_d, sizeof(int) * (n_rows + 1),
                                 hipMemcpyDeviceToHost, ctx->stream));
         RAMD_HIP(hipStreamSynchronize(ctx->stream));
     }
+    if (temp) return A;
     std::vector<int> blocks = make_row_blocks(A->h_rowptr.data(), n_rows, kStreamCap);
     A->n_blocks = (int)blocks.size() - 1;
     A->blocks = dalloc<int>(blocks.size());

@@ -726,8 +726,8 @@ static ramd_csr_s* rs_level_device(ramd_hier_s* h, int level, const double* weig
     Level& L = h->levels[level];
     const int n = L.n;
     double t0 = now_s();
-    ramd_csr_s* S = o.strength_type == RAMD_SYMMETRIC ? gpu_symmetric_strength(L.A, o.strong_threshold)
-                                                      : gpu_classical_strength(L.A, o.strong_threshold);
+    ramd_csr_s* S = o.strength_type == RAMD_SYMMETRIC ? gpu_symmetric_strength(L.A, o.strong_threshold, true)
+                                                      : gpu_classical_strength(L.A, o.strong_threshold, true);
     int* st = nullptr;
     ramd_csr_s* P = nullptr;
     try {
@@ -862,8 +862,8 @@ static ramd_csr_s* sa_level_device(ramd_hier_s* h, int level, const double* weig
     Level& L = h->levels[level];
     const int n = L.n;
     double t0 = now_s();
-    ramd_csr_s* S = o.strength_type == RAMD_SYMMETRIC ? gpu_symmetric_strength(L.A, o.strong_threshold)
-                                                      : gpu_classical_strength(L.A, o.strong_threshold);
+    ramd_csr_s* S = o.strength_type == RAMD_SYMMETRIC ? gpu_symmetric_strength(L.A, o.strong_threshold, true)
+                                                      : gpu_classical_strength(L.A, o.strong_threshold, true);
     int *st = nullptr, *agg = nullptr;
     double* R = nullptr;
     ramd_csr_s *P = nullptr, *M = nullptr, *Q = nullptr;
@@ -882,7 +882,7 @@ static ramd_csr_s* sa_level_device(ramd_hier_s* h, int level, const double* weig
         if (o.prolong_smooth_steps > 0) {
             M = gpu_sa_scaled_operator(L.A, o.prolong_weight);
             for (int step = 0; step < o.prolong_smooth_steps; step++) {
-                Q = spgemm(M, P);
+                Q = spgemm(M, P, true);
                 ramd_csr_s* next = gpu_sa_subtract(P, Q);
                 csr_free(Q);
                 Q = nullptr;

@@ -11,7 +11,8 @@ struct ramd_hier_s;
 
 namespace ramd {
 
-ramd_csr_s* spgemm(ramd_csr_s* A, ramd_csr_s* B);
+// temp: a product that is only multiplied by other sparse matrices, or read
+ramd_csr_s* spgemm(ramd_csr_s* A, ramd_csr_s* B, bool temp = false);
 ramd_csr_s* galerkin(ramd_csr_s* A, ramd_csr_s* P);
 
 struct Level {
@@ -115,8 +116,9 @@ __device__ __forceinline__ void coarse_solve_wave(int n, const double* __restric
 }
 
 // Device setup steps (setup_gpu.hip), bit-identical to the host ones.
-ramd_csr_s* gpu_classical_strength(ramd_csr_s* A, double theta);
-ramd_csr_s* gpu_symmetric_strength(ramd_csr_s* A, double theta);
+// (temp: S is only read by the other setup steps)
+ramd_csr_s* gpu_classical_strength(ramd_csr_s* A, double theta, bool temp = false);
+ramd_csr_s* gpu_symmetric_strength(ramd_csr_s* A, double theta, bool temp = false);
 // PMIS on the device; prior_states (host, n; nullptr for plain PMIS) are
 // states an earlier pass decided (HMIS), applied before the first round
 void gpu_split_pmis(const ramd_csr_s* S, const double* weights, int* states, const int* prior_states = nullptr);

@@ -94,7 +94,7 @@ static std::vector<int> host_rowptr(ramd_ctx ctx, const int* d_cnt, int n)
 
 static dim3 rows_grid(int n) { return dim3((unsigned)std::max(1, (n + 255) / 256)); }
 
-ramd_csr_s* gpu_classical_strength(ramd_csr_s* A, double theta)
+ramd_csr_s* gpu_classical_strength(ramd_csr_s* A, double theta, bool temp)
 {
     ramd_ctx ctx = A->ctx;
     hipStream_t s = ctx->stream;
@@ -119,7 +119,7 @@ ramd_csr_s* gpu_classical_strength(ramd_csr_s* A, double theta)
     hipLaunchKernelGGL((strength_kernel<true>), rows_grid(n), dim3(256), 0, s, n, A->rowptr, A->col, A->val, theta,
                        nullptr, d_rp, d_col, d_val);
     RAMD_HIP(hipGetLastError());
-    return csr_wrap(ctx, n, A->n_cols, nnz, d_rp, d_col, d_val, rp.data());
+    return csr_wrap(ctx, n, A->n_cols, nnz, d_rp, d_col, d_val, rp.data(), temp);
 }
 
 // ---------------------------------------------------------------------------
@@ -198,7 +198,7 @@ __global__ void sym_strength_kernel(int n, const int* __restrict__ rp, const int
     if (!FILL) cnt[i] = o;
 }
 
-ramd_csr_s* gpu_symmetric_strength(ramd_csr_s* A, double theta)
+ramd_csr_s* gpu_symmetric_strength(ramd_csr_s* A, double theta, bool temp)
 {
     ramd_ctx ctx = A->ctx;
     hipStream_t s = ctx->stream;
@@ -232,7 +232,7 @@ ramd_csr_s* gpu_symmetric_strength(ramd_csr_s* A, double theta)
                        b.neg, b.scale, nullptr, d_rp, d_col, d_val);
     RAMD_HIP(hipGetLastError());
     RAMD_HIP(hipStreamSynchronize(s));  // the scratch buffers are freed on return
-    return csr_wrap(ctx, n, A->n_cols, nnz, d_rp, d_col, d_val, rp.data());
+    return csr_wrap(ctx, n, A->n_cols, nnz, d_rp, d_col, d_val, rp.data(), temp);
 }
 
 // ---------------------------------------------------------------------------
@@ -1534,7 +1534,7 @@ ramd_csr_s* gpu_sa_scaled_operator(const ramd_csr_s* A, double omega)
     if (nnz) RAMD_HIP(hipMemcpyAsync(d_col, A->col, sizeof(int) * nnz, hipMemcpyDeviceToDevice, s));
     hipLaunchKernelGGL(sa_scale_kernel, rows_grid(n), dim3(256), 0, s, n, A->rowptr, A->val, omega, d_val);
     RAMD_HIP(hipGetLastError());
-    return csr_wrap(ctx, n, A->n_cols, nnz, d_rp, d_col, d_val, A->h_rowptr.data());
+    return csr_wrap(ctx, n, A->n_cols, nnz, d_rp, d_col, d_val, A->h_rowptr.data(), true);
 }
 
 // Row i of P - Q (the reference's subtract: P's row then Q's row negated,

@@ -19,7 +19,7 @@
 #include <algorithm>
 #include <numeric>
 
-#include "common.hpp"
+#include "hier.hpp"
 
 namespace ramd {
 
@@ -65,18 +65,93 @@ __device__ __forceinline__ int grp_prefix(bool pred)
     return __popcll(m & ((1ull << lane) - 1));
 }
 
-// products per row: sum over j in A_i of nnz(B_j)
-__global__ void count_products(int m, const int* __restrict__ arp, const int* __restrict__ acol,
-                               const int* __restrict__ brp, int64_t* __restrict__ out)
+// Values held by lane t of the caller's group.
+template <int G>
+__device__ __forceinline__ int grp_value(int v, int t)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= m) return;
+    return G == kWave ? __builtin_amdgcn_readlane(v, t) : __shfl(v, t, G);
+}
+template <int G>
+__device__ __forceinline__ double grp_value(double v, int t)
+{
+    return G == kWave ? lane_value(v, t) : __shfl(v, t, G);
+}
+
+// LDS accesses of the wavefront in program order (it executes them so; this
+// keeps the compiler from moving them).
+__device__ __forceinline__ void lds_order()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// Walks the products of a row with a group of G lanes: for each entry a_ij in
+// stored order, fn(bcol, bval, a) on the lanes that hold entries of row j of
+// B, G at a time.  What bounds it is the chain entry -> row bounds -> row j ->
+// table, so the entries and their rows' bounds are read G at a time, one per
+// lane, and the first G entries of the next row j are loaded before the
+// current one is processed.
+template <int G, bool VALUES, typename F>
+__device__ __forceinline__ void walk_products(int row, const int* __restrict__ arp, const int* __restrict__ acol,
+                                              const double* __restrict__ aval, const int* __restrict__ brp,
+                                              const int* __restrict__ bcol, const double* __restrict__ bval, F fn)
+{
+    const int lane = grp_lane<G>();
+    const int e = arp[row + 1];
+    for (int j0 = arp[row]; j0 < e; j0 += G) {
+        const int nj = min(G, e - j0);
+        int bs = 0, be = 0;
+        double av = 0.0;
+        if (lane < nj) {
+            const int c = acol[j0 + lane];
+            if (VALUES) av = aval[j0 + lane];
+            bs = brp[c];
+            be = brp[c + 1];
+        }
+        int s = grp_value<G>(bs, 0), t1 = grp_value<G>(be, 0);
+        int kc = -1;
+        double kv = 0.0;
+        if (s + lane < t1) {
+            kc = bcol[s + lane];
+            if (VALUES) kv = bval[s + lane];
+        }
+        for (int t = 0; t < nj; t++) {
+            const int s0 = s, e0 = t1;
+            const int c0 = kc;
+            const double v0 = kv;
+            const double a = VALUES ? grp_value<G>(av, t) : 0.0;
+            if (t + 1 < nj) {
+                s = grp_value<G>(bs, t + 1);
+                t1 = grp_value<G>(be, t + 1);
+                if (s + lane < t1) {
+                    kc = bcol[s + lane];
+                    if (VALUES) kv = bval[s + lane];
+                }
+            }
+            if (s0 + lane < e0) fn(c0, v0, a);
+            for (int k = s0 + G + lane; k < e0; k += G) fn(bcol[k], VALUES ? bval[k] : 0.0, a);
+            // every lane's update for this a_ij lands before the next a_ij's
+            lds_order();
+        }
+    }
+}
+
+// products per row: sum over j in A_i of nnz(B_j); eight lanes per row
+constexpr int kCountGroup = 8;
+__global__ __launch_bounds__(256) void count_products(int m, const int* __restrict__ arp,
+                                                      const int* __restrict__ acol, const int* __restrict__ brp,
+                                                      int64_t* __restrict__ out)
+{
+    const int i = (int)(((int64_t)blockIdx.x * 256 + threadIdx.x) / kCountGroup);
+    if (i >= m) return;  // a group leaves together
     int64_t s = 0;
-    for (int j = arp[i]; j < arp[i + 1]; j++) {
+    for (int j = arp[i] + grp_lane<kCountGroup>(); j < arp[i + 1]; j += kCountGroup) {
         const int c = acol[j];
         s += brp[c + 1] - brp[c];
     }
-    out[i] = s;
+#pragma unroll
+    for (int off = kCountGroup / 2; off > 0; off >>= 1) s += __shfl_xor(s, off, kCountGroup);
+    if (grp_lane<kCountGroup>() == 0) out[i] = s;
 }
 
 // insert key into open-addressing table (size T, power of two); returns slot
@@ -104,13 +179,11 @@ __device__ void symbolic_row(int row, int* keys, int T, const int* __restrict__ 
 {
     const int lane = grp_lane<G>();
     for (int t = lane; t < T; t += G) keys[t] = -1;
-    __builtin_amdgcn_wave_barrier();
-    for (int j = arp[row]; j < arp[row + 1]; j++) {
-        const int c = acol[j];
-        for (int t = brp[c] + lane; t < brp[c + 1]; t += G) hash_insert(keys, T, bcol[t]);
-    }
-    __builtin_amdgcn_wave_barrier();
-    __threadfence_block();
+    lds_order();
+    walk_products<G, false>(row, arp, acol, nullptr, brp, bcol, nullptr,
+                            [&](int c, double, double) { hash_insert(keys, T, c); });
+    __threadfence_block();  // the global-memory tables too
+    lds_order();
     int cnt = 0;
     for (int t0 = 0; t0 < T; t0 += G) {
         const int t = t0 + lane;
@@ -148,7 +221,7 @@ __global__ __launch_bounds__(kWave) void symbolic_global(int nrows, const int* _
 // ---------------------------------------------------------------------------
 // numeric
 // ---------------------------------------------------------------------------
-template <int G>
+template <int G, bool GLOBAL = false>
 __device__ void numeric_row(int row, int* keys, double* sums, int* lcol, double* lval, int T,
                             const int* __restrict__ arp, const int* __restrict__ acol, const double* __restrict__ aval,
                             const int* __restrict__ brp, const int* __restrict__ bcol, const double* __restrict__ bval,
@@ -160,18 +233,12 @@ __device__ void numeric_row(int row, int* keys, double* sums, int* lcol, double*
         keys[t] = -1;
         sums[t] = 0.0;
     }
-    __builtin_amdgcn_wave_barrier();
-    for (int j = arp[row]; j < arp[row + 1]; j++) {
-        const int c = acol[j];
-        const double a = aval[j];
-        for (int t = brp[c] + lane; t < brp[c + 1]; t += G) {
-            const int slot = hash_insert(keys, T, bcol[t]);
-            sums[slot] += a * bval[t];
-        }
-        // every lane's update for this a_ij lands before the next a_ij's
-        __builtin_amdgcn_wave_barrier();
-        __threadfence_block();
-    }
+    if (GLOBAL) __threadfence_block();
+    lds_order();
+    walk_products<G, true>(row, arp, acol, aval, brp, bcol, bval, [&](int c, double v, double a) {
+        sums[hash_insert(keys, T, c)] += a * v;
+        if (GLOBAL) __threadfence_block();
+    });
     // gather kept entries (|sum| > 1e-16) into a compact list
     int kept = 0;
     for (int t0 = 0; t0 < T; t0 += G) {
@@ -234,7 +301,7 @@ __global__ __launch_bounds__(kWave) void numeric_global(
     const int r = blockIdx.x;
     if (r >= nrows) return;
     const int64_t o = tab_off[r];
-    numeric_row<kWave>(rows[r], kpool + o, spool + o, lcpool + o, lvpool + o, tab_size[r], arp, acol, aval, brp, bcol, bval,
+    numeric_row<kWave, true>(rows[r], kpool + o, spool + o, lcpool + o, lvpool + o, tab_size[r], arp, acol, aval, brp, bcol, bval,
                 crp, ccol, cval, clen);
 }
 
@@ -394,7 +461,8 @@ static int next_pow2(int64_t v)
 // Runs symbolic+numeric for C = A B, returns a new handle.  Everything that
 // scales with the rows stays on the device: the host reads per-bin counts,
 // the rows of the global-hash bins with their sizes, and the totals.
-static ramd_csr_s* spgemm_impl(ramd_csr_s* A, ramd_csr_s* B)
+// temp: the product is only multiplied by other sparse matrices (see csr_wrap).
+static ramd_csr_s* spgemm_impl(ramd_csr_s* A, ramd_csr_s* B, bool temp = false)
 {
     ramd_ctx ctx = A->ctx;
     hipStream_t st = ctx->stream;
@@ -405,7 +473,7 @@ static ramd_csr_s* spgemm_impl(ramd_csr_s* A, ramd_csr_s* B)
     // --- product counts, and the rows binned by them
     int64_t* d_prod = tmp.get<int64_t>((size_t)m);
     if (m) {
-        hipLaunchKernelGGL(count_products, dim3((m + 255) / 256), dim3(256), 0, st, m, A->rowptr, A->col, B->rowptr,
+        hipLaunchKernelGGL(count_products, dim3((unsigned)(((int64_t)m * kCountGroup + 255) / 256)), dim3(256), 0, st, m, A->rowptr, A->col, B->rowptr,
                            d_prod);
         RAMD_HIP(hipGetLastError());
     }
@@ -565,7 +633,7 @@ static ramd_csr_s* spgemm_impl(ramd_csr_s* A, ramd_csr_s* B)
             d_val = v2;
         }
         RAMD_HIP(hipStreamSynchronize(st));
-        return csr_wrap(ctx, m, n, nnz, d_rp, d_col, d_val, nullptr);
+        return csr_wrap(ctx, m, n, nnz, d_rp, d_col, d_val, nullptr, temp);
     } catch (...) {
         dfree(d_col);
         dfree(d_val);
@@ -574,11 +642,11 @@ static ramd_csr_s* spgemm_impl(ramd_csr_s* A, ramd_csr_s* B)
     }
 }
 
-ramd_csr_s* spgemm(ramd_csr_s* A, ramd_csr_s* B) { return spgemm_impl(A, B); }
+ramd_csr_s* spgemm(ramd_csr_s* A, ramd_csr_s* B, bool temp) { return spgemm_impl(A, B, temp); }
 
 ramd_csr_s* galerkin(ramd_csr_s* A, ramd_csr_s* P)
 {
-    ramd_csr_s* AP = spgemm_impl(A, P);
+    ramd_csr_s* AP = spgemm_impl(A, P, true);
     ramd_csr_s* R = csr_transpose(P);
     ramd_csr_s* Ac = nullptr;
     try {
