@@ -406,12 +406,15 @@ void csr_autotune(ramd_csr_s* A, int prec);
 // operands in HBM, as inside a cycle after the other levels' kernels,
 // rather than left in the caches by its own previous launch; a larger one
 // cannot keep its operands cached and is timed back to back, without the
-// flush's write-backs in its time.  One that moves less than kFlushMin is bound
-// by latencies that rank the same either way, and the flush (67 us) would be
-// most of its timing: back to back too.  The autotuners rank kernel choices
-// by it.
+// flush's write-backs in its time.  One that moves less than kFlushSmall is
+// found in the infinity cache by most cycles: the pass before it writes
+// kFlushL2 only, which empties the L2s (14 us instead of 67; without any
+// flush the ranking of such launches follows their overlap with each other
+// and picked kernels that made a 7-point 29^3 solve 10% slower).  The
+// autotuners rank kernel choices by it.
 constexpr size_t kFlushBytes = (size_t)320 << 20;
-constexpr size_t kFlushMin = (size_t)4 << 20;
+constexpr size_t kFlushSmall = (size_t)4 << 20;
+constexpr size_t kFlushL2 = (size_t)64 << 20;
 float cold_median_ms(ramd_ctx ctx, const std::function<void()>& run, int reps, size_t op_bytes);
 // For a matrix with the stencil-diagonal form: times the gather kernel, the
 // LDS x-window kernel (when the window fits kDiaWin) and the plane-march

@@ -314,7 +314,7 @@ static void cycle32(ramd_hier_s* h, int l, float* x, const float* b, bool x_zero
 // Automatic mode: the first cycle in each precision times whole V-cycles
 // with the three largest tails, back to back and in turn (five rounds: the
 // coarse levels stay cached between cycles as they do in a solve), and keeps
-// the one with the smallest median (same bits for all).  No smaller tail and
+// the largest unless a smaller one's median is 1% below (same bits for all).  No smaller tail and
 // not the cycle without one: an operation inside the tail costs 0.7-2.5 us,
 // a launch of its own 3-5 us; only the largest levels' operations, bound by
 // what one compute unit reads, are in doubt (9-point anisotropic 100^2, FP64,
@@ -380,7 +380,9 @@ void cycle_prepare(ramd_hier_s* h, int prec)
         std::vector<float> t(kRounds);
         for (int r = 0; r < kRounds; r++) t[r] = ms[(size_t)r * nc + i];
         std::nth_element(t.begin(), t.begin() + kRounds / 2, t.end());
-        if (i == 0 || t[kRounds / 2] < best_ms) {
+        // a smaller tail's launches only pay when clearly faster: the timing
+        // queues cycles back to back, which hides the launches' host time
+        if (i == 0 || t[kRounds / 2] < 0.99f * best_ms) {
             best_ms = t[kRounds / 2];
             best = cand[i];
         }

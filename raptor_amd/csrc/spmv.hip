@@ -1476,7 +1476,8 @@ __global__ void flush_kernel(uint4* __restrict__ p, int64_t n)
 float cold_median_ms(ramd_ctx ctx, const std::function<void()>& run, int reps, size_t op_bytes)
 {
     hipStream_t s = ctx->stream;
-    const bool flush = op_bytes >= kFlushMin && op_bytes < kFlushBytes;
+    const bool flush = op_bytes < kFlushBytes;
+    const int64_t flush_units = (int64_t)((op_bytes < kFlushSmall ? kFlushL2 : kFlushBytes) / sizeof(uint4));
     if (flush && !ctx->flush_buf) ctx->flush_buf = dmalloc(kFlushBytes);
     std::vector<hipEvent_t> ev(2 * (size_t)reps, nullptr);
     std::vector<float> ms((size_t)reps, 0.f);
@@ -1486,7 +1487,7 @@ float cold_median_ms(ramd_ctx ctx, const std::function<void()>& run, int reps, s
         for (int r = 0; r < reps; r++) {
             if (flush) {
                 hipLaunchKernelGGL(flush_kernel, dim3(4096), dim3(256), 0, s, (uint4*)ctx->flush_buf,
-                                   (int64_t)(kFlushBytes / sizeof(uint4)));
+                                   flush_units);
                 RAMD_HIP(hipGetLastError());
             }
             RAMD_HIP(hipEventRecord(ev[2 * r], s));
