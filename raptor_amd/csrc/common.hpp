@@ -46,6 +46,8 @@ constexpr double kLaneRowsMaxLen = 8.0;
 // this many entries per row
 constexpr double kWaveRowsMinLen = 24.0;
 constexpr int kStreamCap = 4096;     // products staged in LDS per workgroup
+// entry bytes up to which an untuned matrix is read through the caches
+constexpr double kKeepBytes = 96e6;
 constexpr int kMaxRowsPerBlock = 256;
 
 // Row blocks for the LDS-staged kernels: consecutive rows whose nonzeros fit
@@ -211,6 +213,7 @@ constexpr int kBoxMaxPlanes = 256;
 struct DiaBox {
     int L = 0, P = 0;  // 0: the offsets have no box decomposition
     int tx = 64;       // tile width (TY = kBlockThreads / tx)
+    int utx = 32;      // ... of the kernels of uniform operators
     BoxArgs args{};
     int zc[3] = {kBoxPlanes, kBoxPlanes, kBoxPlanes};  // planes per workgroup, per precision pair
 };
@@ -312,6 +315,7 @@ struct ramd_csr_s {
         int n = 0;
         int* d = nullptr;  // == blocks for the default cap
     } rb[2];
+    bool tuned = false;  // csr_autotune chose among the CSR kernels
     // lazily built transpose (gather form of A^T x), same drop-free pattern
     ramd_csr_s* trans = nullptr;
     // FP32 copy of the values (mixed-precision cycle)

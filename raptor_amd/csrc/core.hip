@@ -273,10 +273,20 @@ __global__ __launch_bounds__(kBlockThreads) void dia_check_kernel(int n, int nd,
                                                                   int* __restrict__ flags)
 {
     __shared__ unsigned long long r[kDiaMax];
-    if (threadIdx.x < kDiaMax) r[threadIdx.x] = kNoRef;
+    // the workgroup's first row gives the values to compare with; slots it
+    // does not store take their first one below
+    const int i0 = blockIdx.x * kBlockThreads;
+    if ((int)threadIdx.x < kDiaMax) {
+        const int t = threadIdx.x;
+        unsigned long long v = kNoRef;
+        if (i0 < n && t < nd && ((mask[i0] >> a.ord[t]) & 1u))
+            v = (unsigned long long)__double_as_longlong(v64[dia_index<double>(t, i0, n)]);
+        r[t] = v;
+    }
     __syncthreads();
     int f = 0;
-    for (int i = blockIdx.x * kBlockThreads + threadIdx.x; i < n; i += gridDim.x * kBlockThreads) {
+    for (int i = i0 + threadIdx.x; i < n; i += gridDim.x * kBlockThreads) {
+        if ((f | __atomic_load_n(flags, __ATOMIC_RELAXED)) == 24) break;  // both known
         const unsigned m = mask[i];
         for (int t = 0; t < nd; t++) {
             if (!((m >> a.ord[t]) & 1u)) continue;
@@ -289,11 +299,11 @@ __global__ __launch_bounds__(kBlockThreads) void dia_check_kernel(int n, int nd,
         }
     }
     __syncthreads();
-    if ((int)threadIdx.x < nd && r[threadIdx.x] != kNoRef) {
+    if ((int)threadIdx.x < nd && r[threadIdx.x] != kNoRef && !(f & 16)) {
         const unsigned long long o = atomicCAS(&ref[threadIdx.x], kNoRef, r[threadIdx.x]);
         if (o != kNoRef && o != r[threadIdx.x]) f |= 16;
     }
-    if (f) atomicOr(flags, f);
+    if (f & ~__atomic_load_n(flags, __ATOMIC_RELAXED)) atomicOr(flags, f);
 }
 
 __global__ void dia_check_init_kernel(unsigned long long* __restrict__ ref, int* __restrict__ flags)
@@ -377,6 +387,24 @@ void dia_box_detect(const long long* offs, int nd, int n, DiaBox& b)
     if (!b.L) return;
     // tile width: the widest of 64, 32, 16 that divides the line, else 64
     b.tx = b.L % 64 == 0 ? 64 : b.L % 32 == 0 ? 32 : b.L % 16 == 0 ? 16 : 64;
+    // uniform operators: x and its halo are most of what a workgroup reads, so
+    // the squarer tiles of 32 or 16 (256^3 product 125 us with 64, 114 with 32,
+    // 112 with 16; 101^3, whose lines none divides, 14.5, 14.4 and 13.6): the
+    // one with the fewest positions past the grid, 32 where they are equal.
+    // Planes per workgroup before any timing: eight where that leaves eight
+    // workgroups per compute unit (192^3 50.5 -> 46.3 us), else four (101^3
+    // 14.5 us, with eight 19.2).
+    long long best = 0;
+    for (const int t : {32, 16, 64}) {
+        const long long ty = kBlockThreads / t, ny = b.P / b.L;
+        const long long area = (b.L + t - 1) / t * t * ((ny + ty - 1) / ty * ty);
+        if (!best || area < best) {
+            best = area;
+            b.utx = t;
+        }
+    }
+    const long long wgs8 = best / kBlockThreads * ((n / b.P + 7) / 8);
+    for (int& zc : b.zc) zc = wgs8 >= 2048 ? 2 * kBoxPlanes : kBoxPlanes;
     for (int k = 0; k < kDiaMax; k++) {
         int dz = 0, dy = 0, dx = 0;
         if (k < nd) split(offs[k], b.L, b.P, dz, dy, dx);
