@@ -467,12 +467,17 @@ void launch_stream_op_c(const ramd_csr_s* A, int op, const double* x, const doub
                         double omega, hipStream_t s);
 
 // y = A x (FP64 vectors) with x.y summed per workgroup in the same pass and
-// reduced into *out_d (fixed order: deterministic).  values_fp32 selects the
-// lossless FP32-value form of launch_stream_op_c.
+// reduced into *out_d (fixed order: deterministic; null: left as partial
+// sums).  values_fp32 selects the lossless FP32-value form of
+// launch_stream_op_c.
 void launch_spmv_dot(const ramd_csr_s* A, bool values_fp32, const double* x, double* y, double* out_d,
                      hipStream_t s, double* partials = nullptr);
-// per-workgroup partials launch_spmv_dot writes for A
+// per-workgroup partials launch_spmv_dot writes for A: at most, over every
+// kernel choice, and with the present one
 int spmv_dot_partials(const ramd_csr_s* A);
+int spmv_dot_launch_partials(const ramd_csr_s* A, bool values_fp32);
+// partial sums that one workgroup adds in one stage
+constexpr int kFinalMax = 4096;
 
 // Deterministic device reductions; result left in *out_d (device scalar).
 void launch_dot(ramd_ctx ctx, int64_t n, const double* x, const double* y, double* out_d);

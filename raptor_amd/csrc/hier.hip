@@ -1132,19 +1132,37 @@ void vcycle_from_zero(ramd_hier_s* h, double* x, const double* b) { cycle64(h, 0
 // r -= alpha Ap; r32 = (float) r when given; partial sums of r^2.  alpha =
 // rz / pAp is formed from the device scalars (every thread computes the
 // same value; workgroup 0 stores it for the direction update, which also
-// takes the step x += alpha p).  With z32 given, also the FP32 cycle's first
-// Jacobi sweep from zero on r32 (jacobi_from_zero's operations, diagonal
-// d32, weight w), so the cycle starts from it.
+// takes the step x += alpha p).  With np > 0, p.Ap is not a scalar yet: every
+// workgroup adds its np (<= kFinalMax) partial sums itself, in
+// reduce_final's order, and workgroup 0 stores it -- a launch fewer.  With z
+// given, also the cycle's first Jacobi sweep from zero on r (on r32 in the
+// FP32 form; jacobi_from_zero's operations, diagonal d, weight w), so the
+// cycle starts from it.
+template <typename X>
 __global__ __launch_bounds__(kBlockThreads) void fpcg_update_norm(int n, const double* __restrict__ sc_rz,
-                                                                  const double* __restrict__ sc_pap,
+                                                                  double* __restrict__ sc_pap,
                                                                   double* __restrict__ sc_alpha,
                                                                   const double* __restrict__ Ap,
-                                                                  double* __restrict__ r, float* __restrict__ r32,
+                                                                  double* __restrict__ r, X* __restrict__ r32,
                                                                   double* __restrict__ partials,
-                                                                  const float* __restrict__ d32,
-                                                                  float* __restrict__ z32, float w)
+                                                                  const double* __restrict__ pap_part, int np,
+                                                                  const X* __restrict__ d, X* __restrict__ z, X w)
 {
-    const double alpha = *sc_rz / *sc_pap;
+    double pap;
+    if (np > 0) {
+        __shared__ double sum;
+        double t = strided_sum(pap_part, 0, np);
+        t = block_sum(t);
+        if (threadIdx.x == 0) {
+            sum = t;
+            if (blockIdx.x == 0) *sc_pap = t;
+        }
+        __syncthreads();
+        pap = sum;
+    } else {
+        pap = *sc_pap;
+    }
+    const double alpha = *sc_rz / pap;
     if (blockIdx.x == 0 && threadIdx.x == 0) *sc_alpha = alpha;
     double s = 0;
     const int stride = gridDim.x * kBlockThreads;
@@ -1153,14 +1171,14 @@ __global__ __launch_bounds__(kBlockThreads) void fpcg_update_norm(int n, const d
     constexpr int U = 4;
     for (int i0 = blockIdx.x * kBlockThreads + threadIdx.x; i0 < n; i0 += U * stride) {
         double rv[U], av[U];
-        float dv[U];
+        X dv[U];
 #pragma unroll
         for (int u = 0; u < U; u++) {
             const int i = i0 + u * stride;
             if (i < n) {
                 rv[u] = r[i];
                 av[u] = Ap[i];
-                if (z32) dv[u] = d32[i];
+                if (z) dv[u] = d[i];
             }
         }
 #pragma unroll
@@ -1169,17 +1187,8 @@ __global__ __launch_bounds__(kBlockThreads) void fpcg_update_norm(int n, const d
             if (i >= n) break;
             const double ri = rv[u] - alpha * av[u];
             r[i] = ri;
-            if (r32) {
-                const float rf = (float)ri;
-                r32[i] = rf;
-                if (z32) {
-                    const float di = dv[u];
-                    const float zero = 0.0f;
-                    float v = zero;
-                    if (fabs(di) > float(1e-16)) v = ((1.0f - w) * zero) + (w * ((rf - zero) / di));
-                    z32[i] = v;
-                }
-            }
+            if (sizeof(X) == 4) r32[i] = (X)ri;
+            if (z) z[i] = jacobi_zero_row((X)ri, dv[u], w);
             s += ri * ri;
         }
     }
@@ -1226,7 +1235,7 @@ __global__ __launch_bounds__(kBlockThreads) void fpcg_dots(int n, const double* 
 
 // x += alpha p (when x is given: the step of this iteration, taken here so
 // that p is read once), then p = z + beta p with the flexible
-// (Polak-Ribiere) beta = -alpha (z.Ap) / rz_old from the device scalars
+// (Polak-Ribiere) beta = -alpha (z.Ap) / rz_old from the device scalars.
 template <typename Z>
 __global__ void fpcg_dir(int n, const double* __restrict__ sc_alpha, const double* __restrict__ sc_zap,
                          const double* __restrict__ sc_rz_old, const Z* __restrict__ z, double* __restrict__ p,
@@ -1398,35 +1407,47 @@ static int fpcg_run(ramd_hier_s* h, ramd_csr_s* A, double* x_d, const double* b_
     float *r32 = h->pr32, *z32 = h->pz32;
     const int g = fixed_blocks(n);
     const dim3 gv = grid1(n), bv(256);
-    const size_t npart = (size_t)std::max(spmv_dot_partials(A), 2 * g);
+    const size_t npart = (size_t)std::max(spmv_dot_partials(A), 2 * g + kFinalMax);
     if (noalloc)
         RAMD_CHECK(npart <= (size_t)kNoallocPartials, RAMD_E_ARG,
                    "ramd_fpcg_noalloc: the operator needs %zu partial sums, the scratch holds %d (about %d rows)",
                    npart, kNoallocPartials, kNoallocPartials * kBlockThreads);
     double* part = noalloc ? noalloc_scratch(ctx->device) : fpcg_partials(h, npart);
-    // FP32 form: the update pass also forms the cycle's first Jacobi sweep
-    // from zero on the fine level (Jacobi smoothing, more than one level)
-    const bool fuse_first = f32 && !multicolour(h) && h->opts.num_smooth_sweeps >= 1 && h->levels.size() > 1;
+    // the update pass also forms the cycle's first Jacobi sweep from zero on
+    // the fine level (Jacobi smoothing, more than one level)
+    const bool fuse_first = !multicolour(h) && h->opts.num_smooth_sweeps >= 1 && h->levels.size() > 1;
+    // p.Ap's partial sums, in their own part of the buffer when the update
+    // pass adds them up: few enough that every workgroup can (3456 sums at
+    // 96^3: 27 KB from the L2), else one kernel does
+    const int np_dot = spmv_dot_launch_partials(A, true);
+    const bool pap_here = np_dot <= kFinalMax;
+    double* dot_part = pap_here ? part + 2 * g : part;
     // device scalars: [0] p.Ap, [1] r.r, [2]/[5] r.z (current / next), [3] z.Ap, [4] alpha
     double* sc = ctx->red_result;
     int cur = 2, nxt = 5;
     // operator step: Ap = A p and p.Ap in one pass over A; then r -= alpha Ap,
-    // ||r||^2 (and r32, and in the FP32 form the first sweep z32) in one pass;
+    // ||r||^2 (and r32, and the cycle's first sweep) in one pass;
     // p.Ap and r.r are also written to host memory, read after step_ev
     auto stepA = [&](int c) {
-        launch_spmv_dot(A, true, p, Ap, sc, s, part);
-        hipLaunchKernelGGL(fpcg_update_norm, dim3(g), dim3(kBlockThreads), 0, s, n, sc + c, sc, sc + 4, Ap, r,
-                           f32 ? r32 : nullptr, part, fuse_first ? h->levels[0].diag32 : nullptr,
-                           fuse_first ? z32 : nullptr, (float)h->opts.relax_weight);
+        launch_spmv_dot(A, true, p, Ap, pap_here ? nullptr : sc, s, dot_part);
+        const int np = pap_here ? np_dot : 0;
+        if (f32)
+            hipLaunchKernelGGL((fpcg_update_norm<float>), dim3(g), dim3(kBlockThreads), 0, s, n, sc + c, sc, sc + 4,
+                               Ap, r, r32, part, dot_part, np, h->levels[0].diag32, fuse_first ? z32 : nullptr,
+                               (float)h->opts.relax_weight);
+        else
+            hipLaunchKernelGGL((fpcg_update_norm<double>), dim3(g), dim3(kBlockThreads), 0, s, n, sc + c, sc, sc + 4,
+                               Ap, r, (double*)nullptr, part, dot_part, np, h->levels[0].diag,
+                               fuse_first ? z : nullptr, h->opts.relax_weight);
         RAMD_HIP(hipGetLastError());
         launch_reduce_final_pub(ctx, part, g, sc + 1, sc, ctx->step_pin_d);
     };
-    // preconditioner application: z = M^-1 r (first_done: z32 holds the
+    // preconditioner application: z = M^-1 r (first_done: z holds the
     // fused first sweep), r.z into slot nx and z.Ap.  It writes only z, the
     // cycle's level vectors, the partial sums and scalar slots nx and 3.
     auto stepB = [&](int nx, bool first_done) {
         if (f32) cycle32(h, 0, z32, r32, true, first_done);
-        else cycle64(h, 0, z, r, true);
+        else cycle64(h, 0, z, r, true, first_done);
         if (f32) fpcg_rz_zap(ctx, n, r, (const float*)z32, Ap, sc + nx, sc + 3, part);
         else fpcg_rz_zap(ctx, n, r, (const double*)z, Ap, sc + nx, sc + 3, part);
     };
@@ -1516,7 +1537,7 @@ static int fpcg_run(ramd_hier_s* h, ramd_csr_s* A, double* x_d, const double* b_
                 }
             };
             if (ahead) run_b(plain_b);
-            bool z_first = fuse_first;  // z32 holds the fused first sweep of the current r32
+            bool z_first = fuse_first;  // z holds the fused first sweep of the current r
             RAMD_HIP(hipEventSynchronize(ctx->step_ev));
             const volatile double* pin = ctx->step_pin;
             const double pr[2] = {pin[0], pin[1]};
@@ -1544,7 +1565,7 @@ static int fpcg_run(ramd_hier_s* h, ramd_csr_s* A, double* x_d, const double* b_
                     hipLaunchKernelGGL(to_f32, gv, bv, 0, s, (int64_t)n, r, r32);
                     RAMD_HIP(hipGetLastError());
                 }
-                z_first = false;  // r32 was replaced
+                z_first = false;  // r was replaced
                 r_new = true;
             } else if (relres_hist) {
                 relres_hist[it] = relres;

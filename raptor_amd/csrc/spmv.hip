@@ -1787,19 +1787,25 @@ int spmv_dot_partials(const ramd_csr_s* A)
     return std::max(np, 1);
 }
 
+int spmv_dot_launch_partials(const ramd_csr_s* A, bool values_fp32)
+{
+    const bool dia32 = values_fp32 && A->dia && A->dia->v32 && A->dia->v32_exact && A->v32_outer;
+    return A->dia ? dia_grid(A, dia32 ? 2 : 0) : spmv_dot_partials(A);
+}
+
 void launch_spmv_dot(const ramd_csr_s* A, bool values_fp32, const double* x, double* y, double* out_d,
                      hipStream_t s, double* partials)
 {
     ramd_ctx ctx = A->ctx;
     const bool dia32 = values_fp32 && A->dia && A->dia->v32 && A->dia->v32_exact && A->v32_outer;
-    const int np = A->dia ? dia_grid(A, dia32 ? 2 : 0) : spmv_dot_partials(A);
+    const int np = spmv_dot_launch_partials(A, values_fp32);
     double* part = partials ? partials : ctx_partials(ctx, (size_t)np);
     if (dia32)
         launch_stream<float, double>(A, nullptr, A->dia->v32, OP_SPMV, x, nullptr, y, 0.0, s, part);
     else
         launch_stream<double, double>(A, A->val, A->dia ? A->dia->v64 : nullptr, OP_SPMV, x, nullptr, y, 0.0, s,
                                       part);
-    launch_reduce_final(ctx, part, np, out_d);
+    if (out_d) launch_reduce_final(ctx, part, np, out_d);
 }
 
 // ---------------------------------------------------------------------------
@@ -1940,7 +1946,7 @@ __global__ __launch_bounds__(kBlockThreads) void reduce_chunks(const double* __r
 void launch_reduce_final(ramd_ctx ctx, const double* partials, int np, double* out_d)
 {
     constexpr int kChunks = 256;
-    if (np > 4096) {
+    if (np > kFinalMax) {
         // one workgroup would read every partial serially: split in two stages
         const int chunk = (np + kChunks - 1) / kChunks;
         double* mid = ctx->red_partials + 3072;  // 256 doubles past the grid-stride partials
