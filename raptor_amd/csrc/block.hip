@@ -33,7 +33,7 @@ template <int OP, typename V, typename X, int LPR>
 __global__ __launch_bounds__(256) void bcsr_kernel(int n, int k, const int* __restrict__ rp,
                                                    const int* __restrict__ col, const V* __restrict__ val,
                                                    const X* __restrict__ x, const X* __restrict__ b,
-                                                   X* __restrict__ y, X omega)
+                                                   X* __restrict__ y, X omega, X* __restrict__ y2)
 {
     constexpr int RPW = 256 / LPR;
     constexpr int CPL = kMaxRhs / LPR;  // columns per lane (upper bound)
@@ -71,7 +71,10 @@ __global__ __launch_bounds__(256) void bcsr_kernel(int n, int k, const int* __re
         const int c = g + q * LPR;
         if (c >= k) continue;
         if (OP == OP_SPMV || OP == OP_RESIDUAL) y[o + c] = acc[q];
-        else if (OP == OP_APPEND) y[o + c] += acc[q];
+        else if (OP == OP_SPMV_JFZ) {
+            y[o + c] = acc[q];
+            y2[o + c] = jacobi_zero_row(acc[q], b[row], omega);
+        } else if (OP == OP_APPEND) y[o + c] += acc[q];
         else if (OP == OP_ADD_INTO) y[o + c] = b[o + c] + acc[q];
         else {
             const X xo = x[o + c];
@@ -253,7 +256,7 @@ template <int OP, typename V, typename X, int LPR, int UPL>
 __global__ __launch_bounds__(256) void bcsr_vec_kernel(int n, int k, const int* __restrict__ rp,
                                                        const int* __restrict__ col, const V* __restrict__ val,
                                                        const X* __restrict__ x, const X* __restrict__ b,
-                                                       X* __restrict__ y, X omega)
+                                                       X* __restrict__ y, X omega, X* __restrict__ y2)
 {
     constexpr int VW = 16 / sizeof(X);
     constexpr int RPW = 256 / LPR;
@@ -313,6 +316,19 @@ __global__ __launch_bounds__(256) void bcsr_vec_kernel(int n, int k, const int* 
             cj[t] = cn[t];
             a[t] = an[t];
         }
+    }
+    if (OP == OP_SPMV_JFZ) {
+        const X d = b[row];
+#pragma unroll
+        for (int u = 0; u < UPL; u++) {
+            if (!U.on[u]) continue;
+            X out[VW];
+#pragma unroll
+            for (int t = 0; t < VW; t++) out[t] = jacobi_zero_row(acc[u][t], d, omega);
+            unit_store<X>(y + o + U.off[u], acc[u]);
+            unit_store<X>(y2 + o + U.off[u], out);
+        }
+        return;
     }
     bvec_finish<OP, X, LPR, UPL>(acc, U, x + o, b + o, y + o, diag, s != e && fabs(diag) > X(1e-16), omega);
 }
@@ -376,12 +392,12 @@ __global__ __launch_bounds__(256) void bdia_vec_kernel(int n, int k, DiaArgs a, 
 
 template <int OP, typename V, typename X, int LPR, int UPL>
 static void blaunch_vec_op(const ramd_csr_s* A, const V* val, const V* dval, int k, const X* x, const X* b, X* y,
-                           X omega, hipStream_t s)
+                           X omega, hipStream_t s, X* y2)
 {
     const int n = A->n_rows;
     if (n == 0) return;
     const dim3 grid((unsigned)((n + 256 / LPR - 1) / (256 / LPR))), block(256);
-    if (dval) {
+    if constexpr (OP != OP_SPMV_JFZ) if (dval) {
         const Dia* d = A->dia;
 #define BDIAV(NDV)                                                                                            \
     hipLaunchKernelGGL((bdia_vec_kernel<OP, V, X, LPR, UPL, NDV>), grid, block, 0, s, n, k, d->args, d->nd, \
@@ -391,25 +407,27 @@ static void blaunch_vec_op(const ramd_csr_s* A, const V* val, const V* dval, int
         else if (d->nd == 7) BDIAV(7);
         else BDIAV(kDiaMax);
 #undef BDIAV
-    } else {
-        hipLaunchKernelGGL((bcsr_vec_kernel<OP, V, X, LPR, UPL>), grid, block, 0, s, n, k, A->rowptr, A->col, val,
-                           x, b, y, omega);
+        RAMD_HIP(hipGetLastError());
+        return;
     }
+    hipLaunchKernelGGL((bcsr_vec_kernel<OP, V, X, LPR, UPL>), grid, block, 0, s, n, k, A->rowptr, A->col, val, x, b,
+                       y, omega, y2);
     RAMD_HIP(hipGetLastError());
 }
 
 template <typename V, typename X, int LPR>
 static void blaunch_vec_lpr(const ramd_csr_s* A, const V* val, const V* dval, int op, int k, const X* x,
-                            const X* b, X* y, X omega, hipStream_t s)
+                            const X* b, X* y, X omega, hipStream_t s, X* y2)
 {
     constexpr int VW = 16 / sizeof(X);
     const int upl = (k / VW + LPR - 1) / LPR;
 #define BVEC(UPLV)                                                                                            \
     switch (op) {                                                                                            \
-    case OP_SPMV: blaunch_vec_op<OP_SPMV, V, X, LPR, UPLV>(A, val, dval, k, x, b, y, omega, s); break;       \
-    case OP_RESIDUAL: blaunch_vec_op<OP_RESIDUAL, V, X, LPR, UPLV>(A, val, dval, k, x, b, y, omega, s); break; \
-    case OP_JACOBI: blaunch_vec_op<OP_JACOBI, V, X, LPR, UPLV>(A, val, dval, k, x, b, y, omega, s); break;   \
-    case OP_ADD_INTO: blaunch_vec_op<OP_ADD_INTO, V, X, LPR, UPLV>(A, val, dval, k, x, b, y, omega, s); break; \
+    case OP_SPMV: blaunch_vec_op<OP_SPMV, V, X, LPR, UPLV>(A, val, dval, k, x, b, y, omega, s, y2); break;       \
+    case OP_SPMV_JFZ: blaunch_vec_op<OP_SPMV_JFZ, V, X, LPR, UPLV>(A, val, dval, k, x, b, y, omega, s, y2); break; \
+    case OP_RESIDUAL: blaunch_vec_op<OP_RESIDUAL, V, X, LPR, UPLV>(A, val, dval, k, x, b, y, omega, s, y2); break; \
+    case OP_JACOBI: blaunch_vec_op<OP_JACOBI, V, X, LPR, UPLV>(A, val, dval, k, x, b, y, omega, s, y2); break;   \
+    case OP_ADD_INTO: blaunch_vec_op<OP_ADD_INTO, V, X, LPR, UPLV>(A, val, dval, k, x, b, y, omega, s, y2); break; \
     default: fail(RAMD_E_ARG, "block op %d not supported", op);                                              \
     }
     if (upl == 1) {
@@ -424,12 +442,12 @@ static void blaunch_vec_lpr(const ramd_csr_s* A, const V* val, const V* dval, in
 
 template <int OP, typename V, typename X, int LPR>
 static void blaunch_op(const ramd_csr_s* A, const V* val, const V* dval, int k, const X* x, const X* b, X* y,
-                       X omega, hipStream_t s)
+                       X omega, hipStream_t s, X* y2)
 {
     const int n = A->n_rows;
     if (n == 0) return;
     const dim3 grid((unsigned)((n + 256 / LPR - 1) / (256 / LPR))), block(256);
-    if (dval) {
+    if constexpr (OP != OP_SPMV_JFZ) if (dval) {
         const Dia* d = A->dia;
 #define BDIA(NDV)                                                                                                  \
     hipLaunchKernelGGL((bdia_kernel<OP, V, X, LPR, NDV>), grid, block, 0, s, n, k, d->args, d->nd, d->center, \
@@ -439,22 +457,24 @@ static void blaunch_op(const ramd_csr_s* A, const V* val, const V* dval, int k, 
         else if (d->nd == 7) BDIA(7);
         else BDIA(kDiaMax);
 #undef BDIA
-    } else {
-        hipLaunchKernelGGL((bcsr_kernel<OP, V, X, LPR>), grid, block, 0, s, n, k, A->rowptr, A->col, val, x, b, y,
-                           omega);
+        RAMD_HIP(hipGetLastError());
+        return;
     }
+    hipLaunchKernelGGL((bcsr_kernel<OP, V, X, LPR>), grid, block, 0, s, n, k, A->rowptr, A->col, val, x, b, y, omega,
+                       y2);
     RAMD_HIP(hipGetLastError());
 }
 
 template <typename V, typename X, int LPR>
 static void blaunch_lpr(const ramd_csr_s* A, const V* val, const V* dval, int op, int k, const X* x, const X* b,
-                        X* y, X omega, hipStream_t s)
+                        X* y, X omega, hipStream_t s, X* y2)
 {
     switch (op) {
-    case OP_SPMV: blaunch_op<OP_SPMV, V, X, LPR>(A, val, dval, k, x, b, y, omega, s); break;
-    case OP_RESIDUAL: blaunch_op<OP_RESIDUAL, V, X, LPR>(A, val, dval, k, x, b, y, omega, s); break;
-    case OP_JACOBI: blaunch_op<OP_JACOBI, V, X, LPR>(A, val, dval, k, x, b, y, omega, s); break;
-    case OP_ADD_INTO: blaunch_op<OP_ADD_INTO, V, X, LPR>(A, val, dval, k, x, b, y, omega, s); break;
+    case OP_SPMV: blaunch_op<OP_SPMV, V, X, LPR>(A, val, dval, k, x, b, y, omega, s, y2); break;
+    case OP_SPMV_JFZ: blaunch_op<OP_SPMV_JFZ, V, X, LPR>(A, val, dval, k, x, b, y, omega, s, y2); break;
+    case OP_RESIDUAL: blaunch_op<OP_RESIDUAL, V, X, LPR>(A, val, dval, k, x, b, y, omega, s, y2); break;
+    case OP_JACOBI: blaunch_op<OP_JACOBI, V, X, LPR>(A, val, dval, k, x, b, y, omega, s, y2); break;
+    case OP_ADD_INTO: blaunch_op<OP_ADD_INTO, V, X, LPR>(A, val, dval, k, x, b, y, omega, s, y2); break;
     default: fail(RAMD_E_ARG, "block op %d not supported", op);
     }
 }
@@ -480,8 +500,11 @@ static bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 // vectors are not 16-byte aligned)
 template <typename X>
 static void blaunch(const ramd_csr_s* A, int code, int op, int k, const X* x, const X* b, X* y, X omega,
-                    hipStream_t s)
+                    hipStream_t s, X* y2 = nullptr)
 {
+    RAMD_CHECK(op != OP_SPMV_JFZ || (!A->dia && b && y2), RAMD_E_STATE,
+               "block restriction with the first sweep needs a CSR operator, a diagonal and a second output");
+    if (op == OP_SPMV_JFZ && !aligned16(y2) && code < 0) code = lpr_ok(32, k) ? 32 : 64;
     if (code < 0 && !(aligned16(x) && aligned16(y) && (!b || aligned16(b)))) code = lpr_ok(32, k) ? 32 : 64;
     // FP64 vectors read FP64 values; FP32 vectors read the FP32 copies
     using V = X;
@@ -496,13 +519,13 @@ static void blaunch(const ramd_csr_s* A, int code, int op, int k, const X* x, co
         dval = A->dia ? (const V*)A->dia->v32 : nullptr;
     }
     switch (code) {
-    case 8: blaunch_lpr<V, X, 8>(A, val, dval, op, k, x, b, y, omega, s); break;
-    case 16: blaunch_lpr<V, X, 16>(A, val, dval, op, k, x, b, y, omega, s); break;
-    case 32: blaunch_lpr<V, X, 32>(A, val, dval, op, k, x, b, y, omega, s); break;
-    case 64: blaunch_lpr<V, X, 64>(A, val, dval, op, k, x, b, y, omega, s); break;
-    case -4: blaunch_vec_lpr<V, X, 4>(A, val, dval, op, k, x, b, y, omega, s); break;
-    case -8: blaunch_vec_lpr<V, X, 8>(A, val, dval, op, k, x, b, y, omega, s); break;
-    case -16: blaunch_vec_lpr<V, X, 16>(A, val, dval, op, k, x, b, y, omega, s); break;
+    case 8: blaunch_lpr<V, X, 8>(A, val, dval, op, k, x, b, y, omega, s, y2); break;
+    case 16: blaunch_lpr<V, X, 16>(A, val, dval, op, k, x, b, y, omega, s, y2); break;
+    case 32: blaunch_lpr<V, X, 32>(A, val, dval, op, k, x, b, y, omega, s, y2); break;
+    case 64: blaunch_lpr<V, X, 64>(A, val, dval, op, k, x, b, y, omega, s, y2); break;
+    case -4: blaunch_vec_lpr<V, X, 4>(A, val, dval, op, k, x, b, y, omega, s, y2); break;
+    case -8: blaunch_vec_lpr<V, X, 8>(A, val, dval, op, k, x, b, y, omega, s, y2); break;
+    case -16: blaunch_vec_lpr<V, X, 16>(A, val, dval, op, k, x, b, y, omega, s, y2); break;
     default: fail(RAMD_E_ARG, "block kernel code %d", code);
     }
 }
@@ -1062,7 +1085,7 @@ static void bvec(BlockLevel& L, X*& x, X*& b, X*& t, X*& r)
 }
 
 template <typename X>
-static void bcycle(ramd_hier_s* h, BlockState* bs, int l, X* x, const X* b)
+static void bcycle(ramd_hier_s* h, BlockState* bs, int l, X* x, const X* b, bool first_done = false)
 {
     Level& L = h->levels[l];
     BlockLevel& BL = bs->lv[l];
@@ -1097,7 +1120,8 @@ static void bcycle(ramd_hier_s* h, BlockState* bs, int l, X* x, const X* b)
         RAMD_HIP(hipGetLastError());
     }
     for (int it = 0; it < sweeps; it++) {
-        if (it == 0) {
+        if (it == 0 && first_done) {  // x holds it: written by the restriction that formed b
+        } else if (it == 0) {
             const int kp = pow2_at_least(k);
             hipLaunchKernelGGL((bjacobi_from_zero<X>), dim3(col_blocks(L.n, kp)), dim3(256), 0, s, L.n, k, kp, diag,
                                b, cur, w);
@@ -1113,8 +1137,15 @@ static void bcycle(ramd_hier_s* h, BlockState* bs, int l, X* x, const X* b)
     bvec<X>(BC, cx, cb, ct, cr);
     (void)ct;
     (void)cr;
-    blaunch<X>(L.R, BL.code_R[(sizeof(X) == 4 ? 1 : 0)], OP_SPMV, k, lr, (const X*)nullptr, cb, X(0), s);
-    bcycle<X>(h, bs, l + 1, cx, cb);
+    // a smoothed coarse level's first Jacobi sweep from zero comes with its
+    // right-hand sides
+    const bool cj = sweeps >= 1 && l + 2 < (int)h->levels.size() && !L.R->dia;
+    const X* cdiag;
+    if constexpr (sizeof(X) == 8) cdiag = h->levels[l + 1].diag;
+    else cdiag = h->levels[l + 1].diag32;
+    if (cj) blaunch<X>(L.R, BL.code_R[(sizeof(X) == 4 ? 1 : 0)], OP_SPMV_JFZ, k, lr, cdiag, cb, w, s, cx);
+    else blaunch<X>(L.R, BL.code_R[(sizeof(X) == 4 ? 1 : 0)], OP_SPMV, k, lr, (const X*)nullptr, cb, X(0), s);
+    bcycle<X>(h, bs, l + 1, cx, cb, cj);
     blaunch<X>(L.P, BL.code_P[(sizeof(X) == 4 ? 1 : 0)], OP_ADD_INTO, k, cx, cur, other, X(0), s);
     std::swap(cur, other);
     for (int it = 0; it < sweeps; it++) {

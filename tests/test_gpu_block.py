@@ -207,3 +207,37 @@ def test_block_fpcg_graph_equals_eager(problem, ctx):
         out.append((X.numpy(), its, rel))
     for X, its, rel in out[1:]:
         assert np.array_equal(X, out[0][0]) and np.array_equal(its, out[0][1]) and np.array_equal(rel, out[0][2])
+
+
+@pytest.mark.parametrize("k,codes64,codes32", [(1, (8,), (8,)), (5, (8,), (8,)), (8, (8, -4), (8,)),
+                                               (32, (16, 32, -8, -16), (8, 32, -4, -8)),
+                                               (64, (8, 64, -16), (16, 64, -8, -16))])
+def test_block_restriction_with_first_sweep(ctx, k, codes64, codes32):
+    """Every kernel the block restriction can run on (one column per lane step
+    or 16-byte units, few and many lanes per row, k at the edges of both)
+    writes the coarse right-hand sides and the coarse level's first Jacobi
+    sweep from zero: each column equals the oracle's cycle, FP64 and FP32, bit
+    for bit, over two smoothed coarse levels."""
+    rp, col, val = ra.gallery_laplace27(16)
+    ml = ra.ParRugeStubenSolver(ctx, 0.25, ra.PMIS, ra.Extended, ra.Classical, ra.Jacobi)
+    ml.relax_weight = OMEGA
+    ml.setup(rp, col, val)
+    ml.enable_fp32()
+    assert ml.num_levels >= 3
+    H = oracle_hier(ml)
+    n = rp.size - 1
+    B = np.random.default_rng(60 + k).standard_normal((n, k))
+    B32 = B.astype(np.float32)
+    cols = sorted({0, k // 2, k - 1})
+    want = {c: (H.cycle(np.zeros(n), B[:, c]), H.cycle_fp32(np.zeros(n, np.float32), B32[:, c])) for c in cols}
+    for i, (prec, dt, rhs, codes) in enumerate(((ra.PREC_FP64, np.float64, B, codes64),
+                                                (ra.PREC_FP32, np.float32, B32, codes32))):
+        for code in codes:
+            t = ra.block_tuning(ml, k, prec)
+            t[:-1] = code
+            ra.block_set_tuning(ml, k, t, prec)
+            X = ra.ParVector(ctx, n * k, dt)
+            ra.vcycle_block(ml, X, ra.ParVector.from_numpy(ctx, rhs.ravel()), k, prec)
+            Xh = X.numpy().reshape(n, k)
+            for c in cols:
+                assert np.array_equal(Xh[:, c], want[c][i]), (code, prec, c)
