@@ -696,10 +696,15 @@ __global__ __launch_bounds__(256) void bcol_dots(int n, int k, int kp, const dou
 
 // r -= alpha Ap; r32 = (float) r; per-column sums of r^2.  The step
 // x += alpha p of the iteration is taken by the direction update (bdir),
-// which reads p anyway, or by bstep_x when the iteration ends there.
+// which reads p anyway, or by bstep_x when the iteration ends there.  With z
+// given, also the cycle's first Jacobi sweep from zero on r (r32 in the FP32
+// form; bjacobi_from_zero's operations, diagonal d, weight w): that pass read
+// r again (1M rows x 32, FP32 cycle: 187 + 59 us in two passes, 224 us here).
+template <typename Z>
 __global__ __launch_bounds__(256) void bupdate(int n, int k, int kp, const double* __restrict__ alpha,
                                                const double* __restrict__ Ap, double* __restrict__ r,
-                                               float* __restrict__ r32, double* __restrict__ partials)
+                                               float* __restrict__ r32, double* __restrict__ partials,
+                                               Z* __restrict__ z, const Z* __restrict__ d, Z w)
 {
     const int c = threadIdx.x & (kp - 1);
     const int rpb = 256 / kp;
@@ -709,12 +714,14 @@ __global__ __launch_bounds__(256) void bupdate(int n, int k, int kp, const doubl
         const double al = alpha[c];
         for (int64_t i0 = (int64_t)blockIdx.x * rpb + threadIdx.x / kp; i0 < n; i0 += kColUnroll * stride) {
             double rv[kColUnroll], av[kColUnroll];
+            Z dv[kColUnroll];
 #pragma unroll
             for (int u = 0; u < kColUnroll; u++) {
                 const int64_t i = i0 + u * stride;
                 const size_t e = (size_t)(i < n ? i : 0) * k + c;
                 rv[u] = i < n ? r[e] : 0.0;
                 av[u] = i < n ? Ap[e] : 0.0;
+                dv[u] = z && i < n ? d[i] : Z(0);
             }
 #pragma unroll
             for (int u = 0; u < kColUnroll; u++) {
@@ -724,6 +731,7 @@ __global__ __launch_bounds__(256) void bupdate(int n, int k, int kp, const doubl
                 const double ri = rv[u] - al * av[u];
                 r[e] = ri;
                 if (r32) r32[e] = (float)ri;
+                if (z) z[e] = jacobi_zero_row((Z)ri, dv[u], w);
                 s += ri * ri;
             }
         }
@@ -1189,10 +1197,11 @@ static void bouter(ramd_hier_s* h, BlockState* bs, const ramd_csr_s* A, int op, 
     blaunch<double>(A, code, op, bs->k, x, b, y, 0.0, h->ctx->stream);
 }
 
-static void bprecondition(ramd_hier_s* h, BlockState* bs, bool f32)
+// first_done: Z (Z32) holds the cycle's first sweep
+static void bprecondition(ramd_hier_s* h, BlockState* bs, bool f32, bool first_done = false)
 {
-    if (f32) bcycle<float>(h, bs, 0, bs->Z32, bs->R32);
-    else bcycle<double>(h, bs, 0, bs->Z, bs->R);
+    if (f32) bcycle<float>(h, bs, 0, bs->Z32, bs->R32, first_done);
+    else bcycle<double>(h, bs, 0, bs->Z, bs->R, first_done);
 }
 
 static int fpcg_block_run(ramd_hier_s* h, ramd_csr_s* A, int k, double* X_d, const double* B_d, double rtol,
@@ -1239,20 +1248,29 @@ static int fpcg_block_run(ramd_hier_s* h, ramd_csr_s* A, int k, double* X_d, con
         else RAMD_HIP(hipMemcpyAsync(bs->P, bs->Z, sizeof(double) * m, hipMemcpyDeviceToDevice, s));
         col_dots(ctx, bs, n, 0, bs->R, f32 ? (const void*)bs->Z32 : (const void*)bs->Z, f32, nullptr, S.rz, nullptr);
 
+        // the update pass also forms the cycle's first Jacobi sweep from zero
+        const bool fuse_first = h->levels.size() > 1 && h->opts.num_smooth_sweeps >= 1;
         auto stepA = [&] {
             bouter(h, bs, A, OP_SPMV, bs->P, nullptr, bs->AP);
             col_dots(ctx, bs, n, 0, bs->P, bs->AP, false, nullptr, S.pap, nullptr);
             hipLaunchKernelGGL(bscal_alpha, dim3(1), dim3(64), 0, s, k, S);
-            hipLaunchKernelGGL(bupdate, dim3(gc), dim3(256), 0, s, n, k, kp, S.alpha, bs->AP, bs->R,
-                               f32 ? bs->R32 : nullptr, bs->partials);
+            if (f32)
+                hipLaunchKernelGGL((bupdate<float>), dim3(gc), dim3(256), 0, s, n, k, kp, S.alpha, bs->AP, bs->R,
+                                   bs->R32, bs->partials, fuse_first ? bs->Z32 : nullptr, h->levels[0].diag32,
+                                   (float)h->opts.relax_weight);
+            else
+                hipLaunchKernelGGL((bupdate<double>), dim3(gc), dim3(256), 0, s, n, k, kp, S.alpha, bs->AP, bs->R,
+                                   (float*)nullptr, bs->partials, fuse_first ? bs->Z : nullptr, h->levels[0].diag,
+                                   h->opts.relax_weight);
             hipLaunchKernelGGL(bcol_final, dim3(k), dim3(256), 0, s, gc, k, bs->partials, S.rr);
             hipLaunchKernelGGL(bscal_relres, dim3(1), dim3(64), 0, s, k, rtol, S);
             RAMD_HIP(hipGetLastError());
         };
         // preconditioner step; with step_x the direction update also takes
-        // the iteration's step x += alpha p (one read of p)
+        // the iteration's step x += alpha p (one read of p), and Z holds the
+        // first sweep on the current R from the update pass
         auto stepB = [&](bool step_x) {
-            bprecondition(h, bs, f32);
+            bprecondition(h, bs, f32, fuse_first && step_x);
             col_dots(ctx, bs, n, 1, bs->R, f32 ? (const void*)bs->Z32 : (const void*)bs->Z, f32, bs->AP, S.rzn,
                      S.zap);
             hipLaunchKernelGGL(bscal_beta, dim3(1), dim3(64), 0, s, k, S);

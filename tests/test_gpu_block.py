@@ -241,3 +241,34 @@ def test_block_restriction_with_first_sweep(ctx, k, codes64, codes32):
             Xh = X.numpy().reshape(n, k)
             for c in cols:
                 assert np.array_equal(Xh[:, c], want[c][i]), (code, prec, c)
+
+
+@pytest.mark.parametrize("sweeps", [1, 2])
+@pytest.mark.parametrize("prec", [ra.PREC_FP64, ra.PREC_FP32])
+def test_block_fpcg_first_sweep_in_update(ctx, sweeps, prec):
+    """The lockstep solve whose update pass writes the cycle's first sweep: with
+    one and with two sweeps, every column takes the single-vector solve's
+    iterations (within one: the dots are summed in another order) and reaches
+    its true residual, in eager launches and replayed."""
+    rp, col, val = ra.gallery_laplace27(14)
+    n, k, rtol = rp.size - 1, 5, 1e-9
+    ml = ra.ParRugeStubenSolver(ctx, 0.25, ra.PMIS, ra.Extended, ra.Classical, ra.Jacobi)
+    ml.relax_weight = OMEGA
+    ml.num_smooth_sweeps = sweeps
+    ml.setup(rp, col, val)
+    ml.enable_fp32()
+    A = ra.ParCSRMatrix.from_csr(ctx, rp, col, val)
+    B = np.random.default_rng(70 + sweeps).standard_normal((n, k))
+    a = K.Csr(rp, col, val)
+    for use_graph in (False, True):
+        X = ra.ParVector.from_numpy(ctx, np.zeros(n * k))
+        its, relres, total = ra.FPCG_block(A, ml, X, ra.ParVector.from_numpy(ctx, B.ravel()), k, rtol, 100, prec,
+                                           use_graph)
+        Xh = X.numpy().reshape(n, k)
+        for c in range(k):
+            x = ra.ParVector.from_numpy(ctx, np.zeros(n))
+            b = ra.ParVector.from_numpy(ctx, B[:, c].copy())
+            _, n1, _ = ra.FPCG(A, ml, x, b, rtol, 100, prec)
+            assert abs(int(its[c]) - n1) <= 1, (c, its[c], n1)
+            res = np.linalg.norm(B[:, c] - K.spmv(a, Xh[:, c])) / np.linalg.norm(B[:, c])
+            assert res <= rtol * 1.001, (c, res)
