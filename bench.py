@@ -368,9 +368,10 @@ def kernel_template(slot, kind, nd, staging=None, uniform=False):
     if kind == "dia_kernel":
         mode = staging[0] if staging else 0
         if mode == 2:
-            L = staging[2]
+            L, P = staging[2:4]
             tx = 64 if L % 64 == 0 else 32 if L % 32 == 0 else 16 if L % 16 == 0 else 64
-            if uniform:  # the caller's operator, stored in ascending order
+            if uniform:  # the caller's operator, stored in ascending order; the fewest positions past the grid
+                tx = min((32, 16, 64), key=lambda t: -(-L // t) * t * (-(-(P // L) * t // 256) * 256 // t))
                 return f"ramd::dia_uni_box_kernel<{op}, {vec}, {nd}, {tx}, false>"
             return f"ramd::dia_box_kernel<{op}, float, {vec}, {nd}, {tx}>"
         name = "dia_lds_kernel" if mode == 1 else "dia_kernel"

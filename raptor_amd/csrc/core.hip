@@ -936,9 +936,10 @@ __global__ void transpose_scatter_kernel(int n, const int* __restrict__ rp, cons
 
 // Every column's (row, value) pairs in row order: a group of G lanes per
 // column, each entry's place the number of smaller rows in its column (a row
-// that stores the column twice put its entries in stored order).  One thread per column with an insertion sort
-// took 5.6 ms on average for the aggregation hierarchy of the 7-point 96^3
-// operator, whose coarse columns hold hundreds of entries.
+// that stores the column twice put its entries in stored order).  One thread
+// per column with an insertion sort took 5.6 ms on average for the
+// aggregation hierarchy of the 7-point 96^3 operator, whose coarse columns
+// hold hundreds of entries.
 template <int G>
 __global__ __launch_bounds__(kBlockThreads) void transpose_rank_kernel(int m, const int* __restrict__ tp,
                                                                        const int* __restrict__ row_in,

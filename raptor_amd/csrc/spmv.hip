@@ -944,9 +944,9 @@ __global__ __launch_bounds__(kBlockThreads) void dia_box_kernel(int n, int L, in
 // first), a wavefront whose rows all store every diagonal skips the selects,
 // and the row's mask and b are loaded one plane ahead.  The operations of a
 // row and their order are dia_box_kernel's: the same bits.  27 points, 256^3:
-// the outer product 420 -> 137 us, the FP32 residual and Jacobi 409 and 388
-// -> 101 and 97 us; FP64 residual at 192^3, 351 (gather) -> 58 us, 198 MB of
-// vectors and masks at 3.4 TB/s.
+// the outer product 420 -> 129 us, the FP32 residual and Jacobi 409 and 388
+// -> 101 and 97 us; FP64 residual at 192^3, 351 (gather) -> 57 us, 198 MB of
+// vectors and masks at 3.5 TB/s.
 template <typename X>
 struct DiaUni {
     X v[kDiaMax];

@@ -20,10 +20,10 @@
 // the cycle's vectors, are kept kTailDepth steps ahead in registers, across
 // slices and across the operations' barriers (which wait for LDS only, not
 // for these loads).  In a long row the loads are unconditional, so that the
-// wait before a step covers its own loads and not the younger ones.  Every operation runs
-// through one loop of few instructions per entry: the residual's subtraction
-// is the addition of the negated product (the same value), and padding needs
-// no test: its product is -0.0, and a + (-0.0) is a for every a.  A vector
+// wait before a step covers its own loads and not the younger ones.  Every
+// operation runs through one loop of few instructions per entry: the
+// residual's subtraction is the addition of the negated product (the same
+// value), and padding needs no test: its product is -0.0, and a + (-0.0) is a for every a.  A vector
 // that rows gather from starts with an entry for that, one the padding's
 // columns point to: +0.0, or -0.0 for the residual, whose values are negated
 // (padding's value is -0.0).
