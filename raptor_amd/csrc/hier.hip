@@ -253,16 +253,17 @@ constexpr int64_t kTailMaxOuterNnz = 65536;  // entries of its P
 static bool multicolour(const ramd_hier_s* h);
 static bool jfz_fused(const ramd_hier_s* h, int l);
 
-// Levels that can start the coarse tail, the largest tail first (none with
-// per-level timing on, multicolour smoothing or a coarse system past one
-// wavefront).  Tail levels hold at most kTailMaxRows rows and kTailMaxNnz
-// entries of A and of P; the level above them at most kTailMaxOuterRows
-// rows and kTailMaxOuterNnz entries of P.
-static std::vector<int> tail_candidates(const ramd_hier_s* h)
+// Levels that the coarse tail can be packed from, the largest tail first
+// (none with multicolour smoothing or a coarse system past one wavefront).
+// Tail levels hold at most kTailMaxRows rows and kTailMaxNnz entries of A and
+// of P; the level above them at most kTailMaxOuterRows rows and
+// kTailMaxOuterNnz entries of P.  Per-level timing is not asked about: it can
+// be switched off again after the pack.
+static std::vector<int> tail_packable(const ramd_hier_s* h)
 {
     std::vector<int> c;
     const int nlev = (int)h->levels.size();
-    if (h->track || multicolour(h) || nlev < 2 || h->coarse_n > kCoarseWave) return c;
+    if (multicolour(h) || nlev < 2 || h->coarse_n > kCoarseWave) return c;
     auto small = [&](int l) {
         const Level& L = h->levels[l];
         return L.n <= kTailMaxRows && L.A->diag_first && L.A->nnz <= kTailMaxNnz &&
@@ -283,10 +284,16 @@ static std::vector<int> tail_candidates(const ramd_hier_s* h)
     return c;
 }
 
+// Levels that a cycle can start the tail at: none while per-level timing is on.
+static std::vector<int> tail_candidates(const ramd_hier_s* h)
+{
+    return h->track ? std::vector<int>() : tail_packable(h);
+}
+
 // Packs the largest tail's levels for cycles in precision prec.
 static void pack_tail(ramd_hier_s* h, int prec)
 {
-    const std::vector<int> c = tail_candidates(h);
+    const std::vector<int> c = tail_packable(h);
     if (!c.empty()) tail_pack(h, c[0], prec);
 }
 

@@ -50,3 +50,41 @@ def test_tail_levels_bit_exact(ctx, n, wide, max_coarse, sweeps):
         assert np.array_equal(out[mode][0], out[-1][0]), mode
         assert np.array_equal(out[mode][1], out[-1][1]), mode
     ml.free()
+
+
+@pytest.mark.parametrize("first", ["cycle_fp32", "fpcg", "block"])
+def test_fp32_enabled_while_tracking(ctx, first):
+    """FP32 levels made while per-level timing is on have their tail as well:
+    with timing off again, the cycles with every tail run, and equal the one
+    without."""
+    n = 1000
+    M = laplace_1d(n, 17)
+    ml = ra.ParRugeStubenSolver(ctx, 0.25, ra.PMIS, ra.Direct, ra.Classical, ra.Jacobi)
+    ml.relax_weight = 2.0 / 3.0
+    ml.setup(*M)
+    A = ra.ParCSRMatrix.from_csr(ctx, *M)
+    b = np.random.default_rng(n).standard_normal(n)
+
+    def cycle():
+        x = ra.ParVector(ctx, n, np.float32)
+        ml.cycle_fp32(x, ra.ParVector.from_numpy(ctx, b.astype(np.float32)))
+        return x.numpy()
+
+    ml.set_track_times(True)
+    if first == "cycle_fp32":
+        cycle()
+    elif first == "fpcg":
+        ra.FPCG(A, ml, ra.ParVector.from_numpy(ctx, np.zeros(n)), ra.ParVector.from_numpy(ctx, b), 1e-8, 100,
+                ra.PREC_FP32)
+    else:
+        X = ra.ParVector(ctx, 2 * n, np.float32)
+        ra.vcycle_block(ml, X, ra.ParVector.from_numpy(ctx, np.repeat(b, 2).astype(np.float32)), 2, ra.PREC_FP32)
+    ml.set_track_times(False)
+    ml.set_tail(-1)
+    want = cycle()
+    _, start = ml.tail_level(ra.PREC_FP32)
+    assert start >= 1
+    for mode in [0] + list(range(start, ml.num_levels)):
+        ml.set_tail(mode)
+        assert np.array_equal(cycle(), want), mode
+    ml.free()
