@@ -376,9 +376,9 @@ void dia_box_detect(const long long* offs, int nd, int n, DiaBox& b);
 // (the number of per-workgroup partial sums of a fused product).
 int dia_grid(const ramd_csr_s* A, int pp);
 // The kernel of precision pair pp: lds_x[pp], and where it was not timed yet
-// (-1) the plane march for a uniform operator of a box geometry and the
-// gather for all others.
-int dia_mode(const Dia* d, int pp);
+// (-1) the plane march for a uniform operator of a box geometry that is large
+// enough for it, the gather for all others.
+int dia_mode(const ramd_csr_s* A, int pp);
 // A uniform operator whose diagonals are the built-in ones of the box (27- or
 // 7-point), in ascending order or with the centre first (*diag_first).
 bool dia_uni_box(const Dia* d, bool* diag_first);

@@ -1073,17 +1073,41 @@ bool dia_uni_box(const Dia* d, bool* diag_first)
     return false;
 }
 
-int dia_mode(const Dia* d, int pp)
+// Bytes of a pass that reads a uniform operator's value planes (values, mask,
+// three vectors) from which on the plane march without them is the faster one
+// before any timing.  A workgroup of the march walks four planes one after
+// another, 9 us for 27 points and 6 us for 7 however few rows there are; the
+// gather's time follows its bytes.  FP64 residual, gather / march: 27 points
+// 32^3 6.1 / 9.3 us, 56^3 (43 MB) 8.9 / 9.5, 64^3 (64 MB) 12.0 / 9.6, 101^3
+// 46.8 / 13.4; 7 points 32^3 5.0 / 5.8, 72^3 (31 MB) 6.3 / 6.6, 80^3 (43 MB)
+// 7.9 / 6.6, 128^3 29.9 / 11.8.
+constexpr double kUniMarchBytes = 43e6;
+
+// Whether the plane march of uniform operator A pays by that line times
+// `factor`: not on a grid whose tiles are less than a third full (7 points,
+// 3 x 1000 x 1000, a fifth full: gather 41.7 us, march 54.6).
+static bool uni_march_pays(const ramd_csr_s* A, int pp, double factor)
 {
+    const Dia* d = A->dia;
+    const int tx = d->box.utx, ty = kBlockThreads / tx, ny = d->box.P / d->box.L;
+    const long long area = (long long)((d->box.L + tx - 1) / tx * tx) * ((ny + ty - 1) / ty * ty);
+    const double row = (double)d->nd * (pp == 0 ? 8 : 4) + 4.0 + 3.0 * (pp == 1 ? 4 : 8);
+    return 3ll * d->box.P >= area && row * A->n_rows >= factor * kUniMarchBytes;
+}
+
+int dia_mode(const ramd_csr_s* A, int pp)
+{
+    const Dia* d = A->dia;
     bool df;
-    return d->lds_x[pp] >= 0 ? d->lds_x[pp] : (dia_uni_box(d, &df) ? 2 : 0);
+    return d->lds_x[pp] >= 0 ? d->lds_x[pp] : (dia_uni_box(d, &df) && uni_march_pays(A, pp, 1.0) ? 2 : 0);
 }
 
 // Whether launches of op read no values.
-static bool dia_reads_no_values(const Dia* d, int op, int pp)
+static bool dia_reads_no_values(const ramd_csr_s* A, int op, int pp)
 {
     bool df;
-    return (op == OP_SPMV || op == OP_RESIDUAL || op == OP_JACOBI) && dia_mode(d, pp) == 2 && dia_uni_box(d, &df);
+    return (op == OP_SPMV || op == OP_RESIDUAL || op == OP_JACOBI) && dia_mode(A, pp) == 2 &&
+           dia_uni_box(A->dia, &df);
 }
 
 // Workgroups of the plane march with tile width tx and zc planes each.
@@ -1099,7 +1123,7 @@ int dia_grid(const ramd_csr_s* A, int pp)
     const Dia* d = A->dia;
     const int n = A->n_rows;
     bool df;
-    if (dia_mode(d, pp) == 2 && d->box.L > 0)
+    if (dia_mode(A, pp) == 2 && d->box.L > 0)
         return box_grid(d->box, n, dia_uni_box(d, &df) ? d->box.utx : d->box.tx, d->box.zc[pp]);
     return std::max(1, (n + kBlockThreads - 1) / kBlockThreads);
 }
@@ -1122,7 +1146,7 @@ static void launch_dia_op(const ramd_csr_s* A, const V* val, const X* x, const X
     const int n = A->n_rows;
     dim3 grid((n + kBlockThreads - 1) / kBlockThreads), block(kBlockThreads);
     const int pp = sizeof(X) == 4 ? 1 : (sizeof(V) == 4 ? 2 : 0);
-    const int mode = dia_mode(d, pp);
+    const int mode = dia_mode(A, pp);
     if (mode == 2 && d->box.L > 0) {
         const DiaBox& bx = d->box;
         const int ty = kBlockThreads / bx.tx;
@@ -1232,7 +1256,7 @@ static hipEvent_t prof_event(ramd_ctx ctx)
 static double op_bytes(const ramd_csr_s* A, int op, int sv, int sx, bool dia)
 {
     double b;
-    if (dia && dia_reads_no_values(A->dia, op, sx == 4 ? 1 : (sv == 4 ? 2 : 0))) b = 4.0 * A->n_rows;
+    if (dia && dia_reads_no_values(A, op, sx == 4 ? 1 : (sv == 4 ? 2 : 0))) b = 4.0 * A->n_rows;
     else if (dia) b = (double)A->dia->nd * A->n_rows * sv + 4.0 * A->n_rows;
     else b = (double)A->nnz * (sv + 4.0) + 4.0 * (A->n_rows + 1);
     b += (double)sx * A->n_cols + (double)sx * A->n_rows;
@@ -1729,9 +1753,11 @@ void dia_autotune(ramd_csr_s* A, int pp)
         cands.push_back({2, kBoxPlanes});
         cands.push_back({2, 2 * kBoxPlanes});
         // a uniform operator's kernel reads little besides x, and the halo
-        // planes are a larger part of that
+        // planes are a larger part of that: 16 planes too, and the kernels
+        // that read values only where they can win
         bool df;
-        if (dia_uni_box(d, &df)) cands = {{2, kBoxPlanes}, {2, 2 * kBoxPlanes}, {2, 4 * kBoxPlanes}};
+        if (dia_uni_box(d, &df) && uni_march_pays(A, pp, 2.0))
+            cands = {{2, kBoxPlanes}, {2, 2 * kBoxPlanes}, {2, 4 * kBoxPlanes}};
     }
     float best = 1e30f;
     std::pair<int, int> pick = cands[0];

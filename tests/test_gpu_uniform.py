@@ -95,3 +95,31 @@ def test_value_changes_turn_it_off_and_on(ctx, what):
     D.set_values(ra.ParVector.from_numpy(ctx, 2.0 * A.val))
     assert D.uniform()
     check(ctx, D, K.Csr(A.rowptr, A.col, 2.0 * A.val))
+
+
+@pytest.mark.parametrize("dims,pts", [((56, 56, 56), 27), ((58, 56, 58), 27), ((81, 79, 79), 7), ((81, 79, 81), 7),
+                                      ((3, 700, 300), 7)])
+def test_both_sides_of_the_untimed_rule(ctx, dims, pts):
+    """The largest grids that the gather takes before any timing, the smallest
+    that the plane march takes, and one whose tiles are a fifth full."""
+    A = grid(*dims, pts, seed=5)
+    D = ra.ParCSRMatrix.from_csr(ctx, A.rowptr, A.col, A.val)
+    assert D.uniform() and D.dia_staging(0)[0] == -1
+    check(ctx, D, A)
+
+
+def test_small_operators_are_timed_against_the_gather(ctx):
+    """On 20 x 20 x 20 the march takes 9 us and the gather 5: a solve's timing
+    sees both."""
+    A = grid(20, 20, 20, 27, seed=5)
+    A.val[:] = np.where(A.col == np.repeat(np.arange(A.n_rows), np.diff(A.rowptr)), 26.5, -1.0)
+    ml = ra.ParRugeStubenSolver(ctx, 0.25, ra.PMIS, ra.Extended, ra.Classical, ra.Jacobi)
+    ml.relax_weight = 2.0 / 3.0
+    ml.setup(A.rowptr, A.col, A.val)
+    D = ra.ParCSRMatrix.from_csr(ctx, A.rowptr, A.col, A.val)
+    b = ra.ParVector.from_numpy(ctx, np.random.default_rng(1).standard_normal(A.n_rows))
+    ra.FPCG(D, ml, ra.ParVector.from_numpy(ctx, np.zeros(A.n_rows)), b, 1e-8, 100, ra.PREC_FP32)
+    assert D.uniform() and ml.level(0)[0].uniform()
+    assert D.dia_staging(2)[0] in (0, 1)
+    assert ml.level(0)[0].dia_staging(1)[0] in (0, 1)
+    ml.free()
