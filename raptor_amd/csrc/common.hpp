@@ -229,6 +229,14 @@ constexpr int box_slot(int nd, bool diag_first, int t)
     const int c = nd / 2;
     return !diag_first ? t : (t == 0 ? c : (t <= c ? t - 1 : t));
 }
+// What the device knows of a stencil-diagonal form's values (dia_check):
+// ref[t] is the value of slot t, the first found where rows differ and a
+// signalling NaN where no row stores it; v32 the same in FP32; flags.
+struct DiaValues {
+    double ref[kDiaMax];
+    float v32[kDiaMax];
+    int flags, pad;
+};
 struct Dia {
     int nd = 0;
     int center = -1;            // diagonal index of offset 0 (-1 if none)
@@ -241,10 +249,11 @@ struct Dia {
     // timed yet (gather).  Chosen by timing; the result bits are the same.
     int lds_x[3] = {-1, -1, -1};
     // every diagonal has one value in all rows that store it (constant
-    // coefficients): uval[t] is slot t's; the kernels of uniform operators
-    // read no values
+    // coefficients): the kernels of uniform operators read those of `values`
+    // instead of the planes.  They stay in device memory, so that captured
+    // launches follow a change of the numbers.
     bool uniform = false;
-    double uval[kDiaMax] = {};
+    DiaValues* values = nullptr;  // device
     unsigned* mask = nullptr;   // device, n
     double* v64 = nullptr;      // device, dia_slots<double>(nd) * n, dia_index layout
     float* v32 = nullptr;       // device, dia_slots<float>(nd) * n (built with the FP32 copy)

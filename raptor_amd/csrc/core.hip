@@ -153,6 +153,7 @@ void dia_free(Dia* d)
     dfree(d->mask);
     dfree(d->v64);
     dfree(d->v32);
+    dfree(d->values);
     delete d;
 }
 
@@ -261,21 +262,57 @@ __global__ void dia_fill_kernel(int n, int nd, int center, DiaArgs offs, const i
     if (f) atomicOr(flags, f);
 }
 
-// Sets flag 8 when a value of the planes is not exact in FP32 and 16 when two
-// rows store different values (different bits) of one diagonal; ref[t]
-// receives the value's bits where slot t has one.  Each workgroup compares its
-// rows' values in LDS and touches ref once per slot.
+// What the values of the stencil-diagonal form are: flag 8 when one is not
+// exact in FP32 and 16 when two rows store different values (different bits)
+// of one diagonal; out->ref[t] receives slot t's value where a row stores one.
+// Each workgroup compares its rows' values in LDS (r, the first value found of
+// every slot) and touches *out once per slot and for its flags: with the flags
+// looked at for every row, the loads queued for that one line (7 points, 96^3:
+// 85 us).
 constexpr unsigned long long kNoRef = 0x7ff4dead0000beefull;  // a signalling NaN: never taken as uniform
+constexpr int kDiaAllFlags = 24;
+
+__device__ __forceinline__ int dia_check_value(unsigned long long* r, int t, double v, int f)
+{
+    if ((double)(float)v != v) f |= 8;
+    const unsigned long long bits = (unsigned long long)__double_as_longlong(v);
+    unsigned long long o = r[t];
+    if (o == kNoRef) o = atomicCAS(&r[t], kNoRef, bits);
+    if ((o != kNoRef && o != bits) || bits == kNoRef) f |= 16;
+    return f;
+}
+
+// Every thread of the workgroup, with its flags f; known: the workgroup's
+// flags, `before` at the start.
+__device__ __forceinline__ void dia_check_merge(const unsigned long long* r, int* known, int before, int nd, int f,
+                                                DiaValues* out)
+{
+    if (f & ~before) atomicOr(known, f);
+    __syncthreads();
+    if ((int)threadIdx.x < nd && r[threadIdx.x] != kNoRef && !(*known & 16)) {
+        // mostly there already: looked at before the compare and swap, which
+        // the workgroups would queue for
+        unsigned long long* ref = reinterpret_cast<unsigned long long*>(&out->ref[threadIdx.x]);
+        unsigned long long o = __atomic_load_n(ref, __ATOMIC_RELAXED);
+        if (o == kNoRef) o = atomicCAS(ref, kNoRef, r[threadIdx.x]);
+        if (o != kNoRef && o != r[threadIdx.x]) atomicOr(known, 16);
+    }
+    __syncthreads();
+    if (threadIdx.x == 0 && (*known & ~before)) atomicOr(&out->flags, *known);
+}
+
+// The values of the planes as they are.
 __global__ __launch_bounds__(kBlockThreads) void dia_check_kernel(int n, int nd, DiaArgs a,
                                                                   const unsigned* __restrict__ mask,
                                                                   const double* __restrict__ v64,
-                                                                  unsigned long long* __restrict__ ref,
-                                                                  int* __restrict__ flags)
+                                                                  DiaValues* __restrict__ out)
 {
     __shared__ unsigned long long r[kDiaMax];
+    __shared__ int known;
     // the workgroup's first row gives the values to compare with; slots it
     // does not store take their first one below
     const int i0 = blockIdx.x * kBlockThreads;
+    if (threadIdx.x == 0) known = __atomic_load_n(&out->flags, __ATOMIC_RELAXED);
     if ((int)threadIdx.x < kDiaMax) {
         const int t = threadIdx.x;
         unsigned long long v = kNoRef;
@@ -284,69 +321,96 @@ __global__ __launch_bounds__(kBlockThreads) void dia_check_kernel(int n, int nd,
         r[t] = v;
     }
     __syncthreads();
+    const int before = known;
+    if (before == kDiaAllFlags) return;  // both found already
+    __syncthreads();
     int f = 0;
     for (int i = i0 + threadIdx.x; i < n; i += gridDim.x * kBlockThreads) {
-        if ((f | __atomic_load_n(flags, __ATOMIC_RELAXED)) == 24) break;  // both known
         const unsigned m = mask[i];
-        for (int t = 0; t < nd; t++) {
-            if (!((m >> a.ord[t]) & 1u)) continue;
-            const double v = v64[dia_index<double>(t, i, n)];
-            if ((double)(float)v != v) f |= 8;
-            const unsigned long long bits = (unsigned long long)__double_as_longlong(v);
-            unsigned long long o = r[t];
-            if (o == kNoRef) o = atomicCAS(&r[t], kNoRef, bits);
-            if ((o != kNoRef && o != bits) || bits == kNoRef) f |= 16;
-        }
+        for (int t = 0; t < nd && f != kDiaAllFlags; t++)
+            if ((m >> a.ord[t]) & 1u) f = dia_check_value(r, t, v64[dia_index<double>(t, i, n)], f);
+    }
+    dia_check_merge(r, &known, before, nd, f, out);
+}
+
+// Rewrites the stencil-diagonal planes from new CSR values (same pattern):
+// entry (row, col) lands on the plane of offset col - row.  Looks at the
+// values on the way, which a pass of its own would read again (set_values,
+// 7 points 96^3: 150 us with that pass, 27 points 96^3 990).
+__global__ __launch_bounds__(kBlockThreads) void dia_scatter_kernel(int n, DiaArgs a, int nd,
+                                                                    const int* __restrict__ rp,
+                                                                    const int* __restrict__ col,
+                                                                    const double* __restrict__ val,
+                                                                    double* __restrict__ v64,
+                                                                    DiaValues* __restrict__ out)
+{
+    __shared__ unsigned long long r[kDiaMax];
+    __shared__ int known;
+    const int i0 = blockIdx.x * kBlockThreads;
+    if (threadIdx.x == 0) known = __atomic_load_n(&out->flags, __ATOMIC_RELAXED);
+    if ((int)threadIdx.x < kDiaMax) r[threadIdx.x] = kNoRef;
+    __syncthreads();
+    const int before = known;
+    auto slot = [&](int d) {
+        int k = 0;
+        while (k < nd - 1 && a.off[k] != d) k++;
+        return a.pos[k];
+    };
+    if (i0 < n) {  // the first row's values to compare with
+        const int j = rp[i0] + (int)threadIdx.x;
+        if (j < rp[i0 + 1]) r[slot(col[j] - i0)] = (unsigned long long)__double_as_longlong(val[j]);
     }
     __syncthreads();
-    if ((int)threadIdx.x < nd && r[threadIdx.x] != kNoRef && !(f & 16)) {
-        const unsigned long long o = atomicCAS(&ref[threadIdx.x], kNoRef, r[threadIdx.x]);
-        if (o != kNoRef && o != r[threadIdx.x]) f |= 16;
+    int f = before;
+    for (int row = i0 + threadIdx.x; row < n; row += gridDim.x * kBlockThreads) {
+        for (int j = rp[row]; j < rp[row + 1]; j++) {
+            const int t = slot(col[j] - row);
+            const double v = val[j];
+            v64[dia_index<double>(t, row, n)] = v;
+            if (f != kDiaAllFlags) f = dia_check_value(r, t, v, f);
+        }
     }
-    if (f & ~__atomic_load_n(flags, __ATOMIC_RELAXED)) atomicOr(flags, f);
+    dia_check_merge(r, &known, before, nd, f, out);
 }
 
-__global__ void dia_check_init_kernel(unsigned long long* __restrict__ ref, int* __restrict__ flags)
+__global__ void dia_check_init_kernel(DiaValues* __restrict__ out)
 {
-    ref[threadIdx.x] = kNoRef;
-    if (threadIdx.x == 0) *flags = 0;
+    reinterpret_cast<unsigned long long*>(out->ref)[threadIdx.x] = kNoRef;
+    if (threadIdx.x == 0) out->flags = 0;
 }
 
-// v32_exact, uniform and uval of the planes' current values.
-static void dia_check(ramd_csr_s* A)
+// flags_h: host memory (a copy of one word by the runtime took 10 us more)
+__global__ void dia_check_finish_kernel(DiaValues* __restrict__ out, int* __restrict__ flags_h)
+{
+    out->v32[threadIdx.x] = (float)out->ref[threadIdx.x];
+    if (threadIdx.x == 0) *flags_h = out->flags;
+}
+
+// v32_exact, uniform and the device's values of the planes as they are now;
+// `scatter`: of the CSR values, written to the planes.
+static void dia_check(ramd_csr_s* A, bool scatter)
 {
     Dia* d = A->dia;
     hipStream_t s = A->ctx->stream;
     const int n = A->n_rows;
-    struct Out {
-        unsigned long long ref[kDiaMax];
-        int flags, pad;
-    } out;
-    unsigned long long* buf = dalloc<unsigned long long>(kDiaMax + 1);
-    int* flags = reinterpret_cast<int*>(buf + kDiaMax);
-    try {
-        hipLaunchKernelGGL(dia_check_init_kernel, dim3(1), dim3(kDiaMax), 0, s, buf, flags);
-        hipLaunchKernelGGL(dia_check_kernel, dim3((unsigned)std::min((n + kBlockThreads - 1) / kBlockThreads, 2048)),
-                           dim3(kBlockThreads), 0, s, n, d->nd, d->args, d->mask, d->v64, buf, flags);
-        RAMD_HIP(hipGetLastError());
-        RAMD_HIP(hipMemcpyAsync(&out, buf, sizeof(unsigned long long) * (kDiaMax + 1), hipMemcpyDeviceToHost, s));
-        RAMD_HIP(hipStreamSynchronize(s));
-    } catch (...) {
-        dfree(buf);
-        throw;
-    }
-    dfree(buf);
-    const bool exact = !(out.flags & 8), uniform = !(out.flags & 16);
-    bool same = d->v32_exact == exact && d->uniform == uniform;
-    for (int t = 0; t < d->nd && uniform; t++) {
-        double v = 0.0;
-        if (out.ref[t] != kNoRef) std::memcpy(&v, &out.ref[t], sizeof v);
-        same = same && std::memcmp(&v, &d->uval[t], sizeof v) == 0;
-        d->uval[t] = v;
-    }
+    const dim3 grid((unsigned)std::min((n + kBlockThreads - 1) / kBlockThreads, 2048)), blk(kBlockThreads);
+    if (!d->values) d->values = dalloc<DiaValues>(1);
+    hipLaunchKernelGGL(dia_check_init_kernel, dim3(1), dim3(kDiaMax), 0, s, d->values);
+    if (scatter)
+        hipLaunchKernelGGL(dia_scatter_kernel, grid, blk, 0, s, n, d->args, d->nd, A->rowptr, A->col, A->val, d->v64,
+                           d->values);
+    else hipLaunchKernelGGL(dia_check_kernel, grid, blk, 0, s, n, d->nd, d->args, d->mask, d->v64, d->values);
+    constexpr int kSlot = 7;  // of the context's mapped words; the solvers publish in the first ones
+    hipLaunchKernelGGL(dia_check_finish_kernel, dim3(1), dim3(kDiaMax), 0, s, d->values,
+                       (int*)(A->ctx->step_pin_d + kSlot));
+    RAMD_HIP(hipGetLastError());
+    RAMD_HIP(hipStreamSynchronize(s));
+    const int flags = *(const volatile int*)(A->ctx->step_pin + kSlot);
+    const bool exact = !(flags & 8), uniform = !(flags & 16);
+    // the kernels chosen depend on both (the numbers they read in memory)
+    if (d->v32_exact != exact || d->uniform != uniform) A->forms++;
     d->v32_exact = exact;
     d->uniform = uniform;
-    if (!same) A->forms++;  // the kernels chosen, and the values they are passed
 }
 
 void dia_box_detect(const long long* offs, int nd, int n, DiaBox& b)
@@ -518,7 +582,7 @@ bool dia_build(ramd_csr_s* A)
     }
     A->dia = d;
     A->forms++;
-    dia_check(A);
+    dia_check(A, false);
     return true;
 }
 
@@ -1190,21 +1254,6 @@ void csr_make_fp32(ramd_csr_s* A)
     if (A->dia && !A->dia->v32) dia_make_fp32(A);
 }
 
-// Rewrites the stencil-diagonal planes from new CSR values (same pattern):
-// entry (row, col) lands on the plane of offset col - row.
-__global__ void dia_scatter_kernel(int n, DiaArgs a, int nd, const int* __restrict__ rp, const int* __restrict__ col,
-                                   const double* __restrict__ val, double* __restrict__ v64)
-{
-    const int row = blockIdx.x * blockDim.x + threadIdx.x;
-    if (row >= n) return;
-    for (int j = rp[row]; j < rp[row + 1]; j++) {
-        const int d = col[j] - row;
-        int k = 0;
-        while (k < nd - 1 && a.off[k] != d) k++;
-        v64[dia_index<double>(a.pos[k], row, n)] = val[j];
-    }
-}
-
 void csr_set_values(ramd_csr_s* A, const double* val_d)
 {
     ramd_ctx ctx = A->ctx;
@@ -1227,11 +1276,7 @@ void csr_set_values(ramd_csr_s* A, const double* val_d)
     for (int p = 0; p < 2; p++)  // the sorted values follow (same order)
         if (A->sg[p]) sg_build(A, p);
     if (Dia* d = A->dia) {
-        const int n = A->n_rows;
-        hipLaunchKernelGGL(dia_scatter_kernel, dim3((n + 255) / 256), dim3(256), 0, s, n, d->args, d->nd, A->rowptr,
-                           A->col, A->val, d->v64);
-        RAMD_HIP(hipGetLastError());
-        dia_check(A);
+        dia_check(A, true);
         if (d->v32) dia_make_fp32(A);
     }
     RAMD_HIP(hipStreamSynchronize(s));

@@ -942,19 +942,17 @@ __global__ __launch_bounds__(kBlockThreads) void dia_box_kernel(int n, int L, in
 // instructions; hence the LDS offsets and the order of the diagonals are
 // compiled in (ND = 27: the whole box, ND = 7: its axes; DF: the centre
 // first), a wavefront whose rows all store every diagonal skips the selects,
-// and the row's mask and b are loaded one plane ahead.  The operations of a
-// row and their order are dia_box_kernel's: the same bits.  27 points, 256^3:
+// and the row's mask and b are loaded one plane ahead.  The values uv come
+// through scalar loads from device memory (as kernel arguments, which a capture
+// fixes, no faster: 256^3 product 113 us, 108 from memory; 64^3 9.5 and 9.8).
+// The operations of a row and their order are dia_box_kernel's: the same bits.  27 points, 256^3:
 // the outer product 420 -> 129 us, the FP32 residual and Jacobi 409 and 388
 // -> 101 and 97 us; FP64 residual at 192^3, 351 (gather) -> 57 us, 198 MB of
 // vectors and masks at 3.5 TB/s.
-template <typename X>
-struct DiaUni {
-    X v[kDiaMax];
-};
-
 template <int OP, typename X, int ND, int TX, bool DF>
 __global__ __launch_bounds__(kBlockThreads) void dia_uni_box_kernel(int n, int L, int P, int nxt, int nyt, int zc,
-                                                                   DiaUni<X> uv, const unsigned* __restrict__ mask,
+                                                                   const X* __restrict__ uv,
+                                                                   const unsigned* __restrict__ mask,
                                                                    const X* __restrict__ x, const X* __restrict__ b,
                                                                    X* __restrict__ y, X omega,
                                                                    double* __restrict__ dotp)
@@ -1029,10 +1027,10 @@ __global__ __launch_bounds__(kBlockThreads) void dia_uni_box_kernel(int n, int L
                 const int k = box_slot(ND, DF, t);
                 const bool on = decltype(all)::value || ((m >> k) & 1u);
                 if (OP == OP_JACOBI && k == C) {
-                    diag = on ? uv.v[t] : X(0);
+                    diag = on ? uv[t] : X(0);
                     continue;
                 }
-                const X p = uv.v[t] * pl[box_dz(ND, k) + 1][box_dy(ND, k) * RW + box_dx(ND, k)];
+                const X p = uv[t] * pl[box_dz(ND, k) + 1][box_dy(ND, k) * RW + box_dx(ND, k)];
                 const X nxt_ = OP == OP_RESIDUAL ? acc - p : acc + p;
                 acc = on ? nxt_ : acc;
             }
@@ -1159,8 +1157,9 @@ static void launch_dia_op(const ramd_csr_s* A, const V* val, const X* x, const X
                 const int uty = kBlockThreads / bx.utx;
                 const int unxt = (bx.L + bx.utx - 1) / bx.utx, unyt = (bx.P / bx.L + uty - 1) / uty;
                 const dim3 ugrid((unsigned)box_grid(bx, n, bx.utx, zc));
-                DiaUni<X> uv{};
-                for (int t = 0; t < d->nd; t++) uv.v[t] = X(d->uval[t]);
+                const X* uv;
+                if constexpr (sizeof(X) == 4) uv = d->values->v32;
+                else uv = d->values->ref;
 #define DIA_UNI(NDV, TXV, DFV)                                                                                    \
     hipLaunchKernelGGL((dia_uni_box_kernel<OP, X, NDV, TXV, DFV>), ugrid, block, 0, s, n, bx.L, bx.P, unxt, unyt, \
                        zc, uv, d->mask, x, b, y, omega, dotp)

@@ -123,3 +123,46 @@ def test_small_operators_are_timed_against_the_gather(ctx):
     assert D.dia_staging(2)[0] in (0, 1)
     assert ml.level(0)[0].dia_staging(1)[0] in (0, 1)
     ml.free()
+
+
+@pytest.mark.parametrize("prec", [ra.PREC_FP64, ra.PREC_FP32])
+@pytest.mark.parametrize("block", [False, True])
+def test_replayed_solves_follow_new_values(ctx, prec, block):
+    """One capture serves every constant-coefficient operator: scaled values
+    between replayed solves give the eager solves' bits, and so do values that
+    are not uniform and uniform ones again."""
+    A = grid(65, 64, 66, 27, seed=5)  # past the size from which the march is taken
+    diag = A.col == np.repeat(np.arange(A.n_rows), np.diff(A.rowptr))
+    A.val[:] = np.where(diag, 26.5, -1.0)
+    ml = ra.ParRugeStubenSolver(ctx, 0.25, ra.PMIS, ra.Extended, ra.Classical, ra.Jacobi)
+    ml.relax_weight = 2.0 / 3.0
+    ml.setup(A.rowptr, A.col, A.val)
+    D = ra.ParCSRMatrix.from_csr(ctx, A.rowptr, A.col, A.val)
+    n, k = A.n_rows, 2
+    b = np.random.default_rng(1).standard_normal((n, k) if block else n)
+
+    def solve(graphs):
+        x = ra.ParVector.from_numpy(ctx, np.zeros(b.size))
+        if block:
+            ra.FPCG_block(D, ml, x, ra.ParVector.from_numpy(ctx, b.ravel()), k, 1e-8, 100, prec, graphs)
+        else:
+            ctx.set_graphs(graphs)
+            ra.FPCG(D, ml, x, ra.ParVector.from_numpy(ctx, b), 1e-8, 100, prec)
+            ctx.set_graphs(False)
+        return x.numpy()
+
+    seen = []
+    for step in range(6):
+        v = A.val * (1.0 + step)
+        if step == 3:
+            v[diag] += np.linspace(0.0, 0.1, n)
+        D.set_values(ra.ParVector.from_numpy(ctx, v))
+        assert D.uniform() == (step != 3)
+        got = solve(True)
+        assert np.array_equal(got, solve(False)), step
+        x = got.reshape(n, -1)[:, 0]
+        res = b.reshape(n, -1)[:, 0] - K.spmv(K.Csr(A.rowptr, A.col, v), np.ascontiguousarray(x))
+        assert np.linalg.norm(res) <= 2e-8 * np.linalg.norm(b.reshape(n, -1)[:, 0])
+        seen.append(got)
+    assert not any(np.array_equal(seen[0], s) for s in seen[1:])
+    ml.free()
