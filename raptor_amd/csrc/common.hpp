@@ -215,7 +215,9 @@ struct DiaBox {
     int tx = 64;       // tile width (TY = kBlockThreads / tx)
     int utx = 32;      // ... of the kernels of uniform operators
     BoxArgs args{};
-    int zc[3] = {kBoxPlanes, kBoxPlanes, kBoxPlanes};  // planes per workgroup, per precision pair
+    // planes per workgroup, per precision pair: [0] of the kernels that read
+    // values, [1] while those of uniform operators run
+    int zc[2][3] = {{kBoxPlanes, kBoxPlanes, kBoxPlanes}, {kBoxPlanes, kBoxPlanes, kBoxPlanes}};
 };
 // The 27- and 7-point operators' offsets in ascending order are the whole
 // box or its axes: the kernels of uniform operators have the LDS offsets of
@@ -246,8 +248,10 @@ struct Dia {
     // per (values, vectors) precision ([0] FP64/FP64, [1] FP32/FP32,
     // [2] FP32/FP64): 2 = plane-march with the x planes in LDS (box
     // geometry only), 1 = stage the x window in LDS, 0 = gather, -1 = not
-    // timed yet (gather).  Chosen by timing; the result bits are the same.
-    int lds_x[3] = {-1, -1, -1};
+    // timed yet (dia_mode).  Chosen by timing; the result bits are the same.
+    // [1]: while the kernels of uniform operators run (dia_uni_box), whose
+    // best choice is another one; new values move between the two.
+    int lds_x[2][3] = {{-1, -1, -1}, {-1, -1, -1}};
     // every diagonal has one value in all rows that store it (constant
     // coefficients): the kernels of uniform operators read those of `values`
     // instead of the planes.  They stay in device memory, so that captured
@@ -384,7 +388,7 @@ void dia_box_detect(const long long* offs, int nd, int n, DiaBox& b);
 // Workgroups of the stencil-diagonal kernels of A for precision pair pp
 // (the number of per-workgroup partial sums of a fused product).
 int dia_grid(const ramd_csr_s* A, int pp);
-// The kernel of precision pair pp: lds_x[pp], and where it was not timed yet
+// The kernel of precision pair pp: the choice made, and where it was not timed yet
 // (-1) the plane march for a uniform operator of a box geometry that is large
 // enough for it, the gather for all others.
 int dia_mode(const ramd_csr_s* A, int pp);

@@ -468,7 +468,7 @@ void dia_box_detect(const long long* offs, int nd, int n, DiaBox& b)
         }
     }
     const long long wgs8 = best / kBlockThreads * ((n / b.P + 7) / 8);
-    for (int& zc : b.zc) zc = wgs8 >= 2048 ? 2 * kBoxPlanes : kBoxPlanes;
+    for (int& zc : b.zc[1]) zc = wgs8 >= 2048 ? 2 * kBoxPlanes : kBoxPlanes;
     for (int k = 0; k < kDiaMax; k++) {
         int dz = 0, dy = 0, dx = 0;
         if (k < nd) split(offs[k], b.L, b.P, dz, dy, dx);
@@ -1479,8 +1479,10 @@ int ramd_csr_set_dia_staging(ramd_csr A, int pp, int mode, int planes)
         RAMD_CHECK(planes == 0 || (mode == 2 && planes >= kBoxMinPlanes && planes <= kBoxMaxPlanes), RAMD_E_ARG,
                    "ramd_csr_set_dia_staging: %d planes per workgroup (%d..%d, plane-march only)", planes,
                    kBoxMinPlanes, kBoxMaxPlanes);
-        A->dia->lds_x[pp] = mode;
-        if (planes) A->dia->box.zc[pp] = planes;
+        for (int u = 0; u < 2; u++) {  // whatever values follow
+            A->dia->lds_x[u][pp] = mode;
+            if (planes) A->dia->box.zc[u][pp] = planes;
+        }
         A->forms++;
     });
 }
@@ -1491,8 +1493,10 @@ int ramd_csr_dia_staging(ramd_csr A, int pp, int* mode, int* planes, int* L, int
         RAMD_CHECK(A && pp >= 0 && pp < 3 && mode && planes && L && P, RAMD_E_ARG,
                    "ramd_csr_dia_staging: bad argument");
         RAMD_CHECK(A->dia, RAMD_E_STATE, "ramd_csr_dia_staging: matrix has no stencil-diagonal form");
-        *mode = A->dia->lds_x[pp];
-        *planes = A->dia->box.zc[pp];
+        bool df;
+        const int u = dia_uni_box(A->dia, &df);
+        *mode = A->dia->lds_x[u][pp];
+        *planes = A->dia->box.zc[u][pp];
         *L = A->dia->box.L;
         *P = A->dia->box.P;
     });

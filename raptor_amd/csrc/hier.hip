@@ -1396,7 +1396,11 @@ static int fpcg_run(ramd_hier_s* h, ramd_csr_s* A, double* x_d, const double* b_
     if (noalloc) {
         RAMD_CHECK(!f32 || h->fp32, RAMD_E_STATE,
                    "ramd_fpcg_noalloc: the hierarchy's FP32 copies are not built (ramd_hier_enable_fp32)");
-        RAMD_CHECK(!A->dia || (A->val32 && A->dia->v32 && A->dia->lds_x[A->v32_outer ? 2 : 0] >= 0), RAMD_E_STATE,
+        // (a choice made for either kind of values: without one for the present
+        // kind the untimed rule holds)
+        const int pp = A->v32_outer ? 2 : 0;
+        RAMD_CHECK(!A->dia || (A->val32 && A->dia->v32 && std::max(A->dia->lds_x[0][pp], A->dia->lds_x[1][pp]) >= 0),
+                   RAMD_E_STATE,
                    "ramd_fpcg_noalloc: the operator's FP32 values and kernel choice are made by a first "
                    "ramd_fpcg call with it");
         RAMD_CHECK(!h->track && ctx->prof_min_nnz < 0, RAMD_E_STATE,

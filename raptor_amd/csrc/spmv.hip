@@ -1097,7 +1097,8 @@ int dia_mode(const ramd_csr_s* A, int pp)
 {
     const Dia* d = A->dia;
     bool df;
-    return d->lds_x[pp] >= 0 ? d->lds_x[pp] : (dia_uni_box(d, &df) && uni_march_pays(A, pp, 1.0) ? 2 : 0);
+    const bool u = dia_uni_box(d, &df);
+    return d->lds_x[u][pp] >= 0 ? d->lds_x[u][pp] : (u && uni_march_pays(A, pp, 1.0) ? 2 : 0);
 }
 
 // Whether launches of op read no values.
@@ -1121,8 +1122,8 @@ int dia_grid(const ramd_csr_s* A, int pp)
     const Dia* d = A->dia;
     const int n = A->n_rows;
     bool df;
-    if (dia_mode(A, pp) == 2 && d->box.L > 0)
-        return box_grid(d->box, n, dia_uni_box(d, &df) ? d->box.utx : d->box.tx, d->box.zc[pp]);
+    const bool u = dia_uni_box(d, &df);
+    if (dia_mode(A, pp) == 2 && d->box.L > 0) return box_grid(d->box, n, u ? d->box.utx : d->box.tx, d->box.zc[u][pp]);
     return std::max(1, (n + kBlockThreads - 1) / kBlockThreads);
 }
 
@@ -1149,11 +1150,12 @@ static void launch_dia_op(const ramd_csr_s* A, const V* val, const X* x, const X
         const DiaBox& bx = d->box;
         const int ty = kBlockThreads / bx.tx;
         const int nxt = (bx.L + bx.tx - 1) / bx.tx, nyt = (bx.P / bx.L + ty - 1) / ty;
-        const int zc = bx.zc[pp];
+        bool df = false;
+        const bool u = dia_uni_box(d, &df);
+        const int zc = bx.zc[u][pp];
         const dim3 bgrid((unsigned)box_grid(bx, n, bx.tx, zc));
         if constexpr (OP == OP_SPMV || OP == OP_RESIDUAL || OP == OP_JACOBI) {
-            bool df = false;
-            if (dia_uni_box(d, &df)) {
+            if (u) {
                 const int uty = kBlockThreads / bx.utx;
                 const int unxt = (bx.L + bx.utx - 1) / bx.utx, unyt = (bx.P / bx.L + uty - 1) / uty;
                 const dim3 ugrid((unsigned)box_grid(bx, n, bx.utx, zc));
@@ -1715,7 +1717,9 @@ void csr_autotune(ramd_csr_s* A, int prec)
 void dia_autotune(ramd_csr_s* A, int pp)
 {
     Dia* d = A->dia;
-    if (!d || A->n_rows == 0 || d->lds_x[pp] >= 0) return;
+    bool df;
+    const bool u = d && dia_uni_box(d, &df);
+    if (!d || A->n_rows == 0 || d->lds_x[u][pp] >= 0) return;
     RAMD_CHECK(pp == 0 || d->v32, RAMD_E_STATE, "dia_autotune: FP32 values were not built");
     ramd_ctx ctx = A->ctx;
     hipStream_t s = ctx->stream;
@@ -1754,16 +1758,17 @@ void dia_autotune(ramd_csr_s* A, int pp)
         // a uniform operator's kernel reads little besides x, and the halo
         // planes are a larger part of that: 16 planes too, and the kernels
         // that read values only where they can win
-        bool df;
-        if (dia_uni_box(d, &df) && uni_march_pays(A, pp, 2.0))
+        if (u && uni_march_pays(A, pp, 2.0))
             cands = {{2, kBoxPlanes}, {2, 2 * kBoxPlanes}, {2, 4 * kBoxPlanes}};
     }
     float best = 1e30f;
     std::pair<int, int> pick = cands[0];
-    const int zc0 = d->box.zc[pp];
+    int& mode = d->lds_x[u][pp];
+    int& zc = d->box.zc[u][pp];
+    const int zc0 = zc;
     for (const auto& c : cands) {
-        d->lds_x[pp] = c.first;
-        if (c.first == 2) d->box.zc[pp] = c.second;
+        mode = c.first;
+        if (c.first == 2) zc = c.second;
         // the operations each pair runs: the cycle's residual and Jacobi
         // sweep, the outer product with its fused dot
         auto run = [&](int op) {
@@ -1785,8 +1790,8 @@ void dia_autotune(ramd_csr_s* A, int pp)
             pick = c;
         }
     }
-    d->lds_x[pp] = pick.first;
-    d->box.zc[pp] = pick.first == 2 ? pick.second : zc0;
+    mode = pick.first;
+    zc = pick.first == 2 ? pick.second : zc0;
     A->forms++;
 }
 

@@ -166,3 +166,48 @@ def test_replayed_solves_follow_new_values(ctx, prec, block):
         seen.append(got)
     assert not any(np.array_equal(seen[0], s) for s in seen[1:])
     ml.free()
+
+
+def test_choices_follow_the_kind_of_values(ctx):
+    """The timed kernel choice of a uniform operator and that of the same
+    operator with other values are kept apart, a forced one holds for both, and
+    the solve without allocations runs on a kind of values not timed yet."""
+    A = grid(33, 32, 34, 27, seed=5)
+    diag = A.col == np.repeat(np.arange(A.n_rows), np.diff(A.rowptr))
+    A.val[:] = np.where(diag, 26.5, -1.0)
+    n = A.n_rows
+    other = A.val + np.where(diag, np.float64(np.float32(np.linspace(0.0, 0.5, A.val.size))), 0.0)
+    ml = ra.ParRugeStubenSolver(ctx, 0.25, ra.PMIS, ra.Extended, ra.Classical, ra.Jacobi)
+    ml.relax_weight = 2.0 / 3.0
+    ml.setup(A.rowptr, A.col, A.val)
+    D = ra.ParCSRMatrix.from_csr(ctx, A.rowptr, A.col, A.val)
+    b = np.random.default_rng(1).standard_normal(n)
+
+    def solve(f):
+        x = ra.ParVector.from_numpy(ctx, np.zeros(n))
+        f(D, ml, x, ra.ParVector.from_numpy(ctx, b), 1e-8, 100, ra.PREC_FP32)
+        return x.numpy()
+
+    def values(v):
+        D.set_values(ra.ParVector.from_numpy(ctx, v))
+
+    solve(ra.FPCG)
+    first = D.dia_staging(2)
+    assert first[0] >= 0
+    values(other)
+    assert not D.uniform() and D.dia_staging(2)[0] == -1
+    x = solve(ra.FPCG_noalloc)
+    assert np.linalg.norm(b - K.spmv(K.Csr(A.rowptr, A.col, other), x)) <= 2e-8 * np.linalg.norm(b)
+    solve(ra.FPCG)
+    second = D.dia_staging(2)
+    assert second[0] >= 0
+    values(3.0 * A.val)
+    assert D.uniform() and D.dia_staging(2) == first
+    values(other)
+    assert D.dia_staging(2) == second
+    D.set_dia_staging(2, 2, 5)
+    for v in (A.val, other, A.val):
+        values(v)
+        solve(ra.FPCG)
+        assert D.dia_staging(2)[:2] == (2, 5)
+    ml.free()
