@@ -1742,8 +1742,10 @@ void dia_autotune(ramd_csr_s* A, int pp)
     t.part = dalloc<double>((size_t)dia_grid_bound(A));
     RAMD_HIP(hipMemsetAsync(t.x, 0, bytes, s));
     RAMD_HIP(hipMemsetAsync(t.b, 0, bytes, s));
-    // bytes an operation moves: values, mask and three vectors per row
-    const size_t op_b = (size_t)A->n_rows * ((size_t)d->nd * (pp == 0 ? 8 : 4) + 4 + 3 * w);
+    // bytes an operation moves: values, mask and three vectors per row; for a
+    // uniform operator without the values, also for its candidates that read
+    // them, so that all are timed with the same caches
+    const size_t op_b = (size_t)A->n_rows * ((u ? 0 : (size_t)d->nd * (pp == 0 ? 8 : 4)) + 4 + 3 * w);
     // candidates: (mode, planes per workgroup)
     std::vector<std::pair<int, int>> cands = {{0, 0}};
     if (d->window.win <= kDiaWin) cands.push_back({1, 0});
