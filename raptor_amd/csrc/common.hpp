@@ -46,8 +46,11 @@ constexpr double kLaneRowsMaxLen = 8.0;
 // this many entries per row
 constexpr double kWaveRowsMinLen = 24.0;
 constexpr int kStreamCap = 4096;     // products staged in LDS per workgroup
-// entry bytes up to which an untuned matrix is read through the caches
-constexpr double kKeepBytes = 96e6;
+// entry bytes from and up to which an untuned matrix is read through the
+// caches, the former also with a cycle between its products
+constexpr double kKeepMinBytes = 12e6;
+constexpr double kKeepMinCycled = 50e6;
+constexpr double kKeepMaxBytes = 96e6;
 constexpr int kMaxRowsPerBlock = 256;
 
 // Row blocks for the LDS-staged kernels: consecutive rows whose nonzeros fit
@@ -329,6 +332,7 @@ struct ramd_csr_s {
         int* d = nullptr;  // == blocks for the default cap
     } rb[2];
     bool tuned = false;  // csr_autotune chose among the CSR kernels
+    bool cycled = false;  // a hierarchy's cycle runs between its products (CycledScope)
     // lazily built transpose (gather form of A^T x), same drop-free pattern
     ramd_csr_s* trans = nullptr;
     // FP32 copy of the values (mixed-precision cycle)
@@ -354,6 +358,15 @@ struct ramd_csr_s {
 };
 
 namespace ramd {
+// The operator of a preconditioned solve, while the solve runs.
+struct CycledScope {
+    ramd_csr_s* A;
+    bool was;
+    explicit CycledScope(ramd_csr_s* a, bool on = true) : A(a), was(a->cycled) { A->cycled = was || on; }
+    ~CycledScope() { A->cycled = was; }
+    CycledScope(const CycledScope&) = delete;
+    CycledScope& operator=(const CycledScope&) = delete;
+};
 // Creates a handle around device arrays the library already owns.  temp: a
 // matrix that is never applied to vectors gets no row blocks, nor a host copy
 // of its row pointers that is not given (both are host loops over its rows).

@@ -1387,6 +1387,7 @@ static int fpcg_run(ramd_hier_s* h, ramd_csr_s* A, double* x_d, const double* b_
     hipStream_t s = ctx->stream;
     const int n = A->n_rows;
     RAMD_CHECK(n == h->levels[0].n, RAMD_E_ARG, "ramd_fpcg: A has %d rows, hierarchy %d", n, h->levels[0].n);
+    CycledScope cycled(A);
     const bool f32 = cycle_prec == RAMD_PREC_FP32;
     // Both forms: the outer FP64 operator reads FP32-stored values where
     // every value is exactly representable in FP32 (same FP64 arithmetic and
@@ -2168,6 +2169,7 @@ static int pcg_run(ramd_hier h, ramd_csr A, double* x_d, const double* b_d, doub
         hipStream_t s = ctx->stream;
         const int n = A->n_rows;
         RAMD_CHECK(n == h->levels[0].n, RAMD_E_ARG, "ramd_pcg: A has %d rows, hierarchy %d", n, h->levels[0].n);
+        CycledScope cycled(A);
         double *r = h->pr, *z = h->pz, *p = h->pp, *Ap = h->pAp;
         int nres = 0;
         auto push = [&](double v) {

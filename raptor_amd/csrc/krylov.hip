@@ -58,6 +58,7 @@ int bicgstab_run(ramd_hier_s* h, ramd_csr_s* A, double* x, const double* b, doub
     ramd_ctx ctx = A->ctx;
     hipStream_t s = ctx->stream;
     const int n = A->n_rows;
+    CycledScope cycled(A, h != nullptr);
     struct Bufs {
         double* v[8] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
         ~Bufs()

@@ -1290,12 +1290,20 @@ static void launch_stream_cap(const ramd_csr_s* A, const ramd_csr_s::RowBlocks& 
     }
     // A matrix no tuner has seen, small enough that it, its vectors and a few
     // like it stay in the 256 MB infinity cache between operations, is read
-    // through the caches: 300 thousand rows, 5.3 million entries, 38.1 -> 29.9
-    // us a product.  Inside a cycle the other levels' traffic evicts the
-    // entries anyway and the streaming loads are the faster ones (27-point
+    // through the caches.  Repeated products, streamed / kept: 6.2 MB of
+    // entries 6.1 / 6.0 us, 12.5 MB 6.9 / 6.2, 21 MB 9.7 / 7.8, 63 MB 35.3 /
+    // 29.9, 89 MB 51.7 / 40.9; on a matrix just made they are equal (63 MB 51
+    // us); taken in turn with 600 MB of other matrices, which none stays for,
+    // keeping costs 4 to 8% (36.5 / 39.6).  With a cycle between the products
+    // the kept entries push its vectors out of the L2s, and only from about 50
+    // MB on is that made up for (flexible PCG on a 27-point matrix in CSR form:
+    // 20 MB 1.18 / 1.23 ms, 34 MB 1.35 / 1.40, 44 MB 1.54 / 1.54, 55 MB 1.68 /
+    // 1.64, 82 MB 2.00 / 1.96).  Level operators are tuned and streamed (27-point
     // 101^3 FP32 cycle 147 us, through the caches 157).
     if constexpr (CAP == kStreamCap && sizeof(V) == 8 && sizeof(X) == 8) {
-        if (!A->tuned && (double)A->nnz * 12.0 <= kKeepBytes && op != OP_SPMV_JFZ) {
+        const double bytes = (double)A->nnz * 12.0;
+        if (!A->tuned && bytes >= (A->cycled ? kKeepMinCycled : kKeepMinBytes) && bytes <= kKeepMaxBytes &&
+            op != OP_SPMV_JFZ) {
 #define KEEP_CASE(OPV)                                                                                              \
     case OPV:                                                                                                       \
         hipLaunchKernelGGL((stream_kernel<OPV, V, X, CAP, false, true>), grid, block, 0, s, A->rowptr, A->col, val, \
