@@ -607,10 +607,15 @@ __global__ void csr_check_kernel(int n, int n_cols, const int* __restrict__ rp, 
 // moved to the front (core/matrix.cpp:587-618, 729-787), one thread per row;
 // a row that is sorted already is only shifted.  flags: 2 as above
 // afterwards (a diagonal stored twice), 4 an unsorted row of more than
-// kOrderMaxRow entries, left as it was.
-constexpr int kOrderMaxRow = 512;
+// kOrderLongRow entries, left as it was.  Unsorted rows of more than
+// kOrderMaxRow entries are listed for csr_order_long_kernel: the insertion's
+// moves grow with the square of the length, one after another (a 1-D band's
+// setup with its rows in descending order, on one thread each: 201 entries 31
+// ms, 401 entries 79, sorted 14 and 18; the host's sort 40 and 51).
+constexpr int kOrderMaxRow = 32;
+constexpr int kOrderLongRow = 2048;
 __global__ void csr_order_kernel(int n, const int* __restrict__ rp, int* __restrict__ col, double* __restrict__ val,
-                                 int* __restrict__ flags)
+                                 int* __restrict__ flags, int* __restrict__ long_rows, int* __restrict__ n_long)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
@@ -619,7 +624,8 @@ __global__ void csr_order_kernel(int n, const int* __restrict__ rp, int* __restr
     for (int j = s + 1; j < e && sorted; j++) sorted = col[j - 1] <= col[j];
     if (!sorted) {
         if (e - s > kOrderMaxRow) {
-            atomicOr(flags, 4);
+            if (e - s > kOrderLongRow) atomicOr(flags, 4);
+            else long_rows[atomicAdd(n_long, 1)] = i;
             return;
         }
         for (int a = s + 1; a < e; a++) {
@@ -647,6 +653,38 @@ __global__ void csr_order_kernel(int n, const int* __restrict__ rp, int* __restr
     val[s] = v;
 }
 
+// The listed rows (at most kOrderLongRow entries), a wavefront each: the row in
+// LDS, every entry's place the number of entries before it.
+__global__ __launch_bounds__(64) void csr_order_long_kernel(const int* __restrict__ rows, const int* __restrict__ rp,
+                                                            int* __restrict__ col, double* __restrict__ val,
+                                                            int* __restrict__ flags)
+{
+    __shared__ int c[kOrderLongRow];
+    __shared__ double v[kOrderLongRow];
+    const int i = rows[blockIdx.x];
+    const int s = rp[i], len = rp[i + 1] - s;
+    for (int t = threadIdx.x; t < len; t += 64) {
+        c[t] = col[s + t];
+        v[t] = val[s + t];
+    }
+    __syncthreads();
+    for (int t = threadIdx.x; t < len; t += 64) {
+        const int ct = c[t];
+        int place = 0, before_diag = 0, diags = 0;
+#pragma unroll 8
+        for (int u = 0; u < len; u++) {
+            place += c[u] < ct || (c[u] == ct && u < t);
+            before_diag += c[u] < i;
+            diags += c[u] == i;
+        }
+        // the first diagonal entry goes to the front, those before it one on
+        if (diags) place = place == before_diag ? 0 : place + (place < before_diag ? 1 : 0);
+        col[s + place] = ct;
+        val[s + place] = v[t];
+        if (t == 0 && diags > 1) atomicOr(flags, 2);
+    }
+}
+
 // Host CSR arrays on the device (rowptr non-decreasing from 0 to nnz), their
 // columns checked there and, with `order`, the rows put in the hierarchy's
 // order; nullptr when a row needs the host's sort.  The handle has no
@@ -656,29 +694,28 @@ ramd_csr_s* csr_upload(ramd_ctx ctx, int n_rows, int n_cols, int64_t nnz, const 
 {
     hipStream_t s = ctx->stream;
     struct Tmp {
-        int *rp = nullptr, *col = nullptr, *flags = nullptr;
+        int *rp = nullptr, *col = nullptr, *flags = nullptr, *rows = nullptr;
         double* val = nullptr;
         ~Tmp()
         {
-            dfree(rp);
-            dfree(col);
-            dfree(flags);
+            for (int* p : {rp, col, flags, rows}) dfree(p);
             dfree(val);
         }
     } t;
     t.rp = dalloc<int>((size_t)n_rows + 1);
     t.col = dalloc<int>((size_t)nnz);
     t.val = dalloc<double>((size_t)nnz);
-    t.flags = dalloc<int>(1);
-    int flags = 0;
+    t.flags = dalloc<int>(2);  // and the number of listed rows
+    int out[2] = {0, 0};
+    int& flags = out[0];
     auto read_flags = [&] {
         RAMD_HIP(hipGetLastError());
-        RAMD_HIP(hipMemcpyAsync(&flags, t.flags, sizeof(int), hipMemcpyDeviceToHost, s));
+        RAMD_HIP(hipMemcpyAsync(out, t.flags, sizeof out, hipMemcpyDeviceToHost, s));
         RAMD_HIP(hipStreamSynchronize(s));
     };
     const dim3 grid((unsigned)((n_rows + 255) / 256));
     RAMD_HIP(hipMemcpyAsync(t.rp, rowptr, sizeof(int) * (n_rows + 1), hipMemcpyHostToDevice, s));
-    hipLaunchKernelGGL(fill_int_kernel, dim3(1), dim3(64), 0, s, t.flags, (int64_t)1, 0);
+    hipLaunchKernelGGL(fill_int_kernel, dim3(1), dim3(64), 0, s, t.flags, (int64_t)2, 0);
     if (nnz) {
         RAMD_HIP(hipMemcpyAsync(t.col, col, sizeof(int) * nnz, hipMemcpyHostToDevice, s));
         hipLaunchKernelGGL(csr_check_kernel, grid, dim3(256), 0, s, n_rows, n_cols, t.rp, t.col, t.flags);
@@ -690,10 +727,17 @@ ramd_csr_s* csr_upload(ramd_ctx ctx, int n_rows, int n_cols, int64_t nnz, const 
             RAMD_CHECK(col[j] >= 0 && col[j] < n_cols, RAMD_E_ARG, "%s: column %d of entry %lld outside [0,%d)", who,
                        col[j], (long long)j, n_cols);
     if (order && nnz) {
-        hipLaunchKernelGGL(fill_int_kernel, dim3(1), dim3(64), 0, s, t.flags, (int64_t)1, 0);
-        hipLaunchKernelGGL(csr_order_kernel, grid, dim3(256), 0, s, n_rows, t.rp, t.col, t.val, t.flags);
+        t.rows = dalloc<int>((size_t)(nnz / kOrderMaxRow));  // rows longer than that
+        hipLaunchKernelGGL(fill_int_kernel, dim3(1), dim3(64), 0, s, t.flags, (int64_t)2, 0);
+        hipLaunchKernelGGL(csr_order_kernel, grid, dim3(256), 0, s, n_rows, t.rp, t.col, t.val, t.flags, t.rows,
+                           t.flags + 1);
         read_flags();
         if (flags & 4) return nullptr;
+        if (out[1]) {
+            hipLaunchKernelGGL(csr_order_long_kernel, dim3((unsigned)out[1]), dim3(64), 0, s, t.rows, t.rp, t.col,
+                               t.val, t.flags);
+            read_flags();
+        }
     }
     ramd_csr_s* A = csr_wrap(ctx, n_rows, n_cols, nnz, t.rp, t.col, t.val, rowptr);
     t.rp = t.col = nullptr;

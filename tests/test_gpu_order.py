@@ -1,7 +1,8 @@
 """Row order of a hierarchy's fine matrix formed on the device (rows sorted,
 diagonal first): rows in any order, without a diagonal, with one stored twice,
-empty, and unsorted rows up to and past the device's 512 entries give the level
-that the host's ordering gives; bad columns and row pointers are refused."""
+empty, and unsorted rows up to and past the lengths at which the device changes
+its sort (32 entries) and leaves it to the host (2048) give the level that the
+host's ordering gives; bad columns and row pointers are refused."""
 import numpy as np
 import pytest
 
@@ -34,7 +35,8 @@ def matrix(n, longest, twice, seed):
     return np.array(rp, np.int32), np.concatenate(col).astype(np.int32), np.concatenate(val)
 
 
-@pytest.mark.parametrize("n,longest,twice", [(130, 20, False), (700, 512, False), (700, 513, False), (1500, 700, True)])
+@pytest.mark.parametrize("n,longest,twice", [(130, 20, False), (700, 512, False), (700, 513, False), (1500, 700, True),
+                                             (200, 32, False), (200, 33, True), (200, 64, False), (200, 65, True)])
 def test_fine_level_order(ctx, n, longest, twice):
     M = matrix(n, longest, twice, n + longest)
     got = []
@@ -62,3 +64,41 @@ def test_bad_input_refused(ctx):
     down[5], down[6] = rp[6], rp[5]
     with pytest.raises(ra.RamdError):
         ra.ParCSRMatrix.from_csr(ctx, down, col, val)
+    for device in (True, False):  # refused on the host: no kernel follows such pointers
+        ml = ra.ParRugeStubenSolver(ctx, 0.25, ra.PMIS, ra.Direct)
+        ml.device_setup = device
+        with pytest.raises(ra.RamdError, match="rowptr decreases"):
+            ml.setup(down, col, val)
+
+
+@pytest.mark.parametrize("order", ["shuffled", "descending"])
+@pytest.mark.parametrize("length", [31, 32, 33, 63, 64, 65, 300, 2047, 2048, 2049])
+@pytest.mark.parametrize("diagonals", [0, 1, 2])
+def test_one_long_row_each_way(ctx, length, order, diagonals):
+    """Rows of one length, repeated columns among them, with no diagonal, one
+    and two: the entries in the host's stable order."""
+    n = 500
+    rng = np.random.default_rng(length + diagonals)
+    rp, col, val = [0], [], []
+    for i in range(n):
+        if i % 61 == 7:
+            c = rng.choice(np.delete(np.arange(n), i), length - diagonals)
+            c[: length // 8] = c[length // 8: 2 * (length // 8)]  # some at least twice
+            c = np.concatenate([c, np.full(diagonals, i)])
+            c = rng.permutation(c) if order == "shuffled" else -np.sort(-c)
+        else:
+            c = np.array([i])
+        col.append(c)
+        val.append(rng.uniform(1.0, 2.0, c.size))
+        rp.append(rp[-1] + c.size)
+    M = np.array(rp, np.int32), np.concatenate(col).astype(np.int32), np.concatenate(val)
+    got = []
+    for device in (True, False):
+        ml = ra.ParRugeStubenSolver(ctx, 0.25, ra.PMIS, ra.Direct, ra.Classical, ra.Jacobi)
+        ml.device_setup = device
+        ml.max_levels = 1
+        ml.setup(*M)
+        got.append(ml.level(0)[0].to_csr())
+        ml.free()
+    for a, b in zip(*got):
+        assert np.array_equal(a, b)
