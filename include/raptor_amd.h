@@ -337,8 +337,8 @@ int ramd_hier_enable_fp32(ramd_hier h);
  * them and the interpolation out, as one workgroup in one launch instead of
  * one launch per operation.  Same bits either way.
  * level -1: off; 0 (default): automatic -- the first cycle in each
- * precision times V-cycles with the three largest tails and keeps the
- * fastest; >= 1: the tail starts at that level
+ * precision times V-cycles with the three largest tails and with none and
+ * keeps the fastest; >= 1: the tail starts at that level
  * (RAMD_E_ARG if it cannot).  No reference counterpart
  * (ParMultilevel::cycle, multilevel/par_multilevel.hpp:341-457, is one
  * routine per level); a tuning switch. */

@@ -319,15 +319,19 @@ static void cycle64(ramd_hier_s* h, int l, double* x, const double* b, bool x_ze
 static void cycle32(ramd_hier_s* h, int l, float* x, const float* b, bool x_zero, bool first_done);
 
 // Automatic mode: the first cycle in each precision times whole V-cycles
-// with the three largest tails, back to back and in turn (five rounds: the
-// coarse levels stay cached between cycles as they do in a solve), and keeps
-// the largest unless a smaller one's median is 1% below (same bits for all).  No smaller tail and
-// not the cycle without one: an operation inside the tail costs 0.7-2.5 us,
-// a launch of its own 3-5 us; only the largest levels' operations, bound by
+// with the three largest tails and with none, back to back and in turn (five
+// rounds: the coarse levels stay cached between cycles as they do in a solve),
+// and keeps the largest unless a later one's median is 1% below, without a tail
+// 3% (same bits for all; the queue hides the host time of the launches that a
+// smaller tail adds, about three without one: aggregation, 7 points 16^3, 33.0
+// us against 32.1 in the queue, 41.4 against 35.9 from a slow host).  No smaller tail: an operation inside the tail costs 0.7-2.5 us, a
+// launch of its own 3-5 us; only the largest levels' operations, bound by
 // what one compute unit reads, are in doubt (9-point anisotropic 100^2, FP64,
 // tails from levels of 780, 362, 168, 76, 34 rows and none: 96.6, 93.2,
-// 103.8, 121.0, 134.6, 142.7 us a cycle).  Uses the fine level's own x and b
-// vectors.
+// 103.8, 121.0, 134.6, 142.7 us a cycle).  A tail of the coarsest level alone,
+// whose restriction has a few long rows, can lose to none (aggregation, 7
+// points 80^3, 1173 -> 48 rows, FP32: 82.9 us, none 79.1).  Uses the fine
+// level's own x and b vectors.
 void cycle_prepare(ramd_hier_s* h, int prec)
 {
     if (prec == 1) enable_fp32(h);
@@ -338,10 +342,7 @@ void cycle_prepare(ramd_hier_s* h, int prec)
         return;
     }
     if (cand.size() > 3) cand.resize(3);
-    if (cand.size() == 1) {
-        h->tail_pick[prec] = cand[0];
-        return;
-    }
+    cand.push_back(-1);
     Level& L = h->levels[0];
     hipStream_t s = h->ctx->stream;
     std::function<void()> run;
@@ -387,9 +388,7 @@ void cycle_prepare(ramd_hier_s* h, int prec)
         std::vector<float> t(kRounds);
         for (int r = 0; r < kRounds; r++) t[r] = ms[(size_t)r * nc + i];
         std::nth_element(t.begin(), t.begin() + kRounds / 2, t.end());
-        // a smaller tail's launches only pay when clearly faster: the timing
-        // queues cycles back to back, which hides the launches' host time
-        if (i == 0 || t[kRounds / 2] < 0.99f * best_ms) {
+        if (i == 0 || t[kRounds / 2] < (cand[i] < 0 ? 0.97f : 0.99f) * best_ms) {
             best_ms = t[kRounds / 2];
             best = cand[i];
         }
