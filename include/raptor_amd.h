@@ -339,7 +339,9 @@ int ramd_hier_enable_fp32(ramd_hier h);
  * level -1: off; 0 (default): automatic -- the first cycle in each
  * precision times V-cycles with the three largest tails and with none and
  * keeps the fastest; >= 1: the tail starts at that level
- * (RAMD_E_ARG if it cannot).  No reference counterpart
+ * (RAMD_E_ARG if its sizes do not allow it; where they do but the packed form
+ * does not fit, at the first level below that does: ramd_hier_tail_level tells
+ * which).  No reference counterpart
  * (ParMultilevel::cycle, multilevel/par_multilevel.hpp:341-457, is one
  * routine per level); a tuning switch. */
 int ramd_hier_set_tail(ramd_hier h, int32_t level);

@@ -248,6 +248,7 @@ constexpr int kTailMax = 8;          // levels in the tail, the coarsest include
 constexpr int kTailMaxRows = 2048;   // a tail level's rows
 constexpr int64_t kTailMaxNnz = 32768;   // a tail level's A (and P) entries
 constexpr int kTailMaxOuterRows = 8190;  // rows of the level above the tail (16-bit byte offsets)
+constexpr int kTailSetOuterRows = 8192;  // ... that ramd_hier_set_tail takes
 constexpr int64_t kTailMaxOuterNnz = 65536;  // entries of its P
 
 static bool multicolour(const ramd_hier_s* h);
@@ -288,6 +289,28 @@ static std::vector<int> tail_packable(const ramd_hier_s* h)
 static std::vector<int> tail_candidates(const ramd_hier_s* h)
 {
     return h->track ? std::vector<int>() : tail_packable(h);
+}
+
+// What ramd_hier_set_tail makes of a level (>= 1): the start of the tail, -1
+// for none, or -2 if it is refused.  Levels within the sizes above are taken
+// also where the packed form is not (its 16-bit offsets, its padding, the
+// vectors' LDS): they run a launch per operation, with the same bits, and the
+// tail starts at the first level below them that can be packed.
+static int tail_set_start(const ramd_hier_s* h, int level)
+{
+    const std::vector<int> c = tail_candidates(h);
+    const auto at = std::lower_bound(c.begin(), c.end(), level);
+    if (at != c.end() && *at == level) return level;
+    const int nlev = (int)h->levels.size();
+    if (h->track || multicolour(h) || level >= nlev || nlev - level > kTailMax || h->coarse_n > kCoarseWave) return -2;
+    const Level& B = h->levels[level - 1];
+    bool ok = B.n <= kTailSetOuterRows && B.P->nnz <= kTailMaxOuterNnz;
+    for (int l = level; l < nlev && ok; l++) {
+        const Level& L = h->levels[l];
+        ok = L.n <= kTailMaxRows && L.A->nnz <= kTailMaxNnz && (!L.P || L.P->nnz <= kTailMaxNnz);
+    }
+    if (!ok) return -2;
+    return at == c.end() ? -1 : *at;
 }
 
 // Packs the largest tail's levels for cycles in precision prec.
@@ -2065,15 +2088,15 @@ int ramd_hier_set_tail(ramd_hier h, int32_t level)
 {
     return guarded([&] {
         RAMD_CHECK(h, RAMD_E_ARG, "ramd_hier_set_tail: NULL handle");
+        int start = level;
         if (level >= 1) {
-            const std::vector<int> c = tail_candidates(h);
-            RAMD_CHECK(std::find(c.begin(), c.end(), (int)level) != c.end(), RAMD_E_ARG,
-                       "ramd_hier_set_tail: level %d cannot start the coarse tail", (int)level);
+            start = tail_set_start(h, level);
+            RAMD_CHECK(start > -2, RAMD_E_ARG, "ramd_hier_set_tail: level %d cannot start the coarse tail", (int)level);
         }
         RAMD_CHECK(level >= -1, RAMD_E_ARG, "ramd_hier_set_tail: level %d", (int)level);
         h->ctx->set_current();
         RAMD_HIP(hipStreamSynchronize(h->ctx->stream));
-        h->tail_mode = level;
+        h->tail_mode = start;
     });
 }
 

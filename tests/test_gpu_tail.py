@@ -88,3 +88,54 @@ def test_fp32_enabled_while_tracking(ctx, first):
         ml.set_tail(mode)
         assert np.array_equal(cycle(), want), mode
     ml.free()
+
+
+def band(n, wide):
+    """laplace_1d's matrix without its dense form, constant coefficients."""
+    k = np.arange(-wide, wide + 1)
+    col = np.arange(n)[:, None] + k
+    ok = (col >= 0) & (col < n)
+    val = np.where(k == 0, 2.001 * wide, -1.0) + np.zeros(col.shape)
+    rp = np.concatenate([[0], np.cumsum(ok.sum(axis=1))])
+    return rp.astype(np.int32), col[ok].astype(np.int32), val[ok]
+
+
+@pytest.mark.parametrize("n,accepted", [(4000, True), (8190, True), (8191, True), (8192, True), (8193, False)])
+def test_set_tail_by_sizes(ctx, n, accepted):
+    """A start that its sizes allow is taken whether or not its packed form
+    fits; the tail then starts below it, with the bits of no tail."""
+    ml = ra.ParRugeStubenSolver(ctx, 0.25, ra.PMIS, ra.Direct, ra.Classical, ra.Jacobi)
+    ml.relax_weight = 2.0 / 3.0
+    ml.setup(*band(n, 9))
+    rows, nnz, nnz_p = ml.level_sizes()
+    assert rows[1] <= 2048 and nnz[1] <= 32768 and nnz_p[0] <= 65536 and rows[-1] <= 64 and ml.num_levels >= 3
+    ml.enable_fp32()
+    _, first = ml.tail_level()
+    assert first >= 2 or n <= 8190
+    b = np.random.default_rng(n).standard_normal(n)
+
+    def cycles():
+        x = ra.ParVector(ctx, n)
+        ml.cycle(x, ra.ParVector.from_numpy(ctx, b), x_is_zero=True)
+        x32 = ra.ParVector(ctx, n, np.float32)
+        ml.cycle_fp32(x32, ra.ParVector.from_numpy(ctx, b.astype(np.float32)))
+        return x.numpy(), x32.numpy()
+
+    ml.set_tail(-1)
+    want = cycles()
+    if accepted:
+        ml.set_tail(1)
+        assert ml.tail_level()[0] == first
+        got = cycles()
+        assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
+    else:
+        with pytest.raises(ra.RamdError):
+            ml.set_tail(1)
+    ml.set_track_times(True)
+    with pytest.raises(ra.RamdError):
+        ml.set_tail(1)
+    ml.set_track_times(False)
+    for level in (-2, ml.num_levels):
+        with pytest.raises(ra.RamdError):
+            ml.set_tail(level)
+    ml.free()
