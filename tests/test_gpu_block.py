@@ -272,3 +272,55 @@ def test_block_fpcg_first_sweep_in_update(ctx, sweeps, prec):
             assert abs(int(its[c]) - n1) <= 1, (c, its[c], n1)
             res = np.linalg.norm(B[:, c] - K.spmv(a, Xh[:, c])) / np.linalg.norm(B[:, c])
             assert res <= rtol * 1.001, (c, res)
+
+
+@pytest.mark.parametrize("sweeps", [1, 2])
+@pytest.mark.parametrize("k", [1, 3, 5, 8])
+@pytest.mark.parametrize("prec", [ra.PREC_FP64, ra.PREC_FP32])
+def test_block_fpcg_iterates(ctx, sweeps, k, prec):
+    """The lockstep solve's iterates against the flexible PCG written out with
+    the block cycle, whose first sweep is a pass of its own: a first sweep that
+    the update pass wrote with another weight, diagonal or right-hand side moves
+    them by more than 1e-3.  The dots are summed in another order: a few 1e-16 of
+    each scalar (the iterates 2e-16 apart), which can round single entries of the
+    FP32 cycle's input the other way, 6e-8 of them (the iterates 2e-10 apart).
+    Eager and replayed launches give the same bits."""
+    rp, col, val = ra.gallery_laplace27(13)
+    n, its = rp.size - 1, 4
+    ml = ra.ParRugeStubenSolver(ctx, 0.25, ra.PMIS, ra.Extended, ra.Classical, ra.Jacobi)
+    ml.relax_weight = OMEGA
+    ml.num_smooth_sweeps = sweeps
+    ml.setup(rp, col, val)
+    ml.enable_fp32()
+    A = ra.ParCSRMatrix.from_csr(ctx, rp, col, val)
+    a = K.Csr(rp, col, val)
+    B = np.random.default_rng(80 + k).standard_normal((n, k))
+    dt = np.float32 if prec == ra.PREC_FP32 else np.float64
+
+    def cycle(R):
+        Z = ra.ParVector(ctx, n * k, dt)
+        ra.vcycle_block(ml, Z, ra.ParVector.from_numpy(ctx, R.astype(dt).ravel()), k, prec)
+        return Z.numpy().reshape(n, k).astype(np.float64)
+
+    def product(X):
+        return np.stack([K.spmv(a, np.ascontiguousarray(X[:, c])) for c in range(k)], axis=1)
+
+    X, R = np.zeros((n, k)), B.copy()
+    Z = cycle(R)
+    P, rz = Z.copy(), (R * Z).sum(axis=0)
+    for _ in range(its):
+        AP = product(P)
+        alpha = rz / (P * AP).sum(axis=0)
+        X, R = X + alpha * P, R - alpha * AP
+        Z = cycle(R)
+        beta = -alpha * (Z * AP).sum(axis=0) / rz
+        P, rz = Z + beta * P, (R * Z).sum(axis=0)
+    got = []
+    for use_graph in (False, True):
+        x = ra.ParVector.from_numpy(ctx, np.zeros(n * k))
+        with pytest.raises(ra.RamdError, match="iterations did not reach"):
+            ra.FPCG_block(A, ml, x, ra.ParVector.from_numpy(ctx, B.ravel()), k, 1e-14, its, prec, use_graph)
+        got.append(x.numpy().reshape(n, k))
+    assert np.array_equal(got[0], got[1])
+    err = np.linalg.norm(got[0] - X, axis=0) / np.linalg.norm(X, axis=0)
+    assert (err <= (1e-8 if prec == ra.PREC_FP32 else 1e-14)).all()

@@ -429,3 +429,80 @@ def test_device_aggregate_rejects_unsorted_rows(ctx):
     U = ra.ParCSRMatrix.from_csr(ctx, rp, col, val)
     with pytest.raises(ra.RamdError):
         ra.aggregate_gpu(U, S, st)
+
+
+@pytest.mark.parametrize("length", [158, 159, 160, 161, 162, 240, 300])
+@pytest.mark.parametrize("n_c,c_near", [(250, 0), (256, 0), (120, 40), (90, 9)])
+@pytest.mark.parametrize("filt", [0.0, 0.3])
+def test_extended_rows_around_the_hash_lookup(ctx, length, n_c, c_near, filt):
+    """F rows whose strength row (diagonal included) is as long as the hash table
+    takes the columns of, shorter and longer, with up to 256 columns in the
+    interpolation row (c_near of them strong neighbours themselves, the others
+    reached through F neighbours), weak entries of both signs, and neighbour
+    rows past a wavefront: the host's bits."""
+    n = n_c + 400
+    rng = np.random.default_rng(1000 * length + n_c)
+    rows = [{} for _ in range(n)]
+    hubs = range(n_c, n_c + 6)
+    far = np.arange(n_c + 6, n)  # ordinary F rows
+    for i in hubs:
+        near = rng.choice(n_c, c_near, replace=False)
+        strong = np.concatenate([near, rng.choice(far, length - 1 - c_near, replace=False)])
+        for c in strong:
+            rows[i][c] = -rng.uniform(0.5, 1.0)
+        for c in rng.choice(np.setdiff1d(np.arange(n), np.append(strong, i)), 30, replace=False):
+            rows[i][c] = rng.choice([-0.05, 0.05, 0.4]) * rng.uniform(0.5, 1.0)
+    for f in far:  # three strong C points each, some hubs, now and then a long row
+        for c in rng.choice(n_c, 3, replace=False):
+            rows[f][c] = -rng.uniform(0.5, 1.0)
+        for h in hubs:
+            if f in rows[h] and rows[h][f] < -0.4:
+                rows[f][h] = -rng.uniform(0.5, 1.0)
+        for c in rng.choice(n, 80 if f % 17 == 0 else 2):
+            rows[f].setdefault(c, rng.choice([-0.04, 0.3]) * rng.uniform(0.5, 1.0))
+    for c in range(n_c):
+        for k in rng.choice(n, 5):
+            rows[c].setdefault(k, -rng.uniform(0.5, 1.0))
+    for i in range(n):
+        rows[i][i] = 1.0 + sum(abs(v) for v in rows[i].values())
+    col = np.concatenate([np.array([i] + sorted(set(r) - {i})) for i, r in enumerate(rows)]).astype(np.int32)
+    rp = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int32)
+    val = np.array([rows[i][c] for i in range(n) for c in col[rp[i]:rp[i + 1]]])
+    D = ra.ParCSRMatrix.from_csr(ctx, rp, col, val)
+    S = ra.strength_gpu(D, 0.25)
+    srp, scol, _ = S.to_csr()
+    states = np.zeros(n, np.int32)
+    states[:n_c] = 1
+    assert srp[n_c + 1] - srp[n_c] == length
+    hrp, hcol = ra.strength(rp, col, val, ra.Classical, 0.25)
+    assert np.array_equal(srp, hrp) and np.array_equal(scol, hcol)
+    prp, pcol, pval = ra.interp_extended_gpu(D, S, states, filt).to_csr()
+    wrp, wcol, wval, _ = ra.interpolation(rp, col, val, hrp, hcol, states, ra.Extended, filt)
+    if filt == 0.0 and n_c >= 250:
+        assert np.diff(prp)[n_c:n_c + 6].max() > 180  # most of the C points were reached
+    assert np.array_equal(prp, wrp) and np.array_equal(pcol, wcol) and np.array_equal(pval, wval)
+
+
+@pytest.mark.parametrize("filt", [0.0, 0.3])
+def test_extended_rows_around_the_kept_length(ctx, filt):
+    """Interpolation rows of 1 to 12 entries, those of up to eight kept from the
+    first pass: the host's bits."""
+    n_c, n = 60, 60 + 12 * 20
+    rng = np.random.default_rng(4)
+    rows = [{i: 12.0} for i in range(n)]
+    for f in range(n_c, n):
+        for c in rng.choice(n_c, 1 + (f - n_c) % 12, replace=False):
+            rows[f][c] = -rng.uniform(0.95, 1.0)
+            rows[c][f] = -rng.uniform(0.95, 1.0)
+    col = np.concatenate([np.array([i] + sorted(set(r) - {i})) for i, r in enumerate(rows)]).astype(np.int32)
+    rp = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int32)
+    val = np.array([rows[i][c] for i in range(n) for c in col[rp[i]:rp[i + 1]]])
+    D = ra.ParCSRMatrix.from_csr(ctx, rp, col, val)
+    S = ra.strength_gpu(D, 0.25)
+    hrp, hcol = ra.strength(rp, col, val, ra.Classical, 0.25)
+    states = np.zeros(n, np.int32)
+    states[:n_c] = 1
+    prp, pcol, pval = ra.interp_extended_gpu(D, S, states, filt).to_csr()
+    wrp, wcol, wval, _ = ra.interpolation(rp, col, val, hrp, hcol, states, ra.Extended, filt)
+    assert set(np.diff(prp)) == set(range(1, 13))
+    assert np.array_equal(prp, wrp) and np.array_equal(pcol, wcol) and np.array_equal(pval, wval)
