@@ -51,14 +51,20 @@ def vcycle_bytes(ml, sv):
       post-smooth Jacobi                           nnz (sv+4) + 4(n+1) + 3 sv n
     plus the coarse FP64 LU solve 8 nc^2 + 16 nc.  A level held in the
     stencil-diagonal form streams nd*n values and a 4-byte mask per row
-    instead of nnz (sv+4) + 4(n+1), a uniform one the mask only."""
+    instead of nnz (sv+4) + 4(n+1), a uniform one on the plane march the mask
+    only."""
     n, nnzA, nnzP = ml.level_sizes()
     total = 0.0
     L = len(n)
     for l in range(L - 1):
         nf, nc = int(n[l]), int(n[l + 1])
-        nd = 0 if ml.level(l)[0].uniform() else ml.level(l)[0].diagonals()
-        a = 4 * nf if ml.level(l)[0].uniform() else nd * nf * sv + 4 * nf if nd else nnzA[l] * (sv + 4) + 4 * (nf + 1)
+        A = ml.level(l)[0]
+        nd = A.diagonals()
+        if nd:
+            marched = A.uniform() and A.dia_staging(1 if sv == 4 else 0)[0] == 2
+            a = (0 if marched else nd * nf * sv) + 4 * nf
+        else:
+            a = nnzA[l] * (sv + 4) + 4 * (nf + 1)
         p = nnzP[l] * (sv + 4)
         total += 3 * sv * nf
         total += a + 3 * sv * nf
@@ -280,8 +286,8 @@ def main():
     outer_slot = dom_name.endswith("fp64")
     dom_op = A if outer_slot else ml.level(0)[0]
     staging = dom_op.dia_staging(2 if outer_slot else 1) if dom_op.diagonals() else None
-    kname = kernel_template(dom_name, dom["kernel"], ml.level(0)[0].diagonals(), staging,
-                            dom_op.uniform() and outer_slot)
+    kname = kernel_template(dom_name, dom["kernel"], ml.level(0)[0].diagonals(), staging, dom_op.uniform(),
+                            dom_op.dia_tile())
     traffic = measured_traffic(m, kname)
     roofline = dict(bound="hbm", achieved=round(achieved, 1), peak=PEAK_HBM_GBS, unit="GB/s",
                     frac=round(achieved / PEAK_HBM_GBS, 4), traffic=traffic, kernel=f"{dom['kernel']}:{dom_name}",
@@ -358,22 +364,22 @@ def main():
     ctx.close()
 
 
-def kernel_template(slot, kind, nd, staging=None, uniform=False):
+def kernel_template(slot, kind, nd, staging=None, uniform=False, tile=0):
     """Symbol of the kernel behind a timing slot of the FP32-form solve: the
     FP64-vector slots there read the lossless FP32 values.  staging: the
     stencil-diagonal variant (mode, planes, L, P) of the operator the slot
-    runs on (gather, LDS x window, or plane-march over the box grid)."""
+    runs on (gather, LDS x window, or plane-march over the box grid in tiles
+    of width `tile`).  The FP64 slots are the caller's operator, stored in
+    ascending order, the FP32 ones a hierarchy's, the diagonal first."""
     op = {"spmv": 0, "append": 1, "residual": 2, "jacobi": 3, "add_into": 4}[slot.rsplit("_", 1)[0]]
     vec = "float" if slot.endswith("fp32") else "double"
     if kind == "dia_kernel":
         mode = staging[0] if staging else 0
         if mode == 2:
-            L, P = staging[2:4]
-            tx = 64 if L % 64 == 0 else 32 if L % 32 == 0 else 16 if L % 16 == 0 else 64
-            if uniform:  # the caller's operator, stored in ascending order; the fewest positions past the grid
-                tx = min((32, 16, 64), key=lambda t: -(-L // t) * t * (-(-(P // L) * t // 256) * 256 // t))
-                return f"ramd::dia_uni_box_kernel<{op}, {vec}, {nd}, {tx}, false>"
-            return f"ramd::dia_box_kernel<{op}, float, {vec}, {nd}, {tx}>"
+            if uniform and op in (0, 2, 3):
+                df = "true" if vec == "float" else "false"
+                return f"ramd::dia_uni_box_kernel<{op}, {vec}, {nd}, {tile}, {df}>"
+            return f"ramd::dia_box_kernel<{op}, float, {vec}, {nd}, {tile}>"
         name = "dia_lds_kernel" if mode == 1 else "dia_kernel"
         return f"ramd::{name}<{op}, float, {vec}, {nd}>"
     return f"ramd::stream_kernel<{op}, {vec}, {vec}>"

@@ -94,6 +94,9 @@ int ramd_csr_diagonals(ramd_csr A, int* nd);
  * the diagonals are those of the 27- or 7-point box, so that the plane-march
  * kernel reads no values (followed through ramd_csr_set_values); else 0. */
 int ramd_csr_uniform(ramd_csr A, int* uniform);
+/* Width of the plane-march kernels' tiles for the present values (they are
+ * 256 / width lines high); 0 when the offsets have no box geometry. */
+int ramd_csr_dia_tile(ramd_csr A, int* width);
 /* Kernel variant of the stencil-diagonal form for the precision pair pp
  * (0 FP64 values and vectors, 1 FP32/FP32, 2 FP32 values/FP64 vectors):
  * mode 0 gathers x from memory, 1 stages each workgroup's x window in LDS,

@@ -194,6 +194,13 @@ class ParCSRMatrix:
         check(lib().ramd_csr_uniform(self.h, C.byref(u)))
         return bool(u.value)
 
+    def dia_tile(self):
+        """Tile width of the plane-march kernels for the present values
+        (ramd_csr_dia_tile), 0 without a box geometry."""
+        w = C.c_int()
+        check(lib().ramd_csr_dia_tile(self.h, C.byref(w)))
+        return w.value
+
     def to_csr(self):
         rp = np.empty(self.n_rows + 1, np.int32)
         col = np.empty(max(1, self.nnz), np.int32)

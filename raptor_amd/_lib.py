@@ -85,6 +85,7 @@ _SIGS = {
     "ramd_csr_destroy": (P,),
     "ramd_csr_diagonals": (P, C.POINTER(C.c_int)),
     "ramd_csr_uniform": (P, C.POINTER(C.c_int)),
+    "ramd_csr_dia_tile": (P, C.POINTER(C.c_int)),
     "ramd_csr_set_dia_staging": (P, C.c_int, C.c_int, C.c_int),
     "ramd_csr_dia_staging": (P, C.c_int, C.POINTER(C.c_int), C.POINTER(C.c_int), C.POINTER(C.c_int),
                              C.POINTER(C.c_int)),

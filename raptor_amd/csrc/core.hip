@@ -1640,6 +1640,16 @@ int ramd_csr_uniform(ramd_csr A, int* uniform)
     });
 }
 
+int ramd_csr_dia_tile(ramd_csr A, int* width)
+{
+    return guarded([&] {
+        RAMD_CHECK(A && width, RAMD_E_ARG, "ramd_csr_dia_tile: NULL argument");
+        bool df;
+        const Dia* d = A->dia;
+        *width = !d || d->box.L <= 0 ? 0 : dia_uni_box(d, &df) ? d->box.utx : d->box.tx;
+    });
+}
+
 int ramd_csr_destroy(ramd_csr A)
 {
     return guarded([&] {

@@ -196,6 +196,7 @@ def test_choices_follow_the_kind_of_values(ctx):
     assert first[0] >= 0
     values(other)
     assert not D.uniform() and D.dia_staging(2)[0] == -1
+    assert D.dia_tile() == 64  # lines of 33: no narrower tile divides them
     x = solve(ra.FPCG_noalloc)
     assert np.linalg.norm(b - K.spmv(K.Csr(A.rowptr, A.col, other), x)) <= 2e-8 * np.linalg.norm(b)
     solve(ra.FPCG)
@@ -203,6 +204,7 @@ def test_choices_follow_the_kind_of_values(ctx):
     assert second[0] >= 0
     values(3.0 * A.val)
     assert D.uniform() and D.dia_staging(2) == first
+    assert D.dia_tile() == 16  # the fewest positions past the grid
     values(other)
     assert D.dia_staging(2) == second
     D.set_dia_staging(2, 2, 5)
