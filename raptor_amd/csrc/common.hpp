@@ -48,7 +48,7 @@ constexpr double kWaveRowsMinLen = 24.0;
 constexpr int kStreamCap = 4096;     // products staged in LDS per workgroup
 // entry bytes from and up to which an untuned matrix is read through the
 // caches, the former also with a cycle between its products
-constexpr double kKeepMinBytes = 12e6;
+constexpr double kKeepMinBytes = 24e6;
 constexpr double kKeepMinCycled = 50e6;
 constexpr double kKeepMaxBytes = 96e6;
 constexpr int kMaxRowsPerBlock = 256;

@@ -1290,16 +1290,19 @@ static void launch_stream_cap(const ramd_csr_s* A, const ramd_csr_s::RowBlocks& 
     }
     // A matrix no tuner has seen, small enough that it, its vectors and a few
     // like it stay in the 256 MB infinity cache between operations, is read
-    // through the caches.  Repeated products, streamed / kept: 6.2 MB of
-    // entries 6.1 / 6.0 us, 12.5 MB 6.9 / 6.2, 21 MB 9.7 / 7.8, 63 MB 35.3 /
-    // 29.9, 89 MB 51.7 / 40.9; on a matrix just made they are equal (63 MB 51
-    // us); taken in turn with 600 MB of other matrices, which none stays for,
-    // keeping costs 4 to 8% (36.5 / 39.6).  With a cycle between the products
-    // the kept entries push its vectors out of the L2s, and only from about 50
-    // MB on is that made up for (flexible PCG on a 27-point matrix in CSR form:
-    // 20 MB 1.18 / 1.23 ms, 34 MB 1.35 / 1.40, 44 MB 1.54 / 1.54, 55 MB 1.68 /
-    // 1.64, 82 MB 2.00 / 1.96).  Level operators are tuned and streamed (27-point
-    // 101^3 FP32 cycle 147 us, through the caches 157).
+    // through the caches.  Products with three such matrices in turn, streamed /
+    // kept: 27 MB of entries each 17.7 / 15.2 us, 42 MB 25.4 / 20.0, 63 MB 38.3 /
+    // 30.2, 89 MB 53.4 / 52.0 (one alone 52.1 / 41.1).  Below 24 MB the streamed
+    // entries come from the infinity cache as fast, and kept ones push x out of
+    // the L2s: 12.6 MB 7.9 / 9.0, 21 MB 11.2 / 11.8 (one alone, all of it in the
+    // L2s, 9.9 / 8.7).  On a matrix just made both are equal (63 MB 51 us); in
+    // turn with 600 MB of others, which none stays for, keeping costs 4 to 8%
+    // (63 MB 36.5 / 39.6).  With a cycle between the products the kept entries
+    // push its vectors out as well, and only from about 50 MB on is that made up
+    // for (flexible PCG on a 27-point matrix in CSR form: 20 MB 1.18 / 1.23 ms,
+    // 34 MB 1.35 / 1.40, 44 MB 1.54 / 1.54, 55 MB 1.68 / 1.64, 82 MB 2.00 /
+    // 1.96).  Level operators are tuned and streamed (27-point 101^3 FP32 cycle
+    // 147 us, through the caches 157).
     if constexpr (CAP == kStreamCap && sizeof(V) == 8 && sizeof(X) == 8) {
         const double bytes = (double)A->nnz * 12.0;
         if (!A->tuned && bytes >= (A->cycled ? kKeepMinCycled : kKeepMinBytes) && bytes <= kKeepMaxBytes &&

@@ -1,5 +1,5 @@
 """A matrix that no tuner has seen: on both sides of the sizes between which its
-entries are read through the caches (12 to 96 MB of them, 50 with a cycle
+entries are read through the caches (24 to 96 MB of them, 50 with a cycle
 between the products), with empty rows and rows past one workgroup's products,
 every operation gives the oracle's bits, and a preconditioned solve does on
 either path."""
@@ -28,7 +28,7 @@ def matrix(entries, seed):
     return K.Csr(rp, col.astype(np.int32), rng.standard_normal(col.size))
 
 
-@pytest.mark.parametrize("entries", [500_000, 980_000, 1_080_000, 7_500_000, 8_800_000])
+@pytest.mark.parametrize("entries", [500_000, 1_950_000, 2_200_000, 7_500_000, 8_800_000])
 def test_operations_bit_exact(ctx, entries):
     A = matrix(entries, entries)
     n = A.n_rows
@@ -56,7 +56,7 @@ def test_operations_bit_exact(ctx, entries):
     D.free()
 
 
-@pytest.mark.parametrize("m", [40, 56])  # 1.6 and 4.6 million entries
+@pytest.mark.parametrize("m", [46, 56])  # 2.5 and 4.6 million entries
 def test_solve_operator_outside_and_inside(ctx, m):
     """The 27-point operator in CSR form (rows shuffled in groups of 64): its
     products before, during and after preconditioned solves."""
