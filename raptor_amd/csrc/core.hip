@@ -452,12 +452,14 @@ void dia_box_detect(const long long* offs, int nd, int n, DiaBox& b)
     // tile width: the widest of 64, 32, 16 that divides the line, else 64
     b.tx = b.L % 64 == 0 ? 64 : b.L % 32 == 0 ? 32 : b.L % 16 == 0 ? 16 : 64;
     // uniform operators: x and its halo are most of what a workgroup reads, so
-    // the squarer tiles of 32 or 16 (256^3 product 125 us with 64, 114 with 32,
-    // 112 with 16; 101^3, whose lines none divides, 14.5, 14.4 and 13.6): the
-    // one with the fewest positions past the grid, 32 where they are equal.
+    // the squarer tiles of 32 or 16: the one with the fewest positions past the
+    // grid, 32 where they are equal.  Products back to back, tiles of 64 and
+    // these: 101^3 (no width divides its lines; 16) 14.5 and 13.7 us, 192^3 46.0
+    // and 44.1, 256^3 115.8 and 107.9; in a solve, whose other kernels leave x in
+    // no cache, within 1% (256^3 25.65 and 25.70 ms, 192^3 10.67 and 10.61).
     // Planes per workgroup before any timing: eight where that leaves eight
     // workgroups per compute unit (192^3 50.5 -> 46.3 us), else four (101^3
-    // 14.5 us, with eight 19.2).
+    // 13.8 us, with eight 19.9).
     long long best = 0;
     for (const int t : {32, 16, 64}) {
         const long long ty = kBlockThreads / t, ny = b.P / b.L;

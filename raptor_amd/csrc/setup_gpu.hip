@@ -522,7 +522,9 @@ static void gpu_split_mis(const ramd_csr_s* S, const double* weights, int* state
 // caller then builds this level on the host).
 // ---------------------------------------------------------------------------
 constexpr int kExtCols = 256;
-constexpr int kExtHash = 512;  // load factor <= 1/2
+// 416 keys at most: a list of 256 and the up to 160 columns of a strength row
+// that are put in besides (kExtTagRow)
+constexpr int kExtHash = 512;
 constexpr int kExtWaves = 4;
 
 // LDS written by one lane becomes visible to the wavefront's other lanes

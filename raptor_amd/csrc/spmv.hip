@@ -938,17 +938,20 @@ __global__ __launch_bounds__(kBlockThreads) void dia_box_kernel(int n, int L, in
 
 // Uniform operators (one value per diagonal): the plane march without the
 // value streams.  What is left to read per row is the mask, the staged x and
-// b, so the kernel is bound by the vectors' traffic and, close behind, by its
-// instructions; hence the LDS offsets and the order of the diagonals are
-// compiled in (ND = 27: the whole box, ND = 7: its axes; DF: the centre
-// first), a wavefront whose rows all store every diagonal skips the selects,
-// and the row's mask and b are loaded one plane ahead.  The values uv come
-// through scalar loads from device memory (as kernel arguments, which a capture
-// fixes, no faster: 256^3 product 113 us, 108 from memory; 64^3 9.5 and 9.8).
-// The operations of a row and their order are dia_box_kernel's: the same bits.  27 points, 256^3:
-// the outer product 420 -> 129 us, the FP32 residual and Jacobi 409 and 388
-// -> 101 and 97 us; FP64 residual at 192^3, 351 (gather) -> 57 us, 198 MB of
-// vectors and masks at 3.5 TB/s.
+// b.  At 27 points and 256^3 no unit is full: the product's 350 MB of HBM
+// traffic (1.04x the algorithm's) go at 2.9 TB/s, VALU is busy 42%, LDS 38%
+// (no bank conflicts) and the TA 38% of the time, and the waves wait 73% of
+// theirs, for the planes from memory and at the barrier that follows each.  So
+// the chain of a plane is kept short: the LDS offsets and the order of the
+// diagonals are compiled in (ND = 27: the whole box, ND = 7: its axes; DF: the
+// centre first), a wavefront whose rows all store every diagonal skips the
+// selects, and the row's mask and b are loaded one plane ahead.  The values uv
+// come through scalar loads from device memory (as kernel arguments, which a
+// capture fixes, no faster: 256^3 product 113 us, 108 from memory; 64^3 9.5 and
+// 9.8).  The operations of a row and their order are dia_box_kernel's: the same
+// bits.  27 points, 256^3, in a solve: the outer product 420 -> 120 us, the FP32
+// residual and Jacobi 409 and 388 -> 99 and 97 us; FP64 residual at 192^3, 351
+// (gather) -> 55 us, 198 MB of vectors and masks at 3.6 TB/s.
 template <int OP, typename X, int ND, int TX, bool DF>
 __global__ __launch_bounds__(kBlockThreads) void dia_uni_box_kernel(int n, int L, int P, int nxt, int nyt, int zc,
                                                                    const X* __restrict__ uv,
