@@ -153,7 +153,6 @@ void dia_free(Dia* d)
     dfree(d->mask);
     dfree(d->v64);
     dfree(d->v32);
-    dfree(d->values);
     delete d;
 }
 
@@ -394,7 +393,6 @@ static void dia_check(ramd_csr_s* A, bool scatter)
     hipStream_t s = A->ctx->stream;
     const int n = A->n_rows;
     const dim3 grid((unsigned)std::min((n + kBlockThreads - 1) / kBlockThreads, 2048)), blk(kBlockThreads);
-    if (!d->values) d->values = dalloc<DiaValues>(1);
     hipLaunchKernelGGL(dia_check_init_kernel, dim3(1), dim3(kDiaMax), 0, s, d->values);
     if (scatter)
         hipLaunchKernelGGL(dia_scatter_kernel, grid, blk, 0, s, n, d->args, d->nd, A->rowptr, A->col, A->val, d->v64,
@@ -522,7 +520,9 @@ bool dia_build(ramd_csr_s* A)
     DiaArgs oa{};
     for (int k = 0; k < kDiaMax; k++) oa.off[k] = k < nd ? (int)offs[k] : 0;
     tmp.planes = dalloc<double>((size_t)nd * n);
-    tmp.mask = dalloc<unsigned>((size_t)n);
+    // the masks and, behind them, what dia_check finds
+    const size_t values_at = ((size_t)n + 3) / 4 * 4;
+    tmp.mask = dalloc<unsigned>(values_at + sizeof(DiaValues) / sizeof(unsigned));
     {
         const int g = (int)std::min<int64_t>(((int64_t)nd * n + 255) / 256, 8192);
         hipLaunchKernelGGL(fill_zero_kernel<double>, dim3(g), dim3(256), 0, s, tmp.planes, (int64_t)nd * n);
@@ -575,8 +575,8 @@ bool dia_build(ramd_csr_s* A)
         const int grid = (int)std::min<int64_t>(((int64_t)ns * n + 255) / 256, 8192);
         hipLaunchKernelGGL(dia_group_kernel, dim3(grid), dim3(256), 0, s, n, nd, ns, d->args, tmp.planes, d->v64);
         RAMD_HIP(hipGetLastError());
-        RAMD_HIP(hipStreamSynchronize(s));
         d->mask = tmp.mask;
+        d->values = reinterpret_cast<DiaValues*>(tmp.mask + values_at);
         tmp.mask = nullptr;
     } catch (...) {
         dia_free(d);
@@ -584,7 +584,7 @@ bool dia_build(ramd_csr_s* A)
     }
     A->dia = d;
     A->forms++;
-    dia_check(A, false);
+    dia_check(A, false);  // synchronizes: the scratch buffers are freed on return
     return true;
 }
 
@@ -687,6 +687,18 @@ __global__ __launch_bounds__(64) void csr_order_long_kernel(const int* __restric
     }
 }
 
+bool host_diag_first(int n_rows, const int* rp, const int* col)
+{
+    for (int i = 0; i < n_rows; i++)
+        for (int j = rp[i] + 1; j < rp[i + 1]; j++)
+            if (col[j] == i) return false;
+    return true;
+}
+
+// Entries up to which an upload is checked on the host (9 points, 64^2, 36
+// thousand entries: 156 us checked there, 200 on the device).
+constexpr int64_t kHostCheckNnz = 1 << 17;
+
 // Host CSR arrays on the device (rowptr non-decreasing from 0 to nnz), their
 // columns checked there and, with `order`, the rows put in the hierarchy's
 // order; nullptr when a row needs the host's sort.  The handle has no
@@ -707,7 +719,7 @@ ramd_csr_s* csr_upload(ramd_ctx ctx, int n_rows, int n_cols, int64_t nnz, const 
     t.rp = dalloc<int>((size_t)n_rows + 1);
     t.col = dalloc<int>((size_t)nnz);
     t.val = dalloc<double>((size_t)nnz);
-    t.flags = dalloc<int>(2);  // and the number of listed rows
+    if (order || nnz > kHostCheckNnz) t.flags = dalloc<int>(2);  // and the number of listed rows
     int out[2] = {0, 0};
     int& flags = out[0];
     auto read_flags = [&] {
@@ -716,18 +728,29 @@ ramd_csr_s* csr_upload(ramd_ctx ctx, int n_rows, int n_cols, int64_t nnz, const 
         RAMD_HIP(hipStreamSynchronize(s));
     };
     const dim3 grid((unsigned)((n_rows + 255) / 256));
-    RAMD_HIP(hipMemcpyAsync(t.rp, rowptr, sizeof(int) * (n_rows + 1), hipMemcpyHostToDevice, s));
-    hipLaunchKernelGGL(fill_int_kernel, dim3(1), dim3(64), 0, s, t.flags, (int64_t)2, 0);
-    if (nnz) {
-        RAMD_HIP(hipMemcpyAsync(t.col, col, sizeof(int) * nnz, hipMemcpyHostToDevice, s));
-        hipLaunchKernelGGL(csr_check_kernel, grid, dim3(256), 0, s, n_rows, n_cols, t.rp, t.col, t.flags);
-        RAMD_HIP(hipMemcpyAsync(t.val, val, sizeof(double) * nnz, hipMemcpyHostToDevice, s));
-    }
-    read_flags();
-    if (flags & 1)
+    // a few entries are looked at faster here than by a kernel that is waited for
+    const bool host_check = !order && nnz <= kHostCheckNnz;
+    auto columns_in_range = [&] {
         for (int64_t j = 0; j < nnz; j++)
             RAMD_CHECK(col[j] >= 0 && col[j] < n_cols, RAMD_E_ARG, "%s: column %d of entry %lld outside [0,%d)", who,
                        col[j], (long long)j, n_cols);
+    };
+    if (host_check) columns_in_range();
+    RAMD_HIP(hipMemcpyAsync(t.rp, rowptr, sizeof(int) * (n_rows + 1), hipMemcpyHostToDevice, s));
+    if (nnz) {
+        RAMD_HIP(hipMemcpyAsync(t.col, col, sizeof(int) * nnz, hipMemcpyHostToDevice, s));
+        if (!host_check) {
+            hipLaunchKernelGGL(fill_int_kernel, dim3(1), dim3(64), 0, s, t.flags, (int64_t)2, 0);
+            hipLaunchKernelGGL(csr_check_kernel, grid, dim3(256), 0, s, n_rows, n_cols, t.rp, t.col, t.flags);
+        }
+        RAMD_HIP(hipMemcpyAsync(t.val, val, sizeof(double) * nnz, hipMemcpyHostToDevice, s));
+    }
+    if (host_check) {
+        flags = host_diag_first(n_rows, rowptr, col) ? 0 : 2;
+    } else if (nnz) {
+        read_flags();
+        if (flags & 1) columns_in_range();
+    }
     if (order && nnz) {
         t.rows = dalloc<int>((size_t)(nnz / kOrderMaxRow));  // rows longer than that
         hipLaunchKernelGGL(fill_int_kernel, dim3(1), dim3(64), 0, s, t.flags, (int64_t)2, 0);
@@ -746,14 +769,6 @@ ramd_csr_s* csr_upload(ramd_ctx ctx, int n_rows, int n_cols, int64_t nnz, const 
     t.val = nullptr;
     A->diag_first = !(flags & 2);
     return A;
-}
-
-bool host_diag_first(int n_rows, const int* rp, const int* col)
-{
-    for (int i = 0; i < n_rows; i++)
-        for (int j = rp[i] + 1; j < rp[i + 1]; j++)
-            if (col[j] == i) return false;
-    return true;
 }
 
 // ---------------------------------------------------------------------------

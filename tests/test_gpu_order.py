@@ -51,9 +51,11 @@ def test_fine_level_order(ctx, n, longest, twice):
         assert np.array_equal(a, b)
 
 
-def test_bad_input_refused(ctx):
-    rp, col, val = matrix(100, 10, False, 1)
-    for c in (-1, 100, 2**31 - 1):
+@pytest.mark.parametrize("n", [100, 30000])  # checked on the host, and on the device (from 131 thousand entries)
+def test_bad_input_refused(ctx, n):
+    rp, col, val = matrix(n, 10, False, 1)
+    assert (col.size > 1 << 17) == (n > 100)
+    for c in (-1, n, 2**31 - 1):
         bad = col.copy()
         bad[37] = c
         with pytest.raises(ra.RamdError):
