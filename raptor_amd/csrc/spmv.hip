@@ -1079,10 +1079,10 @@ bool dia_uni_box(const Dia* d, bool* diag_first)
 // before any timing.  A workgroup of the march walks four planes one after
 // another, 9 us for 27 points and 6 us for 7 however few rows there are; the
 // gather's time follows its bytes.  FP64 residual, gather / march: 27 points
-// 32^3 6.1 / 9.3 us, 56^3 (43 MB) 8.9 / 9.5, 64^3 (64 MB) 12.0 / 9.6, 101^3
+// 32^3 6.1 / 9.3 us, 57^3 (45 MB) 9.3 / 9.7, 64^3 (64 MB) 12.0 / 9.6, 101^3
 // 46.8 / 13.4; 7 points 32^3 5.0 / 5.8, 72^3 (31 MB) 6.3 / 6.6, 80^3 (43 MB)
 // 7.9 / 6.6, 128^3 29.9 / 11.8.
-constexpr double kUniMarchBytes = 43e6;
+constexpr double kUniMarchBytes = 48e6;
 
 // Whether the plane march of uniform operator A pays by that line times
 // `factor`: not on a grid whose tiles are less than a third full (7 points,

@@ -97,7 +97,7 @@ def test_value_changes_turn_it_off_and_on(ctx, what):
     check(ctx, D, K.Csr(A.rowptr, A.col, 2.0 * A.val))
 
 
-@pytest.mark.parametrize("dims,pts", [((56, 56, 56), 27), ((58, 56, 58), 27), ((81, 79, 79), 7), ((81, 79, 81), 7),
+@pytest.mark.parametrize("dims,pts", [((58, 58, 58), 27), ((60, 58, 58), 27), ((82, 83, 83), 7), ((84, 85, 81), 7),
                                       ((3, 700, 300), 7)])
 def test_both_sides_of_the_untimed_rule(ctx, dims, pts):
     """The largest grids that the gather takes before any timing, the smallest
