@@ -1059,6 +1059,37 @@ __global__ void transpose_scatter_kernel(int n, const int* __restrict__ rp, cons
     }
 }
 
+// Short columns in row order, in place: a thread holds a column of up to K
+// entries in registers and puts each where its rank says.  No second arrays,
+// whose allocation and release were the larger part (first A^T x of the 7-point
+// 96^3 operator, from which columns are at most 7 long: 2.4-2.6 ms with them).
+template <int K>
+__global__ __launch_bounds__(kBlockThreads) void transpose_short_kernel(int m, const int* __restrict__ tp,
+                                                                        int* __restrict__ row,
+                                                                        double* __restrict__ val)
+{
+    const int c = blockIdx.x * kBlockThreads + threadIdx.x;
+    if (c >= m) return;
+    const int s = tp[c], len = tp[c + 1] - s;
+    int r[K];
+    double v[K];
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+        r[k] = k < len ? row[s + k] : INT_MAX;
+        v[k] = k < len ? val[s + k] : 0.0;
+    }
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+        int rank = 0;
+#pragma unroll
+        for (int j = 0; j < K; j++) rank += r[j] < r[k] || (r[j] == r[k] && j < k);
+        if (k < len) {
+            row[s + rank] = r[k];
+            val[s + rank] = v[k];
+        }
+    }
+}
+
 // Every column's (row, value) pairs in row order: a group of G lanes per
 // column, each entry's place the number of smaller rows in its column (a row
 // that stores the column twice put its entries in stored order).  One thread
@@ -1201,8 +1232,10 @@ int64_t device_rowptr(ramd_ctx ctx, const int* cnt, int n, int* rp, const char* 
     return total;
 }
 
-// longest column that is ranked (the square of its length; longer: host sort)
+// longest column that is ranked (the square of its length; longer: host sort),
+// and that is ranked in registers
 constexpr int kTransposeMaxCol = 2048;
+constexpr int kTransposeShortCol = 16;
 
 ramd_csr_s* csr_transpose(ramd_csr_s* A)
 {
@@ -1245,17 +1278,24 @@ ramd_csr_s* csr_transpose(ramd_csr_s* A)
                     dfree(val);
                 }
             } t;
+            const bool in_place = longest <= kTransposeShortCol;
             t.cursor = dalloc<int>((size_t)std::max(m, 1));
-            t.row = dalloc<int>((size_t)nnz);
-            t.val = dalloc<double>((size_t)nnz);
+            if (!in_place) {
+                t.row = dalloc<int>((size_t)nnz);
+                t.val = dalloc<double>((size_t)nnz);
+            }
             RAMD_HIP(hipMemcpyAsync(t.cursor, d_rp, sizeof(int) * m, hipMemcpyDeviceToDevice, s));
             hipLaunchKernelGGL(transpose_scatter_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, n,
-                               A->rowptr, A->col, A->val, t.cursor, t.row, t.val);
+                               A->rowptr, A->col, A->val, t.cursor, in_place ? d_col : t.row,
+                               in_place ? d_val : t.val);
             // lanes per column: about half its average length, whole
             // wavefronts from 32 entries on
             const int64_t avg = nnz / std::max(m, 1);
             auto grid = [&](int g) { return dim3((unsigned)(((int64_t)m * g + kBlockThreads - 1) / kBlockThreads)); };
-            if (avg < 12)
+            if (in_place)
+                hipLaunchKernelGGL((transpose_short_kernel<kTransposeShortCol>), grid(1), dim3(kBlockThreads), 0, s,
+                                   m, d_rp, d_col, d_val);
+            else if (avg < 12)
                 hipLaunchKernelGGL((transpose_rank_kernel<4>), grid(4), dim3(kBlockThreads), 0, s, m, d_rp, t.row,
                                    t.val, d_col, d_val);
             else if (avg < 32)

@@ -1,7 +1,7 @@
-"""The device transpose at its edges: columns of 0 to 2049 entries (4, 16 and
-64 lanes per column, the longest sorted on the host) and rows that store a
-column twice.  A^T x adds each column's products in ascending row order, so the
-bits follow the order."""
+"""The device transpose at its edges: columns of 0 to 2049 entries (in a thread's
+registers up to 16, else 4, 16 and 64 lanes per column, the longest sorted on
+the host) and rows that store a column twice.  A^T x adds each column's products
+in ascending row order, so the bits follow the order."""
 import numpy as np
 import pytest
 
@@ -12,7 +12,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("rows,cols,avg,longest,twice", [
-    (3000, 900, 3, 40, False), (3000, 900, 11, 30, True), (2000, 333, 12, 17, False), (2000, 333, 31, 64, True),
+    (3000, 900, 3, 15, False), (3000, 900, 5, 16, False), (3000, 900, 5, 17, False), (3000, 900, 4, 9, True),
+    (400, 300, 1, 1, False), (3000, 900, 3, 40, False), (3000, 900, 11, 30, True), (2000, 333, 12, 17, False), (2000, 333, 31, 64, True),
     (5000, 70, 40, 65, False), (5000, 70, 200, 600, True), (2100, 5, 1000, 2048, False), (2100, 5, 1000, 2049, False)])
 def test_transpose_order_bit_exact(ctx, rows, cols, avg, longest, twice):
     rng = np.random.default_rng(rows + cols + avg)
