@@ -728,7 +728,7 @@ def cpu_threads(args_threads):
 
 
 def cpu_baseline(ml, rp, col, val, b_h, x32_h, x64_h, threads=0):
-    """The oracle on the GPU box's host cores, on the product's own
+    """The oracle on the machine's host cores, on the product's own
     hierarchy (outside every timed GPU region):
 
       - cpu_baseline: one whole solve of the same system to a true relative

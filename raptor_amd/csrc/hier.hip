@@ -347,14 +347,14 @@ static void cycle32(ramd_hier_s* h, int l, float* x, const float* b, bool x_zero
 // and keeps the largest unless a later one's median is 1% below, without a tail
 // 3% (same bits for all; the queue hides the host time of the launches that a
 // smaller tail adds, about three without one: aggregation, 7 points 16^3, 33.0
-// us against 32.1 in the queue, 41.4 against 35.9 from a slow host).  No smaller tail: an operation inside the tail costs 0.7-2.5 us, a
-// launch of its own 3-5 us; only the largest levels' operations, bound by
-// what one compute unit reads, are in doubt (9-point anisotropic 100^2, FP64,
-// tails from levels of 780, 362, 168, 76, 34 rows and none: 96.6, 93.2,
-// 103.8, 121.0, 134.6, 142.7 us a cycle).  A tail of the coarsest level alone,
-// whose restriction has a few long rows, can lose to none (aggregation, 7
-// points 80^3, 1173 -> 48 rows, FP32: 82.9 us, none 79.1).  Uses the fine
-// level's own x and b vectors.
+// us against 32.1 in the queue, 41.4 against 35.9 from a slow host).  No
+// smaller tail: an operation inside the tail costs 0.7-2.5 us, a launch of its
+// own 3-5 us; only the largest levels' operations, bound by what one compute
+// unit reads, are in doubt (9-point anisotropic 100^2, FP64, tails from levels
+// of 780, 362, 168, 76, 34 rows and none: 96.6, 93.2, 103.8, 121.0, 134.6,
+// 142.7 us a cycle).  A tail of the coarsest level alone, whose restriction has
+// a few long rows, can lose to none (aggregation, 7 points 80^3, 1173 -> 48
+// rows, FP32: 82.9 us, none 79.1).  Uses the fine level's own x and b vectors.
 void cycle_prepare(ramd_hier_s* h, int prec)
 {
     if (prec == 1) enable_fp32(h);
